@@ -15,7 +15,7 @@
 //    rows no query token picked, the fp32 sum for picked rows, in (query,
 //    token) order), so there is no torch.zeros_like memset and no fp16
 //    atomics; results are bitwise deterministic.
-#include <mutex>
+#include <type_traits>
 
 #include "fmx_device.h"
 #include "fmx_kernels.h"
@@ -98,11 +98,11 @@ __device__ __forceinline__ int doc_len(const BwdArgs& a, int b) {
 // skipped (not multiplied by zero: a row may hold NaN padding); whether a doc
 // counts depends on the doc alone, so the skip is uniform over the wave.
 template <bool BF, bool FULL>
-__device__ __forceinline__ void dq_partial_block(const BwdArgs& a, int bx, int by) {
+__device__ __forceinline__ void dq_partial_block(const BwdArgs& a, int64_t bx, int by) {
   constexpr int DB = 8;
   const int nkc = (a.d + 7) >> 3;
   const int64_t rows = (int64_t)a.Nq * a.Lq;
-  const int64_t tid = (int64_t)bx * 256 + threadIdx.x;
+  const int64_t tid = bx * 256 + threadIdx.x;
   if (tid >= rows * nkc) return;
   const int64_t r = tid / nkc;
   const int k0 = (int)(tid - r * nkc) * 8;
@@ -128,7 +128,7 @@ __device__ __forceinline__ void dq_partial_block(const BwdArgs& a, int bx, int b
 #pragma unroll
     for (int u = 0; u < DB; ++u) {
       live[u] = bb + u < b1;
-      if (a.lengths) live[u] = live[u] && a.lengths[bi[u]] > 0;
+      if (a.lengths) live[u] = live[u] && ld_uniform(a.lengths + bi[u]) > 0;
       j[u] = clamp_index(j[u], a.Ld);
     }
     float x[DB][8];
@@ -161,9 +161,9 @@ __device__ __forceinline__ void dq_partial_block(const BwdArgs& a, int bx, int b
 
 // Stage 2 of dQ: dQ[r][k] = sum over chunks (in order) of ws[chunk][r][k].
 template <bool BF>
-__global__ void __launch_bounds__(256) bwd_dq_finalize_kernel(BwdArgs a) {
+__device__ __forceinline__ void dq_sum_block(const BwdArgs& a, int64_t block) {
   const int64_t n = (int64_t)a.Nq * a.Lq * a.d;
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t i = block * 256 + threadIdx.x;
   if (i >= n) return;
   float s = 0.f;
 #pragma unroll 8
@@ -174,19 +174,106 @@ __global__ void __launch_bounds__(256) bwd_dq_finalize_kernel(BwdArgs a) {
 constexpr int kEntryBits = 13;  // entries of one chunk < 2^13 (kDdChunk)
 constexpr uint32_t kNoRow = 0xffffffffu;
 constexpr int kDdMaxPasses = 4;  // workgroup row passes per dD writer slab, at most
-// dD sizes from which the dQ chain runs on a second stream (launch_bwd_t).
-constexpr int64_t kBwdForkBytes = (int64_t)1 << 24;
+// LDS of an index workgroup: its keys, and with the counting sort four
+// counters per doc row, which fit beside 8192 keys up to Ld = 2040.
+constexpr size_t kDdIndexLds = 65536 - 64;
+constexpr size_t dd_count_bytes(int64_t Ld) { return (size_t)Ld * 4 * sizeof(uint32_t); }
 
 // dD index, one workgroup per (doc, chunk of kDdChunk consecutive (query,
-// token) entries). The chunk's entries e become keys row << 13 | (e - e0) in
-// LDS, bitonic-sorted, so each picked row's entries are contiguous and in
-// entry order. Written to the workspace:
+// token) entries): the chunk's entries sorted by the doc row they picked, in
+// entry order within a row. Written to the workspace:
 //   ent[b][e0 + p]     chunk-local entry of sorted position p (uint16)
 //   rows[c][b][j]      first sorted position | count << 16 of row j within
 //                      chunk c, or kNoRow.
 // Chunks hold consecutive entries, so a row's entries taken chunk by chunk
 // are in entry order. Docs of length 0 pick no rows.
-__device__ __forceinline__ void dd_index_block(const BwdArgs& a, int b, int chunk, uint32_t* keys) {
+//
+// A stable counting sort: wave w takes the w-th quarter of the entries and
+// counts its rows in its own LDS counters; a scan over (row, wave) turns the
+// counts into positions; then each wave places its entries 64 at a time, a
+// lane's place among the lanes of its row found by ballots over the bits of
+// the row number. What bounds it is the number of barriers and dependent LDS
+// round trips per workgroup, as one doc's entries rarely fill more than one
+// workgroup per CU: four barriers here, where a bitonic sort of the keys takes
+// one per step, 55 for 1024 entries (32 queries of 32 tokens over 256 docs of
+// up to 180 tokens: 44.0 -> 6.7 us).
+__device__ __forceinline__ void dd_index_count(const BwdArgs& a, int b, int chunk, uint32_t* smem) {
+  const int NL = a.Nq * a.Lq;
+  const int e0 = chunk * kDdChunk;
+  const int n = NL - e0 < kDdChunk ? NL - e0 : kDdChunk;  // entries of this chunk
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool empty = a.lengths && doc_len(a, b) == 0;
+  uint32_t* keys = smem;                // [sort_n] the row each entry picked
+  uint32_t* pos = smem + a.sort_n;      // [4][Ld] counts, then next positions
+  __shared__ uint32_t wtot[4];
+  for (int i = threadIdx.x; i < 4 * a.Ld; i += 256) pos[i] = 0u;
+  __syncthreads();
+  const int seg = (n + 255) / 256 * 64;  // entries per wave
+  const int p0 = wave * seg, p1 = empty ? p0 : (p0 + seg < n ? p0 + seg : n);
+  uint32_t* mypos = pos + wave * a.Ld;
+  for (int p = p0 + lane; p < p1; p += 64) {
+    const int e = e0 + p;
+    const int qi = e / a.Lq, q = e - qi * a.Lq;
+    const int j = clamp_index(a.argmax[((int64_t)qi * a.B + b) * a.Lq + q], a.Ld);
+    keys[p] = (uint32_t)j;
+    atomicAdd(&mypos[j], 1u);
+  }
+  __syncthreads();
+  // each thread scans `per` consecutive rows
+  const int per = (a.Ld + 255) / 256;
+  const int j0 = threadIdx.x * per, j1 = j0 + per < a.Ld ? j0 + per : a.Ld;
+  uint32_t sum = 0u;
+  for (int j = j0; j < j1; ++j) sum += pos[j] + pos[a.Ld + j] + pos[2 * a.Ld + j] + pos[3 * a.Ld + j];
+  uint32_t incl = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t v = __shfl_up(incl, o);
+    if (lane >= o) incl += v;
+  }
+  if (lane == 63) wtot[wave] = incl;
+  __syncthreads();
+  uint32_t at = incl - sum;
+  for (int w = 0; w < wave; ++w) at += wtot[w];
+  uint32_t* rows = a.dd_rows + ((int64_t)chunk * a.B + b) * a.Ld;
+  for (int j = j0; j < j1; ++j) {
+    const uint32_t first = at;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t c = pos[w * a.Ld + j];
+      pos[w * a.Ld + j] = at;
+      at += c;
+    }
+    rows[j] = at > first ? first | ((at - first) << 16) : kNoRow;
+  }
+  __syncthreads();
+  uint16_t* ent = a.dd_ent + (int64_t)b * NL + e0;
+  const int nbits = a.Ld > 1 ? 32 - __builtin_clz((unsigned)(a.Ld - 1)) : 0;
+  for (int pb = p0; pb < p1; pb += 64) {  // uniform over the wave
+    const int p = pb + lane;
+    const bool in = p < p1;
+    const uint32_t j = in ? keys[p] : 0u;
+    uint64_t same = __builtin_amdgcn_ballot_w64(in);  // lanes of this lane's row
+    for (int bit = 0; bit < nbits; ++bit) {
+      const bool one = (j >> bit) & 1u;
+      const uint64_t ones = __builtin_amdgcn_ballot_w64(one);
+      same &= one ? ones : ~ones;
+    }
+    if (in) {
+      const uint32_t base = mypos[j];
+      const int before = __builtin_popcountll(same & (((uint64_t)1 << lane) - 1));
+      ent[base + before] = (uint16_t)p;
+      // the row's last lane moves its next position on, once every lane has read it
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (same >> lane == 1u) mypos[j] = base + before + 1;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+}
+
+// The same by a bitonic sort of the keys row << 13 | (e - e0) in LDS, for docs
+// whose row counters do not fit there (kDdIndexLds).
+__device__ __forceinline__ void dd_index_sort(const BwdArgs& a, int b, int chunk, uint32_t* keys) {
   const int NL = a.Nq * a.Lq;
   const int e0 = chunk * kDdChunk;
   const int n = NL - e0 < kDdChunk ? NL - e0 : kDdChunk;  // entries of this chunk
@@ -243,18 +330,34 @@ __device__ __forceinline__ void dd_index_block(const BwdArgs& a, int b, int chun
 // no entry picked is zeros; a picked row is the fp32 sum over its entries, in
 // entry order, of g[qi, b] * Q[qi, q]. Lanes cover a row's 8-wide k chunks:
 // L = min(64, pow2 >= chunks) lanes per row, 64 / L rows per wave pass.
-template <bool BF>
-__device__ __forceinline__ void dd_write_block(const BwdArgs& a, int slab) {
+//
+// Sparse rows (one query) are bound by the stores, and take one entry at a
+// time. DENSE, rows that many entries picked (a batch of queries over short
+// docs: 200 a row), are a serial chain, as the sum keeps entry order: the L
+// lanes of a row therefore fetch L entries at a time, each lane one entry's
+// number, Q row and gradient, the next L while the current ones are summed, and
+// the Q rows themselves come up to kDdAhead at a time (an entry at a time is a
+// chain of three memory round trips each: 32 queries of 32 tokens over 256 docs
+// of up to 180 tokens 84 -> 25 us). Rows of one or two entries gain nothing
+// from that, so a wave whose rows all have so few takes them singly here too.
+// kDdAhead: eight rows ahead cost a third of the waves (five per SIMD, seven
+// with four: 1000 docs of 512 x 1024 under 256 tokens 357 -> 323 us, 4000 of
+// 300 x 128 under 200 144 -> 128; the smallest batches 35 -> 38).
+// FULL (DENSE): every 8-wide chunk lies inside d (d % 8 == 0).
+constexpr int kDdAhead = 4;
+template <bool BF, bool DENSE, bool FULL>
+__device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
   const int nkc = (a.d + 7) >> 3;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int lsh = 0;
   while ((1 << lsh) < nkc && lsh < 6) ++lsh;
+  const int L = 1 << lsh;
   const int rpw = 64 >> lsh;               // rows per wave pass
   const int sub = lane >> lsh;             // this lane's row within the pass
-  const int kc0 = lane & ((1 << lsh) - 1);
+  const int kc0 = lane & (L - 1);
   const int64_t total = (int64_t)a.B * a.Ld;
-  const int64_t r0 = (int64_t)slab * a.dd_slab;
+  const int64_t r0 = slab * a.dd_slab;
   const int64_t r1 = r0 + a.dd_slab < total ? r0 + a.dd_slab : total;
   const int step = 4 * rpw;
   int64_t r = r0 + wave * rpw + sub;
@@ -278,7 +381,8 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int slab) {
     const uint32_t info0 = infos[p];
     if (a.dd_chunks == 1 && info0 == kNoRow) {
       for (int kc = kc0; kc < nkc; kc += 64) store8<BF>(orow, kc * 8, a.d, zero);
-    } else {
+    } else if (!DENSE || (a.dd_chunks == 1 &&
+                          __builtin_amdgcn_ballot_w64(info0 != kNoRow && (info0 >> 16) > 2u) == 0)) {
       for (int kc = kc0; kc < nkc; kc += 64) {
         const int k0 = kc * 8;
         float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -301,6 +405,72 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int slab) {
         }
         store8<BF>(orow, k0, a.d, acc);
       }
+    } else if constexpr (DENSE) {
+      // every lane of the row takes part in each step below, those past its
+      // last k chunk too (they fetch entries; their loads repeat chunk 0)
+      for (int kb = 0; kb < nkc; kb += 64) {
+        const bool live = kb + kc0 < nkc;
+        const int k0 = live ? (kb + kc0) * 8 : 0;
+        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        // the row's entries chunk by chunk: entry order overall
+        for (int ch = 0; ch < a.dd_chunks; ++ch) {
+          const uint32_t info = ch == 0 ? info0 : a.dd_rows[(int64_t)ch * total + r];
+          if (info == kNoRow) continue;
+          const int e0 = ch * kDdChunk;
+          const uint16_t* ent = a.dd_ent + (int64_t)b * NL + e0 + (info & 0xffffu);
+          const int n = (int)(info >> 16);
+          // entry i0 + kc0 of the row: its Q row's offset in 8-element units
+          // (query strides are multiples of 8) and its gradient
+          auto fetch = [&](int i0, uint32_t& off, float& g) __attribute__((always_inline)) {
+            off = 0u;
+            g = 0.f;
+            if (i0 + kc0 < n) {
+              const int e = e0 + ent[i0 + kc0];
+              const int qi = e / a.Lq, q = e - qi * a.Lq;
+              off = (uint32_t)(((int64_t)qi * a.sq_n + (int64_t)q * a.sq_l) >> 3);
+              g = a.grad[(int64_t)qi * a.g_n + (int64_t)b * a.g_b];
+            }
+          };
+          auto add = [&](auto count_tag, uint32_t off, float g, int u0) __attribute__((always_inline)) {
+            constexpr int U = decltype(count_tag)::value;
+            float x[U][8], gu[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              const int src = (lane & ~(L - 1)) + u0 + u;
+              const uint16_t* row = Q + (int64_t)lane_fetch(off, src) * 8;
+              gu[u] = __builtin_bit_cast(float, lane_fetch(__builtin_bit_cast(uint32_t, g), src));
+              if constexpr (FULL) {
+                const u32x4_t v = *reinterpret_cast<const u32x4_t*>(row + k0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                  x[u][2 * i] = Elem<BF>::to_f(v[i] & 0xffffu);
+                  x[u][2 * i + 1] = Elem<BF>::to_f(v[i] >> 16);
+                }
+              } else {
+                load8<BF>(row, k0, a.d, x[u]);
+              }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+              for (int k = 0; k < 8; ++k) acc[k] = fmaf(gu[u], x[u][k], acc[k]);
+          };
+          uint32_t off, noff = 0u;
+          float g, ng = 0.f;
+          fetch(0, off, g);
+          for (int i0 = 0; i0 < n; i0 += L) {
+            const int m = n - i0 < L ? n - i0 : L;
+            if (i0 + L < n) fetch(i0 + L, noff, ng);
+            int u0 = 0;
+            for (; u0 + kDdAhead <= m; u0 += kDdAhead) add(std::integral_constant<int, kDdAhead>{}, off, g, u0);
+            for (; u0 + 2 <= m; u0 += 2) add(std::integral_constant<int, 2>{}, off, g, u0);
+            if (u0 < m) add(std::integral_constant<int, 1>{}, off, g, u0);
+            off = noff;
+            g = ng;
+          }
+        }
+        if (live) store8<BF>(orow, k0, a.d, acc);
+      }
     }
     j += step;
     while (j >= a.Ld) {
@@ -310,107 +480,101 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int slab) {
   }
 }
 
-template <bool BF, bool FULL>
-__global__ void __launch_bounds__(256) bwd_dq_partial_kernel(BwdArgs a) {
-  dq_partial_block<BF, FULL>(a, blockIdx.x, blockIdx.y);
-}
-
-__global__ void __launch_bounds__(256) bwd_dd_index_kernel(BwdArgs a) {
+// The backward is two launches. Each carries a small part of one gradient
+// beside the large part of the other, which it does not depend on, so the
+// small parts cost neither a launch nor time of their own:
+//   front: the dD index (the first n_index workgroups) and the dQ gather,
+//   back:  the dQ sum (the first n_sum workgroups) and the dD writer.
+// The gather and the writer do not share a launch: reads of D beside the
+// stores of dD lower the rate of both (interleaved in one grid 15 % slower; on
+// two streams 4 % slower than this with 1000 docs of 512 x 1024, and its event
+// waits cost 20 us where dD is 77 MB, 41.8 -> 24.0 us).
+template <bool BF, bool FULL, bool COUNT>
+__global__ void __launch_bounds__(256) bwd_front_kernel(BwdArgs a, unsigned n_gather, unsigned gather_x) {
   extern __shared__ uint32_t smem[];
-  dd_index_block(a, blockIdx.x, blockIdx.y, smem);
-}
-
-template <bool BF>
-__global__ void __launch_bounds__(256) bwd_dd_write_kernel(BwdArgs a) {
-  dd_write_block<BF>(a, blockIdx.x);
-}
-
-template <bool BF>
-void launch_dq_chain(const BwdArgs& a, hipStream_t s) {
-  const int nkc = (a.d + 7) >> 3;
-  const int64_t threads = (int64_t)a.Nq * a.Lq * nkc;
-  // FULL: every 8-wide chunk lies inside d, so each gather is one 16-byte load
-  const dim3 grid((unsigned)((threads + 255) / 256), a.nchunk);
-  if ((a.d & 7) == 0 && (a.sd_b & 7) == 0 && (a.sd_l & 7) == 0)
-    hipLaunchKernelGGL((bwd_dq_partial_kernel<BF, true>), grid, dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL((bwd_dq_partial_kernel<BF, false>), grid, dim3(256), 0, s, a);
-  const int64_t n = (int64_t)a.Nq * a.Lq * a.d;
-  hipLaunchKernelGGL(bwd_dq_finalize_kernel<BF>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
-}
-
-template <bool BF>
-void launch_dd_chain(const BwdArgs& a, hipStream_t s) {
-  const size_t lds = bwd_dd_lds_bytes((int64_t)a.Nq * a.Lq);
-  hipLaunchKernelGGL(bwd_dd_index_kernel, dim3((unsigned)a.B, (unsigned)a.dd_chunks), dim3(256), lds, s, a);
-  const int64_t slabs = ((int64_t)a.B * a.Ld + a.dd_slab - 1) / a.dd_slab;
-  hipLaunchKernelGGL(bwd_dd_write_kernel<BF>, dim3((unsigned)slabs), dim3(256), 0, s, a);
-}
-
-// A second stream per device for the dQ chain, with the two events that fork
-// it from and join it to the caller's stream. Created on first use (default
-// priority, non-blocking) and kept until the process ends. One mutex orders
-// whole fork/launch/join sequences, so concurrent callers never interleave
-// their event records.
-constexpr int kBwdMaxDevices = 64;
-struct BwdSide {
-  hipStream_t st = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
-};
-std::mutex g_side_mu;
-BwdSide g_side[kBwdMaxDevices];
-
-hipError_t bwd_side(BwdSide** out) {
-  int dev = -1;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  if (dev < 0 || dev >= kBwdMaxDevices) return hipErrorInvalidDevice;
-  BwdSide& b = g_side[dev];
-  if (!b.st) {
-    hipStream_t st = nullptr;
-    hipEvent_t f = nullptr, j = nullptr;
-    if ((e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking)) != hipSuccess) return e;
-    if ((e = hipEventCreateWithFlags(&f, hipEventDisableTiming)) != hipSuccess) return e;
-    if ((e = hipEventCreateWithFlags(&j, hipEventDisableTiming)) != hipSuccess) return e;
-    b.fork = f;
-    b.join = j;
-    b.st = st;
+  const unsigned x = blockIdx.x;
+  if (x < n_gather) {
+    // wave-uniform on purpose: the chunk's lengths then come by scalar loads
+    const int by = __builtin_amdgcn_readfirstlane((int)(x / gather_x));
+    dq_partial_block<BF, FULL>(a, x - (unsigned)by * gather_x, by);
+  } else {
+    const unsigned y = x - n_gather;
+    const int b = (int)(y % (unsigned)a.B), chunk = (int)(y / (unsigned)a.B);
+    if constexpr (COUNT) {
+      dd_index_count(a, b, chunk, smem);
+    } else {
+      dd_index_sort(a, b, chunk, smem);
+    }
   }
-  *out = &b;
-  return hipSuccess;
 }
 
-// dQ and dD run as separate launches: interleaving the read-bound dQ blocks
-// with the write-bound dD blocks in one grid measured 15 % slower on config 5.
-// When both are asked for and dD is large, the dQ chain (gather, sum) runs on
-// a second stream beside the dD chain (index, writer): the two share only
-// their inputs and write disjoint outputs and workspace regions, and the
-// caller's stream waits for both. The small kernels of each chain then
-// overlap the other's large one (config 5's step 430 -> 408 us with the
-// forward). Under stream capture the chains stay on the caller's stream.
+template <bool BF, bool DENSE, bool FULL>
+__global__ void __launch_bounds__(256) bwd_back_kernel(BwdArgs a, unsigned n_sum) {
+  const unsigned x = blockIdx.x;
+  if (x < n_sum) {
+    dq_sum_block<BF>(a, x);
+  } else {
+    dd_write_block<BF, DENSE, FULL>(a, x - n_sum);
+  }
+}
+
+// Which writer: the dense one from an entry a row, or from two entries to five
+// rows where docs have lengths, whose entries then crowd fewer rows. dD alone,
+// one entry at a time against dense (us), docs all long / of U[Ld/32, Ld]
+// tokens, 128 MiB of dD at d = 128:
+//   300 tokens, entries a row 0.21: 36.3 / 33.9 against 41.4 / 36.7, 0.43: 43.7
+//   / 40.9 against 47.8 / 40.3, 0.85: 54.0 / 51.8 against 53.0 / 44.2, 1.7: 69.6
+//   / 74.0 against 59.1 / 51.6, 6.8: 158 / 206 against 104 / 103;
+//   77 tokens, 27: 451 / 745 against 236 / 291; d = 1024 and 300 tokens, 3.4:
+//   70 / 177 against 51 / 55.
+inline bool dd_dense(const BwdArgs& a) {
+  return 5 * (int64_t)a.Nq * a.Lq > (a.lengths ? 2 : 5) * (int64_t)a.Ld;
+}
+
+constexpr int64_t kBwdMaxBlocks = ((int64_t)1 << 24) - 1;  // workgroups of 256 threads per launch
+
+template <bool BF>
+hipError_t launch_front(const BwdArgs& a, int64_t n_index, int64_t n_gather, hipStream_t s) {
+  if (n_index + n_gather == 0) return hipSuccess;
+  if (n_index + n_gather > kBwdMaxBlocks && n_index && n_gather) {
+    const hipError_t e = launch_front<BF>(a, n_index, 0, s);
+    return e != hipSuccess ? e : launch_front<BF>(a, 0, n_gather, s);
+  }
+  const size_t keys = n_index ? (size_t)a.sort_n * sizeof(uint32_t) : 0;
+  const bool count = keys + dd_count_bytes(a.Ld) <= kDdIndexLds;
+  const size_t lds = n_index ? keys + (count ? dd_count_bytes(a.Ld) : 0) : 0;
+  // FULL: every 8-wide chunk lies inside d, so each gather is one 16-byte load
+  const bool full = (a.d & 7) == 0 && (a.sd_b & 7) == 0 && (a.sd_l & 7) == 0;
+  auto kern = full ? (count ? bwd_front_kernel<BF, true, true> : bwd_front_kernel<BF, true, false>)
+                   : (count ? bwd_front_kernel<BF, false, true> : bwd_front_kernel<BF, false, false>);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(n_index + n_gather)), dim3(256), lds, s, a, (unsigned)n_gather,
+                     (unsigned)(n_gather ? n_gather / a.nchunk : 1));
+  return hipGetLastError();
+}
+
+template <bool BF>
+hipError_t launch_back(const BwdArgs& a, int64_t n_sum, int64_t n_write, hipStream_t s) {
+  if (n_sum + n_write == 0) return hipSuccess;
+  if (n_sum + n_write > kBwdMaxBlocks && n_sum && n_write) {
+    const hipError_t e = launch_back<BF>(a, n_sum, 0, s);
+    return e != hipSuccess ? e : launch_back<BF>(a, 0, n_write, s);
+  }
+  auto kern = !dd_dense(a) ? bwd_back_kernel<BF, false, false>
+              : (a.d & 7) == 0 ? bwd_back_kernel<BF, true, true> : bwd_back_kernel<BF, true, false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(n_sum + n_write)), dim3(256), 0, s, a, (unsigned)n_sum);
+  return hipGetLastError();
+}
+
 template <bool BF>
 hipError_t launch_bwd_t(const BwdArgs& a, hipStream_t s) {
   const bool do_dd = a.dD && a.B > 0;
-  const int64_t dd_bytes = (int64_t)a.B * a.Ld * a.d * 2;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (a.dQ && do_dd && dd_bytes >= kBwdForkBytes && hipStreamIsCapturing(s, &cap) == hipSuccess &&
-      cap == hipStreamCaptureStatusNone) {
-    std::lock_guard<std::mutex> lock(g_side_mu);
-    BwdSide* side = nullptr;
-    hipError_t e = bwd_side(&side);
-    if (e != hipSuccess) return e;
-    if ((e = hipEventRecord(side->fork, s)) != hipSuccess) return e;
-    if ((e = hipStreamWaitEvent(side->st, side->fork, 0)) != hipSuccess) return e;
-    launch_dq_chain<BF>(a, side->st);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = hipEventRecord(side->join, side->st)) != hipSuccess) return e;
-    launch_dd_chain<BF>(a, s);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    return hipStreamWaitEvent(s, side->join, 0);
-  }
-  if (a.dQ) launch_dq_chain<BF>(a, s);
-  if (do_dd) launch_dd_chain<BF>(a, s);
-  return hipGetLastError();
+  const int64_t rows = (int64_t)a.Nq * a.Lq;
+  const int64_t n_index = do_dd ? (int64_t)a.B * a.dd_chunks : 0;
+  const int64_t n_gather = a.dQ ? (rows * ((a.d + 7) >> 3) + 255) / 256 * a.nchunk : 0;
+  const int64_t n_sum = a.dQ ? (rows * a.d + 255) / 256 : 0;
+  const int64_t n_write = do_dd ? ((int64_t)a.B * a.Ld + a.dd_slab - 1) / a.dd_slab : 0;
+  const hipError_t e = launch_front<BF>(a, n_index, n_gather, s);
+  return e != hipSuccess ? e : launch_back<BF>(a, n_sum, n_write, s);
 }
 
 }  // namespace
@@ -438,8 +602,6 @@ int bwd_sort_n(int64_t entries) {
 }
 
 int64_t bwd_dd_chunks(int64_t entries) { return entries > 0 ? (entries + kDdChunk - 1) / kDdChunk : 1; }
-
-size_t bwd_dd_lds_bytes(int64_t entries) { return (size_t)bwd_sort_n(entries) * sizeof(uint32_t); }
 
 // Workspace of the dD index: rows [chunks, B, Ld] uint32, then ent [B, entries] uint16.
 size_t bwd_dd_index_bytes(int64_t B, int64_t entries, int64_t Ld) {

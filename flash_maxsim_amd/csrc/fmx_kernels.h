@@ -146,7 +146,6 @@ constexpr int kDdChunk = 8192;                 // (query, token) entries per dD 
 int bwd_dq_chunks(int B, int rows, int d);     // rows = Nq * Lq query tokens
 int bwd_sort_n(int64_t entries);               // power of two >= min(Nq * Lq, kDdChunk) (>= 64)
 int64_t bwd_dd_chunks(int64_t entries);        // dD index chunks per doc
-size_t bwd_dd_lds_bytes(int64_t entries);      // dynamic LDS of the dD index kernel
 size_t bwd_dd_index_bytes(int64_t B, int64_t entries, int64_t Ld);  // its workspace
 int bwd_dd_slab(int d);                         // rows per dD writer workgroup
 hipError_t launch_bwd(int kind, const BwdArgs& a, hipStream_t s);

@@ -272,6 +272,28 @@ def test_bwd_exact_on_integer_grid(Nq, B, Lq, Ld, d):
     assert torch.equal(dQ.cpu().to(torch.int64), dQ_ref)
 
 
+@pytest.mark.parametrize(
+    "Nq, B, Lq, Ld, d",
+    [
+        (1, 3, 1, 1, 8),          # one entry, one row
+        (1, 4, 63, 65, 128),      # just under a wave of entries
+        (1, 4, 65, 255, 104),     # a wave and one, 13 of 16 lanes on a row
+        (5, 3, 51, 256, 16),      # 255 entries, two lanes a row
+        (1, 3, 257, 257, 100),    # one entry past four waves' quarters, d % 8 != 0
+        (33, 3, 31, 40, 128),     # 1023 entries, many a row: batches with remainders
+        (32, 3, 32, 3, 1032),     # 1024 entries on three rows wider than a wave
+        (2, 2, 4097, 300, 24),    # two index chunks
+        (1, 2, 8192, 2040, 8),    # the largest row counters beside a full chunk's keys
+        (1, 2, 8192, 2060, 8),    # the first Ld they do not fit at: the sort
+        (1, 3, 40, 5000, 64),     # a long doc, few entries
+    ],
+)
+def test_bwd_index_and_writers_exact(Nq, B, Lq, Ld, d):
+    """The dD index (counting sort, or the bitonic sort where its counters do not
+    fit) and both dD writers at their edges, exact on the integer grid."""
+    test_bwd_exact_on_integer_grid(Nq, B, Lq, Ld, d)
+
+
 def test_bwd_graph_capture_replays():
     """fmx_bwd_batched captured into a HIP graph at a size that forks the dQ
     chain when run eagerly: under capture both chains stay on the capturing
