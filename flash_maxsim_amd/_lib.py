@@ -54,6 +54,7 @@ _SIGNATURES = {
         _int,
         [_int, _ptr, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _i64, _ptr],
     ),
+    "fmx_dequantize_int8": (_int, [_ptr, _ptr, _ptr, _i64, _i64, _ptr, _ptr]),
     "fmx_fwd_packed": (
         _int,
         [_int, _ptr, _i64, _i64, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _size, _ptr],
@@ -129,6 +130,27 @@ def dtype_code(t: torch.Tensor) -> int:
     if t.dtype == torch.bfloat16:
         return FMX_DTYPE_BF16
     raise TypeError(f"kernel operands must be float16 or bfloat16, got {t.dtype}")
+
+
+def plain(*tensors: torch.Tensor) -> bool:
+    """True when a kernel may take the place of torch ops on these tensors:
+    ordinary strided GPU tensors of one device, with nothing watching the ops
+    (autograd in either mode, tracing, compilation, function transforms,
+    dispatch or function modes)."""
+    dev = tensors[0].device
+    for t in tensors:
+        if (type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or not t.is_cuda or t.device != dev:
+            return False
+        if t.layout is not torch.strided or t.is_neg() or (t.requires_grad and torch.is_grad_enabled()):
+            return False
+    return not (
+        torch.compiler.is_compiling()
+        or torch._C._get_tracing_state() is not None
+        or torch._C._functorch.maybe_current_level() is not None
+        or torch.autograd.forward_ad._current_level >= 0
+        or torch._C._len_torch_dispatch_stack()
+        or torch._C._len_torch_function_stack()
+    )
 
 
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor | None:

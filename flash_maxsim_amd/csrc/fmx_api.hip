@@ -462,12 +462,29 @@ int fmx_quantize_int8(int src_dtype, const void* src, int64_t s_stride_b, int64_
   a.scales = scales;
   a.mins = mins;
   a.sm_stride_b = sm_stride_b;
+  const int64_t code_align = esz == 4 ? 3 : 7;  // fp32 rows store four codes at a time, the others eight
   a.vec = (aligned16(src) && ((s_stride_b * esz) & 15) == 0 && ((s_stride_l * esz) & 15) == 0 &&
-           (reinterpret_cast<uintptr_t>(codes) & 7u) == 0 && (c_stride_l & 7) == 0)
+           (reinterpret_cast<uintptr_t>(codes) & code_align) == 0 && (c_stride_l & code_align) == 0)
               ? 1
               : 0;
   const int kind = src_dtype == FMX_DTYPE_F32 ? 2 : (src_dtype == FMX_DTYPE_BF16 ? 1 : 0);
   return hip_status(fmx::launch_quantize(kind, a, static_cast<hipStream_t>(stream)), "fmx_quantize_int8 launch");
+}
+
+int fmx_dequantize_int8(const uint8_t* codes, const void* scales, const void* mins, int64_t rows, int64_t d, float* out,
+                        void* stream) {
+  if (rows < 0 || d < 0 || d > INT32_MAX || (d > 0 && rows > INT64_MAX / d))
+    return fail(FMX_ERR_INVALID, "invalid sizes rows=%lld d=%lld", (long long)rows, (long long)d);
+  if (rows == 0 || d == 0) return ok();
+  if (rows * d >= ((int64_t)1 << 34)) return fail(FMX_ERR_UNSUPPORTED, "%lld values", (long long)(rows * d));
+  if (!codes || !scales || !mins || !out) return fail(FMX_ERR_INVALID, "codes, scales, mins and out must be non-null");
+  if ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(mins)) & 1u)
+    return fail(FMX_ERR_INVALID, "scales and mins must be 2-byte aligned");
+  if (reinterpret_cast<uintptr_t>(out) & 3u) return fail(FMX_ERR_INVALID, "out must be 4-byte aligned");
+  return hip_status(fmx::launch_dequantize(codes, static_cast<const uint16_t*>(scales),
+                                           static_cast<const uint16_t*>(mins), out, rows, d,
+                                           static_cast<hipStream_t>(stream)),
+                    "fmx_dequantize_int8 launch");
 }
 
 size_t fmx_topk_workspace_bytes(int64_t Nq, int64_t B, int64_t k) {

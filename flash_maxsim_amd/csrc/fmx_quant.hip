@@ -20,7 +20,8 @@
 // scales and mins.
 //
 // Mapping: LPR lanes share a token row (LPR = 8-element chunks of d rounded up
-// to a power of two, at most 64); each lane handles CPL chunks of 8 elements.
+// to a power of two, at most 64); each lane handles CPL chunks of 8 elements
+// (fp32 sources: two quads of 4 each).
 // Row min/max meet through cross-lane shuffles inside the LPR-lane group.
 #include "fmx_device.h"
 #include "fmx_kernels.h"
@@ -48,15 +49,7 @@ __device__ __forceinline__ float src_elem(const void* p, int64_t i) {
 template <int SRC, bool NT>
 __device__ __forceinline__ void load8(const void* row, int k0, int d, bool vec, float (&x)[8]) {
   if (vec && k0 + 8 <= d) {
-    if constexpr (SRC == 2) {
-      const f32x4_t a = *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(row) + k0);
-      const f32x4_t b = *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(row) + k0 + 4);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        x[i] = a[i];
-        x[4 + i] = b[i];
-      }
-    } else {
+    {
       const u32x4_t* p = reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(row) + k0);
       const u32x4_t v = NT ? __builtin_nontemporal_load(p) : *p;
 #pragma unroll
@@ -73,6 +66,25 @@ __device__ __forceinline__ void load8(const void* row, int k0, int d, bool vec, 
   } else {
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] = k0 + i < d ? src_elem<SRC>(row, k0 + i) : 0.f;
+  }
+}
+
+// Four consecutive fp32 source elements k0..k0+3 of a row, as load8. A lane's
+// eight elements are two such quads LPR quads apart, so each load instruction
+// of a wave covers whole lines, which the non-temporal policy needs; eight in a
+// row would take a 32-byte stride (with the branch to the IEEE division gone,
+// 5000 docs of 300 x 128 232 -> 165 us, 5.8 TB/s).
+template <bool NT>
+__device__ __forceinline__ void load4_f32(const void* row, int k0, int d, bool vec, float* x) {
+  const float* r = static_cast<const float*>(row);
+  if (vec && k0 + 4 <= d) {
+    const f32x4_t* p = reinterpret_cast<const f32x4_t*>(r + k0);
+    const f32x4_t v = NT ? __builtin_nontemporal_load(p) : *p;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = v[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = k0 + i < d ? r[k0 + i] : 0.f;
   }
 }
 
@@ -147,16 +159,14 @@ __device__ __forceinline__ void load8_f16(const void* row, int k0, int d, bool v
 // correction, q1 = RN(q0 + RN(a - b*q0) * y), brings it within 1 ulp, after
 // which the remainder a - b*q1 is exact as an fma and RN(q1 + rem * y) is the
 // correctly rounded quotient (Markstein's theorem; Handbook of Floating-Point
-// Arithmetic, 2nd ed., sec. 4.7), provided nothing under- or overflows. Here
-// b >= 1e-8 and a = x - lo is 0 or >= 2^-24 for fp16 sources (a nonzero
-// difference of two fp16 values is a multiple of 2^-24); bf16/fp32 sources can
-// produce tiny nonzero a, and numerators below 2^-64 (where a remainder could
-// leave the normal range) and NaN take the IEEE division (TINY_OK = false).
-template <bool TINY_OK>
+// Arithmetic, 2nd ed., sec. 4.7), provided nothing under- or overflows: b is in
+// [1e-8, 2^121) and a = x - lo is 0 or >= 2^-24 for fp16 sources (a nonzero
+// difference of two fp16 values is a multiple of 2^-24). bf16 and fp32 sources
+// can make a smaller: from 2^-64 up no step leaves the normal range, and below
+// it, where the remainders may, the quotient is below 2^-37 and every step
+// stays below 2^-34, so the code is 0 as it should be. A NaN, and an infinite
+// b, give code 0 here and in IEEE division alike.
 __device__ __forceinline__ float div_rn(float a, float b, float y) {
-  if constexpr (!TINY_OK) {
-    if (!(a >= 0x1p-64f) && a != 0.f) return a / b;
-  }
   const float q0 = a * y;
   const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, b, a), y, q0);
   const float rem = __builtin_fmaf(-q1, b, a);
@@ -221,6 +231,10 @@ __global__ void __launch_bounds__(256) quantize_kernel(QuantArgs a) {
     const int64_t jend = packed ? ((len + 3) & ~(int64_t)3) : a.Ld;
     const int64_t obase = packed ? 4 * a.tok_group[b] : b * a.Ld;
     constexpr bool PK = SRC == 0;  // packed fp16 halves (above)
+    // element i of a lane's chunk cc: k = (cc * LPR + lane) * 8 + i, or for fp32
+    // sources quads, (2 * cc * LPR + (i / 4) * LPR + lane) * 4 + i % 4
+    constexpr bool QUADS = SRC == 2;
+    auto quad_k0 = [&](int cc, int h) { return ((2 * cc + h) * LPR + lane_in_row) * 4; };
     float x[PK ? 1 : R][CPL][8];
     uint32_t xh[PK ? R : 1][CPL][4];
 #pragma unroll
@@ -232,8 +246,11 @@ __global__ void __launch_bounds__(256) quantize_kernel(QuantArgs a) {
         for (int cc = 0; cc < CPL; ++cc) {
           if constexpr (PK)
             load8_f16<(LPR >= 8)>(src, (cc * LPR + lane_in_row) * 8, a.d, a.vec != 0, xh[k][cc]);
-          else
-            load8<SRC, (SRC != 2 && LPR >= 8)>(src, (cc * LPR + lane_in_row) * 8, a.d, a.vec != 0, x[k][cc]);
+          else if constexpr (QUADS) {
+            load4_f32<(LPR >= 8)>(src, quad_k0(cc, 0), a.d, a.vec != 0, x[k][cc]);
+            load4_f32<(LPR >= 8)>(src, quad_k0(cc, 1), a.d, a.vec != 0, x[k][cc] + 4);
+          } else
+            load8<SRC, (LPR >= 8)>(src, (cc * LPR + lane_in_row) * 8, a.d, a.vec != 0, x[k][cc]);
         }
       }
     }
@@ -265,11 +282,19 @@ __global__ void __launch_bounds__(256) quantize_kernel(QuantArgs a) {
             lo = mm<false>(lo, min8_f16(xh[k][cc]));
             hi = mm<true>(hi, max8_f16(xh[k][cc]));
           }
-        } else if (k0 + 8 <= a.d) {
+        } else if (QUADS ? quad_k0(cc, 1) + 4 <= a.d : k0 + 8 <= a.d) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             lo = mm<false>(lo, x[k][cc][i]);
             hi = mm<true>(hi, x[k][cc][i]);
+          }
+        } else if constexpr (QUADS) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            if (quad_k0(cc, i >> 2) + (i & 3) < a.d) {
+              lo = mm<false>(lo, x[k][cc][i]);
+              hi = mm<true>(hi, x[k][cc][i]);
+            }
           }
         } else {
           for (int i = 0; i < 8 && k0 + i < a.d; ++i) {  // the row's last, partial chunk
@@ -285,7 +310,7 @@ __global__ void __launch_bounds__(256) quantize_kernel(QuantArgs a) {
       const float rstep = 1.0f / step;  // correctly rounded
 #pragma unroll
       for (int cc = 0; cc < CPL; ++cc) {
-        const int k0 = (cc * LPR + lane_in_row) * 8;
+        const int k0 = QUADS ? quad_k0(cc, 0) : (cc * LPR + lane_in_row) * 8;
         if (k0 >= a.d) continue;
         uint32_t w[2] = {0u, 0u};
         if constexpr (PK) {
@@ -293,17 +318,27 @@ __global__ void __launch_bounds__(256) quantize_kernel(QuantArgs a) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             const float av = (i & 1) ? sub_f16<1>(xh[k][cc][i >> 1], nlo) : sub_f16<0>(xh[k][cc][i >> 1], nlo);
-            w[i >> 2] = cvt_u8_rne(div_rn<true>(av, step, rstep), i & 3, w[i >> 2]);
+            w[i >> 2] = cvt_u8_rne(div_rn(av, step, rstep), i & 3, w[i >> 2]);
           }
         } else {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
-            w[i >> 2] = cvt_u8_rne(div_rn<SRC == 0>(x[k][cc][i] - lo, step, rstep), i & 3, w[i >> 2]);
+            w[i >> 2] = cvt_u8_rne(div_rn(x[k][cc][i] - lo, step, rstep), i & 3, w[i >> 2]);
           }
         }
-        if (a.vec && k0 + 8 <= a.d) {
-          // non-temporal: the codes are read by a later scoring call, not by
-          // this kernel (config 4's docs: 406.6 -> 400.3 us)
+        // non-temporal: the codes are read by a later scoring call, not by
+        // this kernel (config 4's docs: 406.6 -> 400.3 us)
+        if constexpr (QUADS) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int kq = quad_k0(cc, h);
+            if (a.vec && kq + 4 <= a.d) {
+              __builtin_nontemporal_store(w[h], reinterpret_cast<uint32_t*>(crow + kq));
+            } else {
+              for (int i = 0; i < 4 && kq + i < a.d; ++i) crow[kq + i] = (uint8_t)(w[h] >> (8 * i));
+            }
+          }
+        } else if (a.vec && k0 + 8 <= a.d) {
           __builtin_nontemporal_store(u32x2_t{w[0], w[1]}, reinterpret_cast<u32x2_t*>(crow + k0));
         } else {
           for (int i = 0; i < 8 && k0 + i < a.d; ++i) crow[k0 + i] = (uint8_t)(w[i >> 2] >> (8 * (i & 3)));
@@ -390,7 +425,7 @@ __global__ void __launch_bounds__(256) quantize_wide_kernel(QuantArgs a) {
     if (step < 1e-8f) step = 1e-8f;
     const float rstep = 1.0f / step;
     for (int64_t k = tid; k < a.d; k += 256) {
-      crow[k] = (uint8_t)cvt_u8_rne(div_rn<SRC == 0>(src_elem<SRC>(src, k) - lo, step, rstep), 0, 0u);
+      crow[k] = (uint8_t)cvt_u8_rne(div_rn(src_elem<SRC>(src, k) - lo, step, rstep), 0, 0u);
     }
     if (tid == 0) {
       *sp = __builtin_bit_cast(uint16_t, (_Float16)step);
@@ -420,6 +455,92 @@ hipError_t dispatch_q(const QuantArgs& a, hipStream_t s) {
 }
 
 }  // namespace
+
+namespace {
+
+// Decoding: value = code * scale + min per token row, an fp32 multiply and an
+// fp32 add, each rounded (the torch formula of the reference's dequantize_int8,
+// flash_maxsim_quant.py:31-33), in one pass: 1 byte read and 4 written per
+// value, where the formula's three tensor passes and the codes' conversion move
+// 21. A workgroup takes kDqBlock consecutive values of the [rows, d] matrix; a
+// thread takes 4 at a time (one 4-byte load, one 16-byte store, each contiguous
+// over the wave), all its loads issued first. Bound by the stores: 2000 docs of
+// 512 x 128 (655 MB) 660 -> 92.5 us, 7.1 TB/s.
+// VEC: d % 4 == 0, so four values share a row. NT: non-temporal stores, for
+// results the last-level cache would not hold.
+constexpr int kDqIter = 4, kDqBlock = 256 * 4 * kDqIter;
+
+template <bool VEC, bool NT>
+__global__ void __launch_bounds__(256) dequantize_kernel(const uint8_t* codes, const uint16_t* scales,
+                                                         const uint16_t* mins, float* out, int64_t rows, uint32_t d,
+                                                         uint32_t magic) {
+#pragma clang fp contract(off)
+  const int64_t n = rows * d;
+  const int64_t base = (int64_t)blockIdx.x * kDqBlock;
+  const int64_t row0 = base / d;
+  const uint32_t off0 = (uint32_t)(base - row0 * d);
+  const int64_t left = n - base;
+  // row of the value o places after row0's start: o / d (launch_dequantize bounds o where magic is set)
+  auto row_of = [&](uint32_t o) { return magic ? __umulhi(o, magic) : o / d; };
+  auto value = [](uint32_t c, uint16_t s, uint16_t m) {
+    const float p = (float)c * half_bits_to_float(s);
+    return p + half_bits_to_float(m);
+  };
+  if constexpr (VEC) {
+    uint32_t w[kDqIter];
+    uint16_t s[kDqIter], m[kDqIter];
+#pragma unroll
+    for (int k = 0; k < kDqIter; ++k) {
+      const int i = (k * 256 + (int)threadIdx.x) * 4;
+      if (i < left) {
+        const int64_t r = row0 + row_of(off0 + i);
+        w[k] = *reinterpret_cast<const uint32_t*>(codes + base + i);
+        s[k] = scales[r];
+        m[k] = mins[r];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kDqIter; ++k) {
+      const int i = (k * 256 + (int)threadIdx.x) * 4;
+      if (i < left) {
+        f32x4_t v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = value((w[k] >> (8 * e)) & 255u, s[k], m[k]);
+        f32x4_t* p = reinterpret_cast<f32x4_t*>(out + base + i);
+        if constexpr (NT) {
+          __builtin_nontemporal_store(v, p);
+        } else {
+          *p = v;
+        }
+      }
+    }
+  } else {
+#pragma unroll 4
+    for (int k = 0; k < 4 * kDqIter; ++k) {
+      const int i = k * 256 + (int)threadIdx.x;
+      if (i < left) {
+        const int64_t r = row0 + row_of(off0 + i);
+        out[base + i] = value(codes[base + i], scales[r], mins[r]);
+      }
+    }
+  }
+}
+
+}  // namespace
+
+hipError_t launch_dequantize(const uint8_t* codes, const uint16_t* scales, const uint16_t* mins, float* out,
+                             int64_t rows, int64_t d, hipStream_t s) {
+  const int64_t blocks = (rows * d + kDqBlock - 1) / kDqBlock;
+  if (blocks > 0x7fffff) return hipErrorInvalidValue;
+  // floor(o / d) = (o * magic) >> 32 for magic = floor(2^32 / d) + 1 while o * d < 2^32; o < d + kDqBlock
+  const uint32_t magic = d > 1 && d <= 32768 ? (uint32_t)(((uint64_t)1 << 32) / (uint64_t)d) + 1 : 0;
+  const bool vec = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(codes) & 3u) == 0 &&
+                   (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
+  const bool nt = rows * d * 4 >= ((int64_t)1 << 28);
+  auto kern = vec ? (nt ? dequantize_kernel<true, true> : dequantize_kernel<true, false>) : dequantize_kernel<false, false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, s, codes, scales, mins, out, rows, (uint32_t)d, magic);
+  return hipGetLastError();
+}
 
 hipError_t launch_quantize(int src_kind, const QuantArgs& a, hipStream_t s) {
   switch (src_kind) {

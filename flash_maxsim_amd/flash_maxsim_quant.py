@@ -79,9 +79,40 @@ def _quantize_gpu(D: torch.Tensor):
     return codes, scales, mins
 
 
+def _decodable(codes, scales, mins) -> bool:
+    """Whether fmx_dequantize_int8 takes these operands as they are."""
+    if not (torch.is_tensor(codes) and torch.is_tensor(scales) and torch.is_tensor(mins)):
+        return False
+    return (
+        codes.dtype == torch.uint8 and scales.dtype == torch.float16 and mins.dtype == torch.float16
+        and codes.dim() >= 1 and scales.shape == mins.shape == (*codes.shape[:-1], 1)
+        and _lib.plain(codes, scales, mins)
+        and codes.is_contiguous() and scales.is_contiguous() and mins.is_contiguous()
+        and 0 < codes.numel() < 1 << 34
+    )
+
+
+def _dequantize_gpu(codes, scales, mins) -> torch.Tensor:
+    out = torch.empty(codes.shape, dtype=torch.float32, device=codes.device)
+    with _device_guard(codes.device):
+        rc = _lib.load().fmx_dequantize_int8(
+            codes.data_ptr(), scales.data_ptr(), mins.data_ptr(), scales.numel(), codes.shape[-1], out.data_ptr(),
+            _lib.stream_of(codes),
+        )
+    _lib.check(rc)
+    return out
+
+
 def dequantize_int8(D_uint8: torch.Tensor, scales: torch.Tensor, mins: torch.Tensor) -> torch.Tensor:
     """float32 doc tokens back from codes: code * step + lo (reference
-    flash_maxsim_quant.py:31-33; a separate multiply and add, no fma)."""
+    flash_maxsim_quant.py:31-33; a separate multiply and add, no fma).
+
+    Stored documents on the GPU (contiguous codes with one fp16 step and lo per
+    row) are decoded in one kernel; any other operands that broadcast take the
+    torch formula, to the same bits.
+    """
+    if _decodable(D_uint8, scales, mins):
+        return _dequantize_gpu(D_uint8, scales, mins)
     return D_uint8.to(torch.float32) * scales.to(torch.float32) + mins.to(torch.float32)
 
 

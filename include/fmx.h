@@ -188,6 +188,21 @@ int fmx_quantize_int8(int src_dtype, const void* src, int64_t s_stride_b, int64_
                       int64_t c_stride_l, void* scales, void* mins, int64_t sm_stride_b, void* stream);
 
 /*
+ * The inverse: out[r, k] = codes[r, k] * scales[r] + mins[r], an fp32 multiply
+ * and an fp32 add, each rounded (no fma), over contiguous rows.
+ *
+ *   codes    [rows, d]  uint8, contiguous
+ *   scales   [rows]     fp16, contiguous, 2-byte aligned; mins likewise
+ *   out      [rows, d]  fp32, contiguous
+ * rows * d < 2^34.
+ *
+ * Replaces flash_maxsim/flash_maxsim_quant.py:31-33 (dequantize_int8, torch
+ * ops there).
+ */
+int fmx_dequantize_int8(const uint8_t* codes, const void* scales, const void* mins, int64_t rows, int64_t d, float* out,
+                        void* stream);
+
+/*
  * Packed-doc forwards (no counterpart in the reference, whose docs are always
  * padded [B, Ld, d]): the T token rows of all docs are stored back to back,
  * doc b in rows 4*tok_group[b] .. 4*tok_group[b] + lengths[b] - 1, so padding

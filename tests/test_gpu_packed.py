@@ -369,3 +369,61 @@ def test_quantize_fp16_special_values_bitwise(d):
     np.testing.assert_array_equal(got[0].cpu().numpy(), want[0].numpy())
     np.testing.assert_array_equal(_bits(got[1]), _bits(want[1]))
     np.testing.assert_array_equal(_bits(got[2]), _bits(want[2]))
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 5, 7, 60, 65, 100, 128, 132, 260, 513, 1028, 4100])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_quantize_quads_and_tiny_numerators_bitwise(dtype, d):
+    """fp32 and bf16 rows against torch's formula on the CPU, where the last quad
+    (or chunk) is partial, rows start off 16-byte boundaries, and numerators are
+    tiny: differences below 2^-64 beside zero and large ones, subnormals, rows
+    that are constant, infinite or hold a NaN."""
+    gen = torch.Generator().manual_seed(2400 + d)
+    x = torch.randn(3, 41, d, generator=gen)
+    x[0, :8] = (2.0 ** -torch.randint(40, 149, (8, d), generator=gen).float()) * torch.randint(-3, 4, (8, d), generator=gen)
+    x[0, 8:16] = torch.randint(0, 2, (8, d), generator=gen).float() * 2.0**-100
+    x[0, 16] = 0.25
+    x[0, 17, d // 2] = float("nan")
+    x[0, 18, 0] = float("inf")
+    x[0, 19, d - 1] = float("-inf")
+    x[0, 20] = torch.linspace(-3e38, 3e38, d)
+    x[0, 21:24] *= 2.0**-70
+    x = x.to(dtype)
+    for src in (x, torch.nn.functional.pad(x, (1, 2))[..., 1:1 + d]):
+        want = fm.quantize_int8(src)
+        got = fm.quantize_int8(src.to(DEV))
+        for w, g in zip(want, got):
+            g = g.cpu()
+            if w.dtype == torch.float16:
+                same = torch.isnan(w) & torch.isnan(g) | (w == g)
+                assert bool(same.all())
+            else:
+                assert torch.equal(w, g)
+
+
+@pytest.mark.parametrize(
+    "shape", [(1, 1, 1), (2, 3, 4), (5, 41, 3), (7, 11, 100), (3, 33, 128), (1, 4097, 5), (9, 57, 260), (2, 3, 32768),
+              (2, 3, 32772), (1, 2, 70001)])
+def test_dequantize_gpu_bitwise_torch(shape):
+    """The decode kernel against the torch formula on the CPU, bit for bit: rows
+    that end off a workgroup's block, d with and without whole quads, rows past
+    the reciprocal's range, codes at odd addresses, infinities and NaN; operands
+    it does not take go through the torch ops to the same values."""
+    gen = torch.Generator().manual_seed(2500 + shape[2])
+    codes = torch.randint(0, 256, shape, generator=gen, dtype=torch.uint8)
+    scales = torch.randn(*shape[:2], 1, generator=gen).half()
+    mins = torch.randn(*shape[:2], 1, generator=gen).half()
+    scales.view(-1)[0], mins.view(-1)[-1] = float("inf"), float("nan")
+    want = codes.float() * scales.float() + mins.float()
+    c, s, m = codes.to(DEV), scales.to(DEV), mins.to(DEV)
+    buf = torch.zeros(codes.numel() + 1, dtype=torch.uint8, device=DEV)
+    buf[1:] = c.reshape(-1)
+    odd = buf[1:].view(shape)
+    twice = torch.cat([c, c], dim=-1)[..., : shape[2]]  # not contiguous
+    for got in (fm.dequantize_int8(c, s, m), fm.dequantize_int8(odd, s, m), fm.dequantize_int8(twice, s, m),
+                fm.dequantize_int8(c, s.float(), m)):
+        assert got.dtype == torch.float32 and got.is_contiguous()
+        np.testing.assert_array_equal(got.cpu().numpy(), want.numpy())
+    s2 = s.clone().requires_grad_(True)
+    fm.dequantize_int8(c, s2, m).nan_to_num(0, 0, 0).sum().backward()
+    assert s2.grad is not None and s2.grad.shape == s.shape
