@@ -55,6 +55,8 @@ _SIGNATURES = {
         [_int, _ptr, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _i64, _ptr],
     ),
     "fmx_dequantize_int8": (_int, [_ptr, _ptr, _ptr, _i64, _i64, _ptr, _ptr]),
+    "fmx_packed_layout": (_int, [_ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr]),
+    "fmx_pack_rows": (_int, [_ptr, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _i64, _ptr, _ptr]),
     "fmx_fwd_packed": (
         _int,
         [_int, _ptr, _i64, _i64, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _size, _ptr],

@@ -487,6 +487,39 @@ int fmx_dequantize_int8(const uint8_t* codes, const void* scales, const void* mi
                     "fmx_dequantize_int8 launch");
 }
 
+int fmx_packed_layout(const int32_t* lengths, int64_t B, int64_t Ld, int32_t* lengths_out, int64_t* tok_group,
+                      int64_t* totals, void* stream) {
+  if (B < 0 || Ld < 0 || Ld > INT32_MAX) return fail(FMX_ERR_INVALID, "invalid sizes B=%lld Ld=%lld", (long long)B, (long long)Ld);
+  if (!totals || (B > 0 && (!lengths || !lengths_out || !tok_group)))
+    return fail(FMX_ERR_INVALID, "lengths, lengths_out, tok_group and totals must be non-null");
+  return hip_status(fmx::launch_layout(lengths, B, (int32_t)Ld, lengths_out, tok_group, totals,
+                                       static_cast<hipStream_t>(stream)),
+                    "fmx_packed_layout launch");
+}
+
+int fmx_pack_rows(const void* src, int64_t s_stride_b, int64_t s_stride_l, int64_t B, int64_t Ld, int64_t row_bytes,
+                  const int32_t* lengths, const int64_t* tok_group, int64_t tok_rows, void* dst, void* stream) {
+  if (B < 0 || Ld < 0 || row_bytes < 0 || tok_rows < 0 || s_stride_b < 0 || s_stride_l < 0)
+    return fail(FMX_ERR_INVALID, "sizes and strides must be >= 0");
+  if (B == 0 || Ld == 0 || row_bytes == 0 || tok_rows == 0) return ok();
+  if (!src || !lengths || !tok_group || !dst)
+    return fail(FMX_ERR_INVALID, "src, lengths, tok_group and dst must be non-null");
+  if (row_bytes > ((int64_t)1 << 30) || Ld > ((int64_t)1 << 31) / row_bytes)
+    return fail(FMX_ERR_UNSUPPORTED, "doc of %lld x %lld bytes exceeds 2 GiB", (long long)Ld, (long long)row_bytes);
+  fmx::PackArgs a = {};
+  a.src = src;
+  a.s_stride_b = s_stride_b;
+  a.s_stride_l = s_stride_l;
+  a.B = B;
+  a.Ld = Ld;
+  a.row_bytes = row_bytes;
+  a.lengths = lengths;
+  a.tok_group = tok_group;
+  a.tok_rows = tok_rows;
+  a.dst = dst;
+  return hip_status(fmx::launch_pack(a, static_cast<hipStream_t>(stream)), "fmx_pack_rows launch");
+}
+
 size_t fmx_topk_workspace_bytes(int64_t Nq, int64_t B, int64_t k) {
   if (Nq < 1 || B < 1 || k < 1 || k > FMX_MAX_TOPK) return 0;
   return (size_t)fmx::topk_ws_keys(Nq, B, k, fmx::topk_chunk((int)k)) * sizeof(uint64_t);

@@ -129,6 +129,20 @@ hipError_t launch_quantize(int src_kind, const QuantArgs& a, hipStream_t s);  //
 hipError_t launch_dequantize(const uint8_t* codes, const uint16_t* scales, const uint16_t* mins, float* out,
                              int64_t rows, int64_t d, hipStream_t s);
 
+// Packed docs: where each doc starts, and the copy of its rows.
+hipError_t launch_layout(const int32_t* lengths, int64_t B, int32_t Ld, int32_t* out, int64_t* tok_group,
+                         int64_t* totals, hipStream_t s);
+struct PackArgs {
+  const void* src;            // [B, Ld] rows of row_bytes bytes, strides s_stride_b, s_stride_l in bytes
+  int64_t s_stride_b, s_stride_l;
+  int64_t B, Ld, row_bytes;
+  const int32_t* lengths;     // [B]
+  const int64_t* tok_group;   // [B]: doc b starts at row 4*tok_group[b] of dst
+  int64_t tok_rows;           // rows of dst (rows outside are not written)
+  void* dst;
+};
+hipError_t launch_pack(const PackArgs& a, hipStream_t s);
+
 // Top-k selection over score rows (descending, NaN first, ties to the smaller
 // index).
 struct TopkArgs {

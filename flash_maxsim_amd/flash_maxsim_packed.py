@@ -53,15 +53,40 @@ class PackedInt8Docs(NamedTuple):
     doc_ids: torch.Tensor | None = None  # [B] int32: the doc in slot s (None: slot s is doc s)
 
 
+# Docs that the one-workgroup layout kernel takes (it walks them 4096 at a
+# time); longer lists scan faster over many workgroups, with torch's ops.
+_LAYOUT_DOCS = 1 << 16
+
+
+def _layout_gpu(lengths: torch.Tensor, Ld: int):
+    """_layout of GPU lengths in one kernel and one read back."""
+    B, dev = lengths.numel(), lengths.device
+    out = torch.empty(B, dtype=torch.int32, device=dev)
+    tok_group = torch.empty(B, dtype=torch.int64, device=dev)
+    totals = torch.empty(2, dtype=torch.int64, device=dev)
+    with _device_guard(dev):
+        rc = _lib.load().fmx_packed_layout(lengths.data_ptr(), B, Ld, out.data_ptr(), tok_group.data_ptr(),
+                                           totals.data_ptr(), _lib.stream_of(lengths))
+    _lib.check(rc)
+    T, max_len = totals.tolist()
+    return out, tok_group, T, max_len, None
+
+
 def _layout(B: int, Ld: int, doc_lengths, device, sort_by_length: bool = False):
     """(lengths int32 clamped to [0, Ld] and tok_group int64, both per doc;
     total rows T; max_len; the slot order: doc ids longest first (int64,
     stable among equal lengths) when sort_by_length, else None)."""
     if doc_lengths is None:
         lengths = torch.full((B,), Ld, dtype=torch.int32, device=device)
+        if not sort_by_length and Ld > 0:  # every doc alike: nothing to read back
+            g = (Ld + 3) // 4
+            return lengths, torch.arange(0, B * g, g, device=device), 4 * B * g, Ld if B > 0 else 0, None
     else:
         assert doc_lengths.numel() == B, f"doc_lengths has {doc_lengths.numel()} entries, expected {B}"
-        lengths = doc_lengths.to(device=device, dtype=torch.int32).reshape(B).clamp(0, Ld).contiguous()
+        lengths = doc_lengths.to(device=device, dtype=torch.int32).reshape(B)
+        if not sort_by_length and 0 < B <= _LAYOUT_DOCS and Ld < 1 << 31 and _lib.plain(lengths):
+            return _layout_gpu(lengths.contiguous(), Ld)
+        lengths = lengths.clamp(0, Ld).contiguous()
     order = torch.sort(lengths, descending=True, stable=True).indices if sort_by_length and B > 0 else None
     groups = (lengths.to(torch.int64) + 3) // 4
     slot_groups = groups if order is None else groups[order]
@@ -94,6 +119,19 @@ def _ids(docs) -> tuple:
     return (ids,)
 
 
+def _pack_gpu(D: torch.Tensor, lengths: torch.Tensor, tok_group: torch.Tensor, T: int) -> torch.Tensor:
+    B, Ld, d = D.shape
+    dev, size = D.device, D.element_size()
+    tokens = torch.empty(T, d, dtype=D.dtype, device=dev)
+    with _device_guard(dev):
+        rc = _lib.load().fmx_pack_rows(
+            D.data_ptr(), D.stride(0) * size, D.stride(1) * size, B, Ld, d * size, lengths.data_ptr(),
+            tok_group.data_ptr(), T, tokens.data_ptr(), _lib.stream_of(D),
+        )
+    _lib.check(rc)
+    return tokens
+
+
 def pack_docs(D: torch.Tensor, doc_lengths=None, sort_by_length: bool = False) -> PackedDocs:
     """Packs the first doc_lengths[b] tokens of each doc of D [B, Ld, d]
     (all Ld when doc_lengths is None; lengths are clamped to [0, Ld]).
@@ -102,12 +140,15 @@ def pack_docs(D: torch.Tensor, doc_lengths=None, sort_by_length: bool = False) -
     assert D.dim() == 3
     B, Ld, d = D.shape
     lengths, tok_group, T, max_len, order = _layout(B, Ld, doc_lengths, D.device, sort_by_length)
-    tokens = torch.zeros(T, d, dtype=D.dtype, device=D.device)
-    if T:
-        j = torch.arange(Ld, device=D.device)
-        valid = j[None, :] < lengths[:, None].to(torch.int64)
-        rows = (4 * tok_group[:, None] + j[None, :])[valid]
-        tokens[rows] = D[valid]
+    if T and d and _lib.plain(D) and not D.is_complex() and D.stride(2) == 1 and Ld * d * D.element_size() < 1 << 30:
+        tokens = _pack_gpu(D, lengths, tok_group, T)
+    else:
+        tokens = torch.zeros(T, d, dtype=D.dtype, device=D.device)
+        if T:
+            j = torch.arange(Ld, device=D.device)
+            valid = j[None, :] < lengths[:, None].to(torch.int64)
+            rows = (4 * tok_group[:, None] + j[None, :])[valid]
+            tokens[rows] = D[valid]
     slot_lengths, slot_group, doc_ids = _slots(lengths, tok_group, order)
     return PackedDocs(tokens, slot_group, slot_lengths, max_len, doc_ids)
 

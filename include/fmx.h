@@ -203,6 +203,28 @@ int fmx_dequantize_int8(const uint8_t* codes, const void* scales, const void* mi
                         void* stream);
 
 /*
+ * The layout of packed docs (no counterpart in the reference), doc by doc in
+ * order: lengths_out[b] = lengths[b] clamped to [0, Ld], tok_group[b] = the
+ * sum of ceil(lengths_out / 4) over the docs before b, totals[0] = 4 times
+ * that sum over all docs (the rows T of the packed tensors), totals[1] = the
+ * longest length. lengths [B] int32; lengths_out [B] int32 (may be lengths
+ * itself), tok_group [B] int64 and totals [2] int64 are device memory. One
+ * workgroup: meant for up to some ten thousand docs.
+ */
+int fmx_packed_layout(const int32_t* lengths, int64_t B, int64_t Ld, int32_t* lengths_out, int64_t* tok_group,
+                      int64_t* totals, void* stream);
+
+/*
+ * Packs rows of any type (no counterpart in the reference): the first
+ * lengths[b] rows of each doc of src [B, Ld], rows of row_bytes bytes at byte
+ * strides s_stride_b and s_stride_l, to rows 4*tok_group[b] .. of dst
+ * [tok_rows] (contiguous rows); rows up to the doc's next multiple of 4 are
+ * zeroed, and rows outside [0, tok_rows) are not written.
+ */
+int fmx_pack_rows(const void* src, int64_t s_stride_b, int64_t s_stride_l, int64_t B, int64_t Ld, int64_t row_bytes,
+                  const int32_t* lengths, const int64_t* tok_group, int64_t tok_rows, void* dst, void* stream);
+
+/*
  * Packed-doc forwards (no counterpart in the reference, whose docs are always
  * padded [B, Ld, d]): the T token rows of all docs are stored back to back,
  * doc b in rows 4*tok_group[b] .. 4*tok_group[b] + lengths[b] - 1, so padding

@@ -427,3 +427,40 @@ def test_dequantize_gpu_bitwise_torch(shape):
     s2 = s.clone().requires_grad_(True)
     fm.dequantize_int8(c, s2, m).nan_to_num(0, 0, 0).sum().backward()
     assert s2.grad is not None and s2.grad.shape == s.shape
+
+
+@pytest.mark.parametrize("B, Ld, d", [(1, 1, 1), (5, 7, 3), (9, 33, 100), (300, 20, 64), (3, 300, 128), (4, 9, 2050),
+                                      (4095, 3, 2), (4097, 5, 8), (65537, 2, 1)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.uint8, torch.float64])
+def test_pack_docs_gpu_equals_cpu(B, Ld, d, dtype):
+    """pack_docs on GPU tensors (layout and copy kernels, up to 65536 docs) against
+    the torch ops it runs on the CPU: lengths below 0 and past Ld, rows of any
+    width and alignment, strided and expanded docs, the sorted layout, no lengths."""
+    gen = torch.Generator().manual_seed(2600 + B + d)
+    x = torch.randint(0, 200, (B, Ld, d + 1), generator=gen).to(dtype)
+    lengths = torch.randint(-1, Ld + 2, (B,), generator=gen)
+    lengths[0] = Ld
+    views = [x[..., :d].contiguous(), x[..., 1:], x[:1, :, :d].expand(B, Ld, d)]
+    for v in views:
+        base = x.to(DEV)
+        g = {0: base[..., :d].contiguous(), 1: base[..., 1:], 2: base[:1, :, :d].expand(B, Ld, d)}[
+            next(i for i, u in enumerate(views) if u is v)]
+        for ln, srt in ((lengths, False), (lengths, True), (None, False), (None, True)):
+            want = fm.pack_docs(v, ln, srt)
+            got = fm.pack_docs(g, None if ln is None else ln.to(DEV), srt)
+            assert got.max_len == want.max_len
+            assert (got.doc_ids is None) == (want.doc_ids is None)
+            for a, b in zip(got[:3], want[:3]):
+                assert a.dtype == b.dtype and a.is_contiguous() and torch.equal(a.cpu(), b)
+            if want.doc_ids is not None:
+                assert torch.equal(got.doc_ids.cpu(), want.doc_ids)
+
+
+def test_pack_docs_keeps_gradients():
+    D = torch.randn(3, 5, 8, generator=torch.Generator().manual_seed(1)).to(DEV).requires_grad_(True)
+    out = fm.pack_docs(D, torch.tensor([2, 0, 5])).tokens
+    out.sum().backward()
+    want = torch.zeros(3, 5, 8)
+    want[0, :2] = 1
+    want[2] = 1
+    assert torch.equal(D.grad.cpu(), want)
