@@ -42,37 +42,37 @@ struct Elem<true> {
   }
 };
 
-// Loads elements k0 .. k0+7 (those < d) of a 2-byte row as fp32.
+// Loads elements k0 .. k0+7 of a 2-byte row as fp32, k0 < d: one 16-byte load
+// (rows start 16-byte aligned, a multiple of 8 elements apart). Elements at or
+// past d may be anything; they reach only sums that are not stored.
 template <bool BF>
-__device__ __forceinline__ void load8(const uint16_t* row, int k0, int d, float (&x)[8]) {
-  if (k0 + 8 <= d) {
-    const uint4 v = *reinterpret_cast<const uint4*>(row + k0);
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+__device__ __forceinline__ void load8(const uint16_t* row, int k0, float (&x)[8]) {
+  const u32x4_t v = *reinterpret_cast<const u32x4_t*>(row + k0);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      x[2 * e] = Elem<BF>::to_f(w[e] & 0xffffu);
-      x[2 * e + 1] = Elem<BF>::to_f(w[e] >> 16);
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = (k0 + e < d) ? Elem<BF>::to_f(row[k0 + e]) : 0.f;
+  for (int e = 0; e < 4; ++e) {
+    x[2 * e] = Elem<BF>::to_f(v[e] & 0xffffu);
+    x[2 * e + 1] = Elem<BF>::to_f(v[e] >> 16);
   }
 }
 
 // Stores elements k0 .. k0+7 (those < d); 16-byte stores need d % 8 == 0 so
-// that every row of the contiguous output starts 16-byte aligned. dD is
+// that every row of the contiguous output starts 16-byte aligned, 8-byte ones
+// d % 4 == 0 (backward of 18 queries of 32 tokens over 2000 docs of 1048 x 100: 512
+// -> 165 us with whole-row loads and these). dD is
 // written once and read only by the optimiser later: non-temporal stores
 // stream it out instead of leaving it dirty in the caches, where its
 // write-back would compete with the next forward's reads.
 template <bool BF>
 __device__ __forceinline__ void store8(uint16_t* row, int k0, int d, const float (&x)[8]) {
+  u32x4_t v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    v[i] = (uint32_t)Elem<BF>::from_f(x[2 * i]) | ((uint32_t)Elem<BF>::from_f(x[2 * i + 1]) << 16);
   if ((d & 7) == 0) {
-    u32x4_t v;
-    v[0] = (uint32_t)Elem<BF>::from_f(x[0]) | ((uint32_t)Elem<BF>::from_f(x[1]) << 16);
-    v[1] = (uint32_t)Elem<BF>::from_f(x[2]) | ((uint32_t)Elem<BF>::from_f(x[3]) << 16);
-    v[2] = (uint32_t)Elem<BF>::from_f(x[4]) | ((uint32_t)Elem<BF>::from_f(x[5]) << 16);
-    v[3] = (uint32_t)Elem<BF>::from_f(x[6]) | ((uint32_t)Elem<BF>::from_f(x[7]) << 16);
     __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(row + k0));
+  } else if ((d & 3) == 0) {
+    __builtin_nontemporal_store(u32x2_t{v[0], v[1]}, reinterpret_cast<u32x2_t*>(row + k0));
+    if (k0 + 4 < d) __builtin_nontemporal_store(u32x2_t{v[2], v[3]}, reinterpret_cast<u32x2_t*>(row + k0 + 4));
   } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e)
@@ -97,7 +97,7 @@ __device__ __forceinline__ int doc_len(const BwdArgs& a, int b) {
 // Positions past the chunk read its last doc again and, like empty docs, are
 // skipped (not multiplied by zero: a row may hold NaN padding); whether a doc
 // counts depends on the doc alone, so the skip is uniform over the wave.
-template <bool BF, bool FULL>
+template <bool BF>
 __device__ __forceinline__ void dq_partial_block(const BwdArgs& a, int64_t bx, int by) {
   constexpr int DB = 8;
   const int nkc = (a.d + 7) >> 3;
@@ -135,17 +135,7 @@ __device__ __forceinline__ void dq_partial_block(const BwdArgs& a, int64_t bx, i
 #pragma unroll
     for (int u = 0; u < DB; ++u) {
       const uint16_t* row = D + (int64_t)bi[u] * a.sd_b + (int64_t)j[u] * a.sd_l;
-      if constexpr (FULL) {
-        const uint4 v = *reinterpret_cast<const uint4*>(row + k0);
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x[u][2 * e] = Elem<BF>::to_f(w[e] & 0xffffu);
-          x[u][2 * e + 1] = Elem<BF>::to_f(w[e] >> 16);
-        }
-      } else {
-        load8<BF>(row, k0, a.d, x[u]);
-      }
+      load8<BF>(row, k0, x[u]);
     }
 #pragma unroll
     for (int u = 0; u < DB; ++u)
@@ -343,9 +333,8 @@ __device__ __forceinline__ void dd_index_sort(const BwdArgs& a, int b, int chunk
 // kDdAhead: eight rows ahead cost a third of the waves (five per SIMD, seven
 // with four: 1000 docs of 512 x 1024 under 256 tokens 357 -> 323 us, 4000 of
 // 300 x 128 under 200 144 -> 128; the smallest batches 35 -> 38).
-// FULL (DENSE): every 8-wide chunk lies inside d (d % 8 == 0).
 constexpr int kDdAhead = 4;
-template <bool BF, bool DENSE, bool FULL>
+template <bool BF, bool DENSE>
 __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
   const int nkc = (a.d + 7) >> 3;
   const int lane = threadIdx.x & 63;
@@ -398,7 +387,7 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
             const int qi = e / a.Lq, q = e - qi * a.Lq;
             const float g = a.grad[(int64_t)qi * a.g_n + (int64_t)b * a.g_b];
             float x[8];
-            load8<BF>(Q + (int64_t)qi * a.sq_n + (int64_t)q * a.sq_l, k0, a.d, x);
+            load8<BF>(Q + (int64_t)qi * a.sq_n + (int64_t)q * a.sq_l, k0, x);
 #pragma unroll
             for (int k = 0; k < 8; ++k) acc[k] = fmaf(g, x[k], acc[k]);
           }
@@ -439,16 +428,7 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
               const int src = (lane & ~(L - 1)) + u0 + u;
               const uint16_t* row = Q + (int64_t)lane_fetch(off, src) * 8;
               gu[u] = __builtin_bit_cast(float, lane_fetch(__builtin_bit_cast(uint32_t, g), src));
-              if constexpr (FULL) {
-                const u32x4_t v = *reinterpret_cast<const u32x4_t*>(row + k0);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                  x[u][2 * i] = Elem<BF>::to_f(v[i] & 0xffffu);
-                  x[u][2 * i + 1] = Elem<BF>::to_f(v[i] >> 16);
-                }
-              } else {
-                load8<BF>(row, k0, a.d, x[u]);
-              }
+              load8<BF>(row, k0, x[u]);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u)
@@ -489,14 +469,14 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
 // stores of dD lower the rate of both (interleaved in one grid 15 % slower; on
 // two streams 4 % slower than this with 1000 docs of 512 x 1024, and its event
 // waits cost 20 us where dD is 77 MB, 41.8 -> 24.0 us).
-template <bool BF, bool FULL, bool COUNT>
+template <bool BF, bool COUNT>
 __global__ void __launch_bounds__(256) bwd_front_kernel(BwdArgs a, unsigned n_gather, unsigned gather_x) {
   extern __shared__ uint32_t smem[];
   const unsigned x = blockIdx.x;
   if (x < n_gather) {
     // wave-uniform on purpose: the chunk's lengths then come by scalar loads
     const int by = __builtin_amdgcn_readfirstlane((int)(x / gather_x));
-    dq_partial_block<BF, FULL>(a, x - (unsigned)by * gather_x, by);
+    dq_partial_block<BF>(a, x - (unsigned)by * gather_x, by);
   } else {
     const unsigned y = x - n_gather;
     const int b = (int)(y % (unsigned)a.B), chunk = (int)(y / (unsigned)a.B);
@@ -508,13 +488,13 @@ __global__ void __launch_bounds__(256) bwd_front_kernel(BwdArgs a, unsigned n_ga
   }
 }
 
-template <bool BF, bool DENSE, bool FULL>
+template <bool BF, bool DENSE>
 __global__ void __launch_bounds__(256) bwd_back_kernel(BwdArgs a, unsigned n_sum) {
   const unsigned x = blockIdx.x;
   if (x < n_sum) {
     dq_sum_block<BF>(a, x);
   } else {
-    dd_write_block<BF, DENSE, FULL>(a, x - n_sum);
+    dd_write_block<BF, DENSE>(a, x - n_sum);
   }
 }
 
@@ -543,10 +523,7 @@ hipError_t launch_front(const BwdArgs& a, int64_t n_index, int64_t n_gather, hip
   const size_t keys = n_index ? (size_t)a.sort_n * sizeof(uint32_t) : 0;
   const bool count = keys + dd_count_bytes(a.Ld) <= kDdIndexLds;
   const size_t lds = n_index ? keys + (count ? dd_count_bytes(a.Ld) : 0) : 0;
-  // FULL: every 8-wide chunk lies inside d, so each gather is one 16-byte load
-  const bool full = (a.d & 7) == 0 && (a.sd_b & 7) == 0 && (a.sd_l & 7) == 0;
-  auto kern = full ? (count ? bwd_front_kernel<BF, true, true> : bwd_front_kernel<BF, true, false>)
-                   : (count ? bwd_front_kernel<BF, false, true> : bwd_front_kernel<BF, false, false>);
+  auto kern = count ? bwd_front_kernel<BF, true> : bwd_front_kernel<BF, false>;
   hipLaunchKernelGGL(kern, dim3((unsigned)(n_index + n_gather)), dim3(256), lds, s, a, (unsigned)n_gather,
                      (unsigned)(n_gather ? n_gather / a.nchunk : 1));
   return hipGetLastError();
@@ -559,8 +536,7 @@ hipError_t launch_back(const BwdArgs& a, int64_t n_sum, int64_t n_write, hipStre
     const hipError_t e = launch_back<BF>(a, n_sum, 0, s);
     return e != hipSuccess ? e : launch_back<BF>(a, 0, n_write, s);
   }
-  auto kern = !dd_dense(a) ? bwd_back_kernel<BF, false, false>
-              : (a.d & 7) == 0 ? bwd_back_kernel<BF, true, true> : bwd_back_kernel<BF, true, false>;
+  auto kern = dd_dense(a) ? bwd_back_kernel<BF, true> : bwd_back_kernel<BF, false>;
   hipLaunchKernelGGL(kern, dim3((unsigned)(n_sum + n_write)), dim3(256), 0, s, a, (unsigned)n_sum);
   return hipGetLastError();
 }

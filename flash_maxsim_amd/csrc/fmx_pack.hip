@@ -18,7 +18,7 @@ constexpr int kLayoutPer = 4;  // consecutive docs per thread and step
 // rows, and totals[0] = rows in all, totals[1] = the longest length. One
 // workgroup walks the docs in order, kLayoutThreads * kLayoutPer a step, its
 // sums meeting through LDS: a step is bound by its two barriers, and the whole
-// by launch latency (5000 docs @LY@ us).
+// by launch latency (5000 docs 7 us).
 __global__ void __launch_bounds__(kLayoutThreads) layout_kernel(const int32_t* lengths, int64_t B, int32_t Ld,
                                                                 int32_t* out, int64_t* tok_group, int64_t* totals) {
   __shared__ int64_t wsum[kLayoutThreads / 64];
@@ -81,7 +81,7 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_kernel(const int32_t* l
 // multiples of). A workgroup takes kPackBlock consecutive units of one packed
 // doc, whose rows are contiguous there; rows past the doc's length, up to its
 // group's end, are zeros. Bound by memory: 10799 docs of 197 x 128 fp16 (545 MB
-// read and as many written) @PK@.
+// read and as many written) 2012 -> 201 us, 5.4 TB/s.
 // NT: both sides non-temporal, for docs the last-level cache would not hold.
 constexpr int kPackIter = 4, kPackBlock = 256 * kPackIter;
 
