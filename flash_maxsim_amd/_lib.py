@@ -112,6 +112,21 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The native host path (csrc/native.cpp): one function per ordinary call,
+    each returning None where the call has to take the Python path."""
+    global _native
+    if _native is None:
+        load()  # names what is missing; the module links to the same library
+        from . import _native as module
+
+        _native = module
+    return _native
+
+
 def check(rc: int) -> None:
     if rc != 0:
         msg = load().fmx_last_error().decode(errors="replace")

@@ -124,6 +124,9 @@ def flash_maxsim(Q: torch.Tensor, D: torch.Tensor, doc_lengths=None) -> torch.Te
     best similarity among doc b's first doc_lengths[b] tokens (all Ld when
     doc_lengths is None). Reference signature: flash_maxsim.py:221.
     """
+    out = _lib.native().score(Q, D, doc_lengths)
+    if out is not None:
+        return out
     assert Q.ndim == 2 and D.ndim == 3 and Q.size(1) == D.size(2)
     Lq, d = Q.shape
     B, Ld = D.shape[:2]
@@ -142,6 +145,9 @@ def flash_maxsim_batched(Q: torch.Tensor, D: torch.Tensor, doc_lengths=None,
     doc_lengths, if given, holds Nq*B entries in that order. Reference
     signature: flash_maxsim.py:233.
     """
+    out = _lib.native().batched(Q, D, doc_lengths, shared_docs)
+    if out is not None:
+        return out
     assert Q.ndim == 3 and Q.size(2) == D.size(-1)
     Nq, Lq, d = Q.shape
     if shared_docs:
@@ -177,7 +183,8 @@ class _FlashMaxSimFn(torch.autograd.Function):
         B, Ld = D.shape[:2]
         kdt = _kernel_dtype(Q, D)
         Qk, Dk = _prep(Q3, kdt), _prep(D, kdt)
-        scores, argmax = _launch_fwd(Qk, Dk, lengths, Nq, B, Lq, Ld, d, True, True)
+        out = _lib.native().forward(Qk, Dk, lengths, d)
+        scores, argmax = out if out is not None else _launch_fwd(Qk, Dk, lengths, Nq, B, Lq, Ld, d, True, True)
         ctx.save_for_backward(Qk, Dk, argmax, lengths)
         ctx.d = d
         ctx.batched = batched
@@ -190,6 +197,11 @@ class _FlashMaxSimFn(torch.autograd.Function):
         Nq, Lq = Qk.shape[:2]
         B, Ld = Dk.shape[:2]
         need_q, need_d = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+        grad = grad_scores if ctx.batched else grad_scores.unsqueeze(0)
+        out = _lib.native().backward(Qk, Dk, lengths, argmax, grad, d, need_q, need_d)
+        if out is not None:
+            grad_Q, grad_D = out
+            return (grad_Q if ctx.batched or grad_Q is None else grad_Q[0]), grad_D, None
         dev = _check_devices(Qk, Dk, grad_scores)
         grad_Q = torch.empty(Nq, Lq, d, device=dev, dtype=Qk.dtype) if need_q else None
         grad_D = torch.empty(B, Ld, d, device=dev, dtype=Dk.dtype) if need_d else None

@@ -183,6 +183,9 @@ def quantize_int8_packed(D: torch.Tensor, doc_lengths=None, sort_by_length: bool
 def flash_maxsim_packed(Q: torch.Tensor, docs: PackedDocs) -> torch.Tensor:
     """flash_maxsim over packed docs: float32 [B], equal to
     flash_maxsim(Q, D, lengths) on the padded docs."""
+    out = _lib.native().packed(Q, docs.tokens, docs.tok_group, docs.lengths, docs.max_len, docs.doc_ids)
+    if out is not None:
+        return out
     assert Q.dim() == 2 and docs.tokens.dim() == 2 and Q.size(1) == docs.tokens.size(1)
     Lq, d = Q.shape
     B = docs.lengths.numel()
@@ -213,6 +216,10 @@ def flash_maxsim_packed(Q: torch.Tensor, docs: PackedDocs) -> torch.Tensor:
 def flash_maxsim_int8_packed(Q: torch.Tensor, docs: PackedInt8Docs) -> torch.Tensor:
     """flash_maxsim_int8 over packed uint8 docs: float32 [B], equal to
     flash_maxsim_int8(Q, codes, scales, mins, lengths) on the padded docs."""
+    out = _lib.native().int8_packed(Q, docs.codes, docs.scales, docs.mins, docs.tok_group, docs.lengths, docs.max_len,
+                                    docs.doc_ids)
+    if out is not None:
+        return out
     assert Q.dim() == 2 and docs.codes.dim() == 2 and Q.size(1) == docs.codes.size(1)
     Lq, d = Q.shape
     B = docs.lengths.numel()

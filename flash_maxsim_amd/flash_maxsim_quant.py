@@ -138,6 +138,9 @@ def flash_maxsim_int8(
     of shape [B, Ld, 1] or [B, Ld]. Reference signature:
     flash_maxsim_quant.py:105.
     """
+    out = _lib.native().int8(Q, D_uint8, scales, mins, doc_lengths)
+    if out is not None:
+        return out
     assert Q.dim() == 2 and D_uint8.dim() == 3 and Q.shape[1] == D_uint8.shape[2]
     Lq, d = Q.shape
     B, Ld, _ = D_uint8.shape

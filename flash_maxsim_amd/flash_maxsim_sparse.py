@@ -26,6 +26,9 @@ def flash_maxsim_sparse(
     (a row outside [0, Lq) contributes a zero query token), doc_lengths
     optional [B]. Reference signature: flash_maxsim_sparse.py:98.
     """
+    out = _lib.native().sparse(Q, D, indices, doc_lengths)
+    if out is not None:
+        return out
     assert Q.dim() == 2 and D.dim() == 3 and indices.dim() == 2
     Lq, d = Q.shape
     B, Ld, _ = D.shape

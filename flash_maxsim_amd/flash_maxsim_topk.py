@@ -53,6 +53,9 @@ def flash_maxsim_topk(Q: torch.Tensor, D: torch.Tensor, k: int, doc_lengths=None
     One call of fmx_fwd_topk (the scoring and the selection kernels back to
     back); the results equal topk_scores(flash_maxsim(Q, D), k).
     """
+    out = _lib.native().topk(Q, D, k, doc_lengths)
+    if out is not None:
+        return out
     assert Q.ndim == 2 and D.ndim == 3 and Q.size(1) == D.size(2)
     Lq, d = Q.shape
     B, Ld = D.shape[:2]

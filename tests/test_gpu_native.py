@@ -1,0 +1,171 @@
+"""The native host path (csrc/native.cpp) against the Python path it stands in
+front of: every form of operand that either takes gives the same bits, and what
+one refuses the other refuses in the same words."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import flash_maxsim_amd as fm
+from conftest import sim
+from flash_maxsim_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+class _Absent:
+    """A native module that takes no call."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def both(monkeypatch, call):
+    """(result or error of the call as it is, the same by the Python path alone)."""
+    out = []
+    for absent in (False, True):
+        with monkeypatch.context() as m:
+            if absent:
+                m.setattr(_lib, "native", lambda: _Absent())
+            try:
+                out.append(call())
+            except Exception as e:  # noqa: BLE001
+                out.append((type(e), str(e)))
+    return out
+
+
+def same(a, b):
+    if torch.is_tensor(a):
+        assert a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride()
+        return torch.equal(a, b)
+    if isinstance(a, tuple) and a and torch.is_tensor(a[0]):
+        return len(a) == len(b) and all(same(x, y) for x, y in zip(a, b))
+    return a == b
+
+
+def forms(t):
+    """t and other layouts of the same values: rows of a wider buffer (in place and
+    off alignment), transposed storage, a copy at an odd address."""
+    wide = torch.zeros(*t.shape[:-1], t.shape[-1] + 8, dtype=t.dtype, device=t.device)
+    wide[..., : t.shape[-1]] = t
+    odd = torch.zeros(*t.shape[:-1], t.shape[-1] + 1, dtype=t.dtype, device=t.device)
+    odd[..., 1:] = t
+    turned = t.transpose(0, 1).contiguous().transpose(0, 1)
+    flat = torch.zeros(t.numel() + 1, dtype=t.dtype, device=t.device)
+    flat[1:] = t.reshape(-1)
+    return [t, wide[..., : t.shape[-1]], odd[..., 1:], turned, flat[1:].view(t.shape)]
+
+
+@pytest.mark.parametrize("dtypes", [("f16", "f16"), ("bf16", "bf16"), ("f16", "bf16"), ("f32", "f32")])
+@pytest.mark.parametrize("d", [64, 100, 128, 300])
+def test_scoring_forms(monkeypatch, dtypes, d):
+    kinds = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}
+    Q = sim((3, 20, d), 1, torch.float32).to(kinds[dtypes[0]]).to(DEV)
+    D = sim((3, 6, 37, d), 2, torch.float32).to(kinds[dtypes[1]]).to(DEV)
+    ln = torch.tensor([37, 0, 5, 40, -1, 16], device=DEV)
+    idx = torch.randint(-1, 22, (6, 7), generator=torch.Generator().manual_seed(3)).to(DEV)
+    lengths = [None, ln, ln.to(torch.int32), ln.to(torch.int32).cpu(), torch.stack([ln, ln], 1).to(torch.int32)[:, 0]]
+    for q in forms(Q[0]):
+        for x in forms(D[0]):
+            for le in lengths:
+                assert same(*both(monkeypatch, lambda: fm.flash_maxsim(q, x, le)))
+                assert same(*both(monkeypatch, lambda: fm.flash_maxsim_topk(q, x, 4, le)))
+            for ix in (idx, idx.to(torch.int32), idx.to(torch.int32).t().contiguous().t()):
+                assert same(*both(monkeypatch, lambda: fm.flash_maxsim_sparse(q, x, ix, lengths[2])))
+            assert same(*both(monkeypatch, lambda: fm.flash_maxsim_packed(q, fm.pack_docs(x, ln, True))))
+    for q in forms(Q):
+        for x in forms(D[0]):
+            assert same(*both(monkeypatch, lambda: fm.flash_maxsim_batched(q, x, lengths[2])))
+        for x in forms(D):
+            for le in (None, torch.stack([ln, ln, ln]).to(torch.int32)):
+                assert same(*both(monkeypatch, lambda: fm.flash_maxsim_batched(q, x, le, False)))
+
+
+def test_int8_forms(monkeypatch):
+    Q = sim((20, 128), 4, torch.float16).to(DEV)
+    codes, sc, mn = (t.to(DEV) for t in fm.quantize_int8(sim((6, 36, 128), 5, torch.float32)))
+    ln = torch.tensor([36, 0, 5, 40, -1, 16], dtype=torch.int32, device=DEV)
+    wide = torch.zeros(6, 40, 1, dtype=torch.float16, device=DEV)
+    wide[:, :36] = sc
+    for q in forms(Q) + [Q.float()]:
+        for x in forms(codes):
+            for s, m in ((sc, mn), (sc[..., 0], mn[..., 0]), (wide[:, :36], mn), (sc.float(), mn)):
+                assert same(*both(monkeypatch, lambda: fm.flash_maxsim_int8(q, x, s, m, ln)))
+        p = fm.quantize_int8_packed(sim((6, 36, 128), 5, torch.float32).to(DEV), ln, True)
+        for docs in (p, p._replace(scales=p.scales.float()), p._replace(tok_group=p.tok_group.clone())):
+            assert same(*both(monkeypatch, lambda: fm.flash_maxsim_int8_packed(q, docs)))
+
+
+@pytest.mark.parametrize("nq", [1, 3])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_training_forms(monkeypatch, nq, dtype):
+    Q = sim((nq, 20, 100), 6, torch.float32).to(dtype).to(DEV)
+    D = sim((6, 37, 100), 7, torch.float32).to(dtype).to(DEV)
+    ln = torch.tensor([37, 1, 5, 37, 9, 16], dtype=torch.int32, device=DEV)
+    g = torch.randn(nq, 6, generator=torch.Generator().manual_seed(8)).to(DEV)
+
+    def step(need_q, need_d, grad):
+        q = (Q if nq > 1 else Q[0]).clone().requires_grad_(need_q)
+        x = D.clone().requires_grad_(need_d)
+        s = (fm.flash_maxsim_train_batched if nq > 1 else fm.flash_maxsim_train)(q, x, ln)
+        if grad is None:
+            s.sum().backward()
+        else:
+            s.backward(grad)
+        return tuple(t for t in (s.detach(), q.grad, x.grad) if t is not None)
+
+    g1 = g if nq > 1 else g[0]
+    turned = g.t().contiguous().t() if nq > 1 else torch.stack([g[0], g[0]], 1)[:, 0]
+    for need_q, need_d in ((True, True), (True, False), (False, True)):
+        for grad in (None, g1, turned, torch.zeros_like(g1)):
+            assert same(*both(monkeypatch, lambda: step(need_q, need_d, grad)))
+
+
+def test_refusals(monkeypatch):
+    Q, D = sim((20, 128), 9, torch.float16).to(DEV), sim((6, 36, 128), 10, torch.float16).to(DEV)
+    calls = [
+        lambda: fm.flash_maxsim(Q, D[0]),
+        lambda: fm.flash_maxsim(Q[:, :64], D),
+        lambda: fm.flash_maxsim(Q.cpu(), D),
+        lambda: fm.flash_maxsim(Q, D, torch.ones(5, dtype=torch.int32, device=DEV)),
+        lambda: fm.flash_maxsim_batched(Q, D),
+        lambda: fm.flash_maxsim_topk(Q, D, 7),
+        lambda: fm.flash_maxsim_topk(Q, D, -1),
+        lambda: fm.flash_maxsim_topk(Q, D, 0),
+        lambda: fm.flash_maxsim_sparse(Q, D, torch.zeros(5, 2, dtype=torch.int32, device=DEV)),
+        lambda: fm.flash_maxsim(Q[:0], D),
+        lambda: fm.flash_maxsim(Q, D[:0]),
+        lambda: fm.flash_maxsim(Q, D[:, :0]),
+    ]
+    for call in calls:
+        assert same(*both(monkeypatch, call))
+
+
+def test_native_takes_the_ordinary_calls():
+    Q, D = sim((2, 20, 128), 11, torch.float16).to(DEV), sim((6, 36, 128), 12, torch.float16).to(DEV)
+    n = _lib.native()
+    assert n.score(Q[0], D, None) is not None and n.batched(Q, D, None, True) is not None
+    assert n.topk(Q[0], D, 3, None) is not None and n.forward(Q, D, None, 128) is not None
+    assert n.score(Q[0].cpu(), D, None) is None and n.score(Q[0].float(), D, None) is None
+    assert n.score(Q[0], [1], None) is None
+    with pytest.raises(TypeError):
+        n.score(Q[0], D)
+
+
+def test_native_launches_on_the_current_stream():
+    """A captured call replays on new inputs: it was recorded, so it ran on the
+    capturing stream; replays with eager work between them equal the eager result."""
+    Q, D = sim((20, 128), 13, torch.float16).to(DEV), sim((60, 36, 128), 14, torch.float16).to(DEV)
+    fm.flash_maxsim(Q, D)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fm.flash_maxsim(Q, D)
+    for i in range(4):
+        D.copy_(sim((60, 36, 128), 20 + i, torch.float16))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, fm.flash_maxsim(Q, D))
