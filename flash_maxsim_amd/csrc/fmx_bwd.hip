@@ -57,18 +57,18 @@ __device__ __forceinline__ void load8(const uint16_t* row, int k0, float (&x)[8]
 
 // Stores elements k0 .. k0+7 (those < d); 16-byte stores need d % 8 == 0 so
 // that every row of the contiguous output starts 16-byte aligned, 8-byte ones
-// d % 4 == 0 (backward of 18 queries of 32 tokens over 2000 docs of 1048 x 100: 512
+// d % 4 == 0 (D8: d % 8 == 0; backward of 18 queries of 32 tokens over 2000 docs of 1048 x 100: 512
 // -> 165 us with whole-row loads and these). dD is
 // written once and read only by the optimiser later: non-temporal stores
 // stream it out instead of leaving it dirty in the caches, where its
 // write-back would compete with the next forward's reads.
-template <bool BF>
+template <bool BF, bool D8>
 __device__ __forceinline__ void store8(uint16_t* row, int k0, int d, const float (&x)[8]) {
   u32x4_t v;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     v[i] = (uint32_t)Elem<BF>::from_f(x[2 * i]) | ((uint32_t)Elem<BF>::from_f(x[2 * i + 1]) << 16);
-  if ((d & 7) == 0) {
+  if constexpr (D8) {
     __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(row + k0));
   } else if ((d & 3) == 0) {
     __builtin_nontemporal_store(u32x2_t{v[0], v[1]}, reinterpret_cast<u32x2_t*>(row + k0));
@@ -334,7 +334,7 @@ __device__ __forceinline__ void dd_index_sort(const BwdArgs& a, int b, int chunk
 // with four: 1000 docs of 512 x 1024 under 256 tokens 357 -> 323 us, 4000 of
 // 300 x 128 under 200 144 -> 128; the smallest batches 35 -> 38).
 constexpr int kDdAhead = 4;
-template <bool BF, bool DENSE>
+template <bool BF, bool DENSE, bool D8>
 __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
   const int nkc = (a.d + 7) >> 3;
   const int lane = threadIdx.x & 63;
@@ -369,7 +369,7 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
     uint16_t* orow = static_cast<uint16_t*>(a.dD) + r * a.d;
     const uint32_t info0 = infos[p];
     if (a.dd_chunks == 1 && info0 == kNoRow) {
-      for (int kc = kc0; kc < nkc; kc += 64) store8<BF>(orow, kc * 8, a.d, zero);
+      for (int kc = kc0; kc < nkc; kc += 64) store8<BF, D8>(orow, kc * 8, a.d, zero);
     } else if (!DENSE || (a.dd_chunks == 1 &&
                           __builtin_amdgcn_ballot_w64(info0 != kNoRow && (info0 >> 16) > 2u) == 0)) {
       for (int kc = kc0; kc < nkc; kc += 64) {
@@ -392,7 +392,7 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
             for (int k = 0; k < 8; ++k) acc[k] = fmaf(g, x[k], acc[k]);
           }
         }
-        store8<BF>(orow, k0, a.d, acc);
+        store8<BF, D8>(orow, k0, a.d, acc);
       }
     } else if constexpr (DENSE) {
       // every lane of the row takes part in each step below, those past its
@@ -449,7 +449,7 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
             g = ng;
           }
         }
-        if (live) store8<BF>(orow, k0, a.d, acc);
+        if (live) store8<BF, D8>(orow, k0, a.d, acc);
       }
     }
     j += step;
@@ -488,13 +488,13 @@ __global__ void __launch_bounds__(256) bwd_front_kernel(BwdArgs a, unsigned n_ga
   }
 }
 
-template <bool BF, bool DENSE>
+template <bool BF, bool DENSE, bool D8>
 __global__ void __launch_bounds__(256) bwd_back_kernel(BwdArgs a, unsigned n_sum) {
   const unsigned x = blockIdx.x;
   if (x < n_sum) {
     dq_sum_block<BF>(a, x);
   } else {
-    dd_write_block<BF, DENSE>(a, x - n_sum);
+    dd_write_block<BF, DENSE, D8>(a, x - n_sum);
   }
 }
 
@@ -511,6 +511,11 @@ inline bool dd_dense(const BwdArgs& a) {
   return 5 * (int64_t)a.Nq * a.Lq > (a.lengths ? 2 : 5) * (int64_t)a.Ld;
 }
 
+// Unused LDS that keeps the writer, a stream of stores, to seven workgroups per
+// CU: more spread the stores over more of dD than the memory takes well, fewer
+// leave it waiting (step of 1000 docs of 512 x 1024, eight to five workgroups:
+// 410-420, 396, 402, 415 us).
+constexpr size_t kWriterLds = 23000;
 constexpr int64_t kBwdMaxBlocks = ((int64_t)1 << 24) - 1;  // workgroups of 256 threads per launch
 
 template <bool BF>
@@ -536,8 +541,11 @@ hipError_t launch_back(const BwdArgs& a, int64_t n_sum, int64_t n_write, hipStre
     const hipError_t e = launch_back<BF>(a, n_sum, 0, s);
     return e != hipSuccess ? e : launch_back<BF>(a, 0, n_write, s);
   }
-  auto kern = dd_dense(a) ? bwd_back_kernel<BF, true> : bwd_back_kernel<BF, false>;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(n_sum + n_write)), dim3(256), 0, s, a, (unsigned)n_sum);
+  const bool dense = dd_dense(a);
+  auto kern = (a.d & 7) == 0 ? (dense ? bwd_back_kernel<BF, true, true> : bwd_back_kernel<BF, false, true>)
+                             : (dense ? bwd_back_kernel<BF, true, false> : bwd_back_kernel<BF, false, false>);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(n_sum + n_write)), dim3(256),
+                     kWriterLds, s, a, (unsigned)n_sum);
   return hipGetLastError();
 }
 
