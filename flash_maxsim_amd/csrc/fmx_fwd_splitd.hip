@@ -26,11 +26,25 @@ namespace {
 
 constexpr int kSplitWaves = 8;
 
+// How resident workgroups walk shared docs (WALK): U units, each qp whole
+// queries or one pass of a long query, times `groups` doc groups; group g takes
+// docs g, g + groups, ...
+struct SplitWalk {
+  int qp, U, groups;
+  int xcd;  // units of a doc group share an XCD (groups is a multiple of 8)
+};
+
 // VEC: uint8 vector load path (FwdArgs::vec); true for fp16/bf16.
-// PERSIST (one query, one pass, no query gather): a fixed grid of resident
-// workgroups loads the query slice once and walks docs b, b + G, ...
-template <int KIND, int NQB, int KSW, bool KMASK, bool ARGMAX, bool VEC, bool PERSIST = false, bool C16 = VEC>
-__global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a) {
+// WALK (shared docs, no query gather): a grid of resident workgroups, each of
+// which loads the query slice of its unit once and walks its group's docs.
+// AHEAD: the next doc's first tiles are loaded ahead of this one's end, which
+// short docs gain from (2 x 128 tokens over 11901 docs of 72 x 1024 694 -> 673
+// us, of ragged lengths 462 -> 439; 32 x 32 over 200 ragged docs of 180 x 1024
+// 77 -> 68). Not with one unit whose query slice takes 128 VGPRs, which it
+// pushes into spills (128 tokens over 1000 ragged docs of 512 x 1024 131 -> 141).
+template <int KIND, int NQB, int KSW, bool KMASK, bool ARGMAX, bool VEC, bool WALK = false, bool C16 = VEC,
+          bool AHEAD = false>
+__global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a, SplitWalk wk) {
   constexpr int NW = kSplitWaves, QROWS = NQB * 16;
   // Tiles in flight per wave: 2 when the query slice takes 128 VGPRs, which
   // leaves room for the pipelined tile's results next to the buffers.
@@ -56,8 +70,18 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a) {
   const bool shared_q = a.shared_docs && a.Nq > 1;
   const int U = (shared_q ? a.Nq : 1) * npass;
   const int nslots = shared_q ? a.B : a.Nq * a.B;
-  int slot = blockIdx.x, u = 0;
-  if (U > 1) {
+  int slot = blockIdx.x, u = 0, grp0 = 0;
+  if constexpr (WALK) {
+    const int x = blockIdx.x;
+    if (wk.xcd) {
+      const int k = x & 7, r = x >> 3;
+      u = r % wk.U;
+      grp0 = 8 * (r / wk.U) + k;
+    } else {
+      u = x % wk.U;
+      grp0 = x / wk.U;
+    }
+  } else if (U > 1) {
     const int x = blockIdx.x, k = x & 7, r = x >> 3;
     const int grp = r / U;
     u = r - grp * U;
@@ -65,8 +89,12 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a) {
     if (slot >= nslots) return;  // uniform over the workgroup, before any barrier
   }
   const int pass = u % npass;
-  int qi, b;
-  if (shared_q) {
+  int qi, b, nqh = 1;  // nqh: queries of this unit
+  if constexpr (WALK) {
+    b = grp0;
+    qi = u / npass * wk.qp;
+    nqh = a.Nq - qi < wk.qp ? a.Nq - qi : wk.qp;
+  } else if (shared_q) {
     b = slot;
     qi = u / npass;
   } else {
@@ -85,11 +113,18 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a) {
 
   // ---- query slice of this pass ----
   const int q0 = pass * QROWS;
-  const rsrc_t rq = make_rsrc((const char*)a.Q + (int64_t)qi * a.sq_n * 2, (uint32_t)(a.Lq_rows * a.sq_l * 2));
+  const rsrc_t rq = make_rsrc((const char*)a.Q + (int64_t)qi * a.sq_n * 2,
+                              (uint32_t)(((nqh - 1) * a.sq_n + a.Lq_rows * a.sq_l) * 2));
   u32x4_t qf[NQB][KSW];
 #pragma unroll
   for (int nb = 0; nb < NQB; ++nb) {
-    const uint32_t rowoff = query_row_offset(a, b, q0 + nb * 16 + c);
+    uint32_t rowoff;
+    if constexpr (WALK) {  // row r of the pass: token r % Lq of the unit's query r / Lq
+      const int r = q0 + nb * 16 + c, qq = npass == 1 ? r / a.Lq : 0, tok = r - qq * a.Lq;
+      rowoff = qq < nqh && tok < a.Lq ? (uint32_t)((qq * a.sq_n + tok * a.sq_l) * 2) : kOOB;
+    } else {
+      rowoff = query_row_offset(a, b, q0 + nb * 16 + c);
+    }
 #pragma unroll
     for (int t = 0; t < KSW; ++t) {
       const int k0 = 32 * tbase + frag_k0<KIND>(t, g);
@@ -115,16 +150,15 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a) {
     }
   }
 
-  for (;;) {
-  const int item = qi * a.B + b;
-  const int64_t drow = a.shared_docs ? (int64_t)b : (int64_t)item;
-  int len = a.lengths ? a.lengths[drow] : a.Ld;
-  // uniform: the loads below take it into scalar buffer resources
-  len = __builtin_amdgcn_readfirstlane(len < 0 ? 0 : (len > a.Ld ? a.Ld : len));
-  const int ntiles = (len + 15) >> 4;
-
   // ---- doc stream ----
-  const DocRes dr = make_doc_res<KIND, VEC>(a, drow, len);
+  auto doc_len = [&](int64_t drow) {
+    const int l = a.lengths ? a.lengths[drow] : a.Ld;
+    // uniform: the loads take it into scalar buffer resources
+    return __builtin_amdgcn_readfirstlane(l < 0 ? 0 : (l > a.Ld ? a.Ld : l));
+  };
+  const int64_t drow0 = a.shared_docs ? (int64_t)b : (int64_t)(qi * a.B + b);
+  int len = doc_len(drow0);
+  DocRes dr = make_doc_res<KIND, VEC>(a, drow0, len);
   uint32_t koff[KSW];
 #pragma unroll
   for (int t = 0; t < KSW; ++t) {
@@ -132,6 +166,33 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a) {
     koff[t] = (KMASK && k0 >= a.d) ? kOOB : (uint32_t)(k0 * ESZ);  // past d: zeros
   }
 
+  Tile<KIND, KSW> buf[P];
+  // FIXED: a fixed load pattern. The first P tiles are loaded, and every group
+  // of P tiles that has a successor refills all P slots; tiles past the doc
+  // read zeros from outside its buffer range without touching memory. The
+  // compiler's wait before each tile then counts the tiles still in flight
+  // behind it, where a conditional load makes it wait for all of them (a full
+  // drain every other tile at P = 2). The largest masked instances keep
+  // conditional loads (the fixed pattern's extra registers spill there), and
+  // so do uint8 rows without 16-byte alignment (one wave per SIMD fewer).
+  constexpr bool FIXED = VEC && !(KMASK && (NQB * KSW >= 32 || KSW >= 16));
+  static_assert(!WALK || FIXED, "the walk loads a doc's first tiles unconditionally");
+  auto first_tiles = [&](auto sm_tag) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < P; ++s) load_tile<KIND, KSW, VEC, decltype(sm_tag)::value, C16>(buf[s], dr, s, c, g, koff);
+  };
+  auto open_doc = [&]() __attribute__((always_inline)) {
+    if (!U8 || owner) {
+      first_tiles(std::true_type{});
+    } else {
+      first_tiles(std::false_type{});
+    }
+  };
+  if constexpr (AHEAD) open_doc();
+
+  for (;;) {
+  if constexpr (FIXED && !AHEAD) open_doc();
+  const int ntiles = (len + 15) >> 4;
   float m = -INFINITY;
   int mi = 0;
   // Owner waves: folds tile rt (its eight partials in part[rt & 1]) into the
@@ -163,7 +224,6 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a) {
   // then reduces tile t-1 (written before the previous barrier) while they
   // run, then stores tile t's partials. part[t & 1] is rewritten at tile t+2,
   // after every owner passed tile t+1's barrier, i.e. finished reducing t.
-  Tile<KIND, KSW> buf[P];
   float psc[4] = {0.f, 0.f, 0.f, 0.f}, poff[4] = {0.f, 0.f, 0.f, 0.f};  // tile t-1 (uint8 docs)
   // Tile `tile` from ring slot T. Its slot's refill (tile + P) is issued
   // after the MFMAs have taken the operands (so they need no copy of their
@@ -218,23 +278,12 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a) {
   using RefillIf = std::integral_constant<int, REFILL_IF>;
   using RefillAny = std::integral_constant<int, REFILL_ANY>;
   // ntiles is uniform over the workgroup, so the barriers inside are safe.
-  // FIXED: a fixed load pattern. The first P tiles are loaded, and every group
-  // of P tiles that has a successor refills all P slots; tiles past the doc
-  // read zeros from outside its buffer range without touching memory. The
-  // compiler's wait before each tile then counts the tiles still in flight
-  // behind it, where a conditional load makes it wait for all of them (a full
-  // drain every other tile at P = 2). The largest masked instances keep
-  // conditional loads (the fixed pattern's extra registers spill there), and
-  // so do uint8 rows without 16-byte alignment (one wave per SIMD fewer).
-  constexpr bool FIXED = VEC && !(KMASK && (NQB * KSW >= 32 || KSW >= 16));
+  int nlen = 0;  // WALK: the next doc's length
   if constexpr (FIXED) {
     // uint8 docs: only the owner waves apply the affine epilogue, so only they
     // load the tiles' scales and mins; the others run a copy of the loop
     // without those loads (same tiles and barriers).
     auto run = [&](auto sm_tag) __attribute__((always_inline)) {
-      constexpr bool SM = decltype(sm_tag)::value;
-#pragma unroll
-      for (int s = 0; s < P; ++s) load_tile<KIND, KSW, VEC, SM, C16>(buf[s], dr, s, c, g, koff);
       int i0 = 0;
       for (; i0 + P < ntiles; i0 += P) {
 #pragma unroll
@@ -243,6 +292,14 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a) {
 #pragma unroll
       for (int s = 0; s < P; ++s)
         if (i0 + s < ntiles) process(RefillNone{}, sm_tag, buf[s], i0 + s);
+      if constexpr (AHEAD) {
+        // the next doc's first tiles, ahead of this one's last reduction
+        if (b + wk.groups < a.B) {
+          nlen = doc_len(b + wk.groups);
+          dr = make_doc_res<KIND, VEC>(a, b + wk.groups, nlen);
+          first_tiles(sm_tag);
+        }
+      }
     };
     if constexpr (U8) {
       if (owner) {
@@ -280,27 +337,36 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a) {
     }
   }
   __syncthreads();
-  if (wave == 0) {
+  // one wave per query of the unit
+  for (int qq = wave; qq < nqh; qq += NW) {
+    const int item = (qi + qq) * a.B + b;
+    const int r0 = qq * a.Lq;  // 0 unless the unit holds several queries
     float partsum = 0.f;
     for (int r = lane; r < QROWS; r += 64) {
       const int q = q0 + r;
       if (q < a.Lq) {
-        partsum += red_m[r];
-        if constexpr (ARGMAX) a.argmax[(int64_t)item * a.Lq + q] = red_i[r];
+        partsum += red_m[r0 + r];
+        if constexpr (ARGMAX) a.argmax[(int64_t)item * a.Lq + q] = red_i[r0 + r];
       }
     }
     const float total = wave_sum(partsum);
     if (lane == 0) {
       if (npass == 1) {
-        store_score(a, qi, b, total);
+        store_score(a, qi + qq, b, total);
       } else {
         a.partial[(int64_t)pass * a.Nq * a.B + item] = total;
       }
     }
   }
-  if (!PERSIST) break;
-  b += gridDim.x;
+  if (!WALK) break;
+  b += wk.groups;
   if (b >= a.B) break;
+  if constexpr (AHEAD) {
+    len = nlen;
+  } else {
+    len = doc_len(b);
+    dr = make_doc_res<KIND, VEC>(a, b, len);
+  }
   __syncthreads();  // red_m / red_i are rewritten for the next doc
   }
 }
@@ -315,43 +381,82 @@ __global__ void __launch_bounds__(256) splitd_sum_passes_kernel(FwdArgs a, int n
   store_score(a, qi, b, s);
 }
 
+// Whole queries that one unit of the walk holds: as many of Nq as fit the
+// largest query tile the walk runs (128 rows, or 64 at masked widths past 512),
+// when that is more than 32 rows; else 1. Each doc is then streamed for all of
+// them at once instead of once per query (2 x 128 tokens over 11901 docs of 72 x
+// 1024 1306 -> 694 us, 100 x 32 over 1000 of 150 x 384 1675 -> 876, 16 x 32 over
+// 1000 of 300 x 384 477 -> 255, 32 x 32 over 200 of 180 x 1024 293 -> 104).
+// Fewer where there are too few docs to fill the CUs with units otherwise.
+int splitd_unit_queries(const FwdArgs& a) {
+  const int ksw = splitd_fwd_ksw(a.d);
+  if (a.Nq <= 1 || ksw > 4) return 1;
+  const int cap = a.d != 32 * ksw * kSplitWaves && ksw == 4 ? 64 : 128;
+  int qp = cap / a.Lq;
+  if (qp > a.Nq) qp = a.Nq;
+  while (qp > 1 && (int64_t)((a.Nq + qp - 1) / qp) * a.B < 256) qp = qp / 2;
+  if (qp < 1 || qp * a.Lq <= 32) return 1;
+  // the unit's queries are read through one buffer range
+  if (a.sq_n < 0 || ((qp - 1) * a.sq_n + (a.Lq + 16) * a.sq_l) * 2 >= ((int64_t)1 << 31)) return 1;
+  return qp;
+}
+
 template <int KIND, int NQB, int KSW, bool KMASK, bool ARGMAX, bool VEC = true, bool C16 = VEC>
 hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
   constexpr int QROWS = NQB * 16;
   const int npass = (a.Lq + QROWS - 1) / QROWS;
   const int64_t items = (int64_t)a.Nq * a.B;
-  // One query in one pass: resident workgroups walk the docs with the query
-  // slice loaded once (config 5: 201 -> 189 us), for query tiles of 64 rows
-  // or more with aligned rows; smaller tiles gain nothing against more
-  // workgroups per CU, and the masked 128-row instances would spill.
+  // Shared docs (or one query): resident workgroups walk the docs with their
+  // query slice loaded once, for query tiles of 64 rows or more with aligned
+  // rows; smaller tiles gain nothing against more workgroups per CU, and the
+  // masked 128-row instances would spill.
   if constexpr (NQB >= 4 && VEC && !(KMASK && NQB * KSW >= 32)) {
-   if (npass == 1 && a.Nq == 1 && !a.qidx) {
-    // resident workgroups per CU x CUs (cached per device)
-    static int cache[64] = {0};
-    int dev = 0;
-    int n = 0;
-    if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) n = cache[dev];
-    if (n == 0) {
-      int cus = 0, per = 0;
-      if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-              &per, reinterpret_cast<const void*>(splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true>), 512,
-              0) != hipSuccess || per <= 0)
-        per = 1;
-      n = cus * per;
-      if (dev >= 0 && dev < 64) cache[dev] = n;
+    if ((a.Nq == 1 || a.shared_docs) && !a.qidx) {
+      // resident workgroups: per CU x CUs (cached per device)
+      static int cache[64] = {0};
+      int dev = 0;
+      int n = 0;
+      if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) n = cache[dev];
+      if (n == 0) {
+        int cus = 0, per = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per, reinterpret_cast<const void*>(splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, true>), 512,
+                0) != hipSuccess || per <= 0)
+          per = 1;
+        n = cus * per;
+        if (dev >= 0 && dev < 64) cache[dev] = n;
+      }
+      SplitWalk wk = {};
+      wk.qp = npass == 1 ? splitd_unit_queries(a) : 1;
+      wk.U = (a.Nq + wk.qp - 1) / wk.qp * npass;
+      // All units of a doc group on one XCD, unless that leaves over a tenth
+      // of the workgroups out: they read the doc through one L2.
+      const int per_xcd = n / 8;
+      if (wk.U > 1 && wk.U <= per_xcd && per_xcd % wk.U * 10 <= per_xcd && a.B >= 8) {
+        wk.xcd = 1;
+        wk.groups = 8 * (per_xcd / wk.U);
+        if (wk.groups > a.B) wk.groups = a.B / 8 * 8;
+      } else {
+        wk.groups = wk.U < n ? n / wk.U : 1;
+        if (wk.groups > a.B) wk.groups = a.B;
+      }
+      auto kern = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, true>;
+      if constexpr (NQB * KSW >= 32) {
+        if (wk.U == 1) kern = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, false>;
+      }
+      hipLaunchKernelGGL(kern, dim3((unsigned)wk.U * (unsigned)wk.groups), dim3(512), 0, s, a, wk);
+      if (npass > 1) {
+        hipLaunchKernelGGL(splitd_sum_passes_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, a, npass);
+      }
+      return hipGetLastError();
     }
-    const int64_t grid = a.B < n ? a.B : n;
-    hipLaunchKernelGGL((splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true>), dim3((unsigned)grid), dim3(512),
-                       0, s, a);
-    return hipGetLastError();
-   }
   }
   const int64_t U = (a.shared_docs && a.Nq > 1 ? a.Nq : 1) * (int64_t)npass;
   const int64_t nslots = a.shared_docs && a.Nq > 1 ? a.B : items;
   const int64_t grid = U > 1 ? ((nslots + 7) / 8) * 8 * U : items;
   hipLaunchKernelGGL((splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, false, C16>), dim3((unsigned)grid),
-                     dim3(512), 0, s, a);
+                     dim3(512), 0, s, a, SplitWalk{});
   if (npass > 1) {
     hipLaunchKernelGGL(splitd_sum_passes_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, a,
                        npass);
@@ -381,9 +486,12 @@ hipError_t dispatch_flags(const FwdArgs& a, bool am, hipStream_t s) {
   }
 }
 
+// Rows a workgroup holds at once: the query's, or those of the queries that
+// share a unit (shared docs, several queries).
 template <int KIND, int KSW>
 hipError_t dispatch_nqb(const FwdArgs& a, bool am, hipStream_t s) {
-  switch (splitd_fwd_nqb(a.Lq, a.d)) {
+  const int qp = KIND != KIND_U8 && a.shared_docs && !a.qidx ? splitd_unit_queries(a) : 1;
+  switch (splitd_fwd_nqb(qp * a.Lq, a.d)) {
     case 1: return dispatch_flags<KIND, 1, KSW>(a, am, s);
     case 2:
       if constexpr (KSW <= 8) return dispatch_flags<KIND, 2, KSW>(a, am, s);

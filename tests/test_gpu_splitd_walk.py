@@ -1,0 +1,66 @@
+"""The split-d kernel's walk (256 < d): units of several whole queries or of one
+pass of a long query over shared docs, against integer arithmetic, exact in every
+sum, so scores and the saved argmax must be equal."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from flash_maxsim_amd.flash_maxsim import _launch_fwd
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+@pytest.mark.parametrize(
+    "Nq, Lq, B, Ld, d",
+    [
+        (5, 32, 300, 20, 384),    # four queries a unit, the second unit with one
+        (2, 128, 300, 33, 1024),  # a query a unit, 128 rows
+        (7, 20, 130, 17, 512),    # six a unit, rows past the unit's queries
+        (3, 43, 260, 50, 300),    # three units: 32 workgroups an XCD do not divide
+        (17, 120, 40, 16, 384),   # seventeen units, no XCD mapping
+        (9, 8, 600, 31, 260),     # sixteen tokens' room left over
+        (6, 32, 140, 48, 768),    # masked width past 512: two queries a unit
+        (4, 32, 5, 40, 1024),     # too few docs for units
+        (3, 33, 100, 1, 640),     # one-token docs
+        (300, 128, 3, 16, 320),   # more units than workgroups that fit
+        (1, 200, 270, 70, 1024),  # passes of one query
+        (1, 64, 9, 90, 512),
+        (1, 128, 600, 31, 1024),  # one unit of 128 VGPRs
+        (1, 1000, 20, 35, 384),
+        (2, 200, 70, 30, 384),    # several passes of several queries
+        (2, 20, 70, 30, 2048),    # past the walk
+    ],
+)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_walk_exact_on_integer_grid(Nq, Lq, B, Ld, d, dtype):
+    gen = torch.Generator().manual_seed(2700 + d + Lq)
+    Q = torch.randint(-2, 3, (Nq, Lq, d), generator=gen)
+    D = torch.randint(-2, 3, (B, Ld, d), generator=gen)
+    lengths = torch.randint(0, Ld + 1, (B,), generator=gen, dtype=torch.int32)
+    lengths[:2] = torch.tensor([Ld, 0], dtype=torch.int32)
+    S = torch.mm(D.reshape(-1, d).double().to(DEV), Q.reshape(-1, d).double().t().contiguous().to(DEV))
+    S = S.view(B, Ld, Nq * Lq)
+    past = torch.arange(Ld)[None, :, None] >= lengths[:, None, None]
+    S.masked_fill_(past.to(DEV), float("-inf"))
+    best = S.max(dim=1).values  # [B, Nq * Lq]
+    first = (S == best[:, None]).to(torch.int32).argmax(dim=1)  # the first place that reaches it
+    want = best.view(B, Nq, Lq).sum(dim=2).t()
+    want_at = first.view(B, Nq, Lq).transpose(0, 1).reshape(Nq * B, Lq)
+
+    dp = (d + 7) // 8 * 8
+    wide = torch.full((Nq, Lq + 1, dp), float("nan"), dtype=dtype, device=DEV)  # queries apart, rows past Lq unread
+    wide[:, :Lq, :d] = Q.to(dtype).to(DEV)
+    Qd, Dd = wide[:, :Lq, :d], D.to(dtype).to(DEV)
+    if d % 8:
+        Dd = torch.nn.functional.pad(Dd, (0, dp - d))
+    for save in (False, True):
+        scores, at = _launch_fwd(Qd, Dd, lengths.to(DEV), Nq, B, Lq, Ld, d, True, save)
+        assert torch.equal(scores.double(), want)
+        if save:
+            live = (lengths > 0).repeat(Nq).to(DEV)
+            assert torch.equal(at[live].long(), want_at[live].long())
+            assert (at[~live] == 0).all()
