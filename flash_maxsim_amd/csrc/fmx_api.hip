@@ -625,11 +625,15 @@ size_t fmx_bwd_workspace_bytes(int64_t B, int64_t Lq, int64_t Ld, int64_t d) {
   return fmx_bwd_batched_workspace_bytes(1, B, Lq, Ld, d);
 }
 
-int fmx_bwd_batched(int dtype, const void* Q, int64_t q_stride_n, int64_t q_stride_l, const void* D,
-                    int64_t d_stride_b, int64_t d_stride_l, const int32_t* lengths, const int32_t* argmax,
-                    const float* grad_scores, int64_t g_stride_n, int64_t g_stride_b, void* dQ, void* dD,
-                    int64_t Nq, int64_t B, int64_t Lq, int64_t Ld, int64_t d, void* workspace,
-                    size_t workspace_bytes, void* stream) {
+}  // extern "C"
+
+namespace {
+
+// fmx_bwd_batched and fmx_bwd_batched_f32.
+int bwd_impl(int dtype, const void* Q, int64_t q_stride_n, int64_t q_stride_l, const void* D, int64_t d_stride_b,
+             int64_t d_stride_l, const int32_t* lengths, const int32_t* argmax, const float* grad_scores,
+             int64_t g_stride_n, int64_t g_stride_b, void* dQ, void* dD, int64_t Nq, int64_t B, int64_t Lq, int64_t Ld,
+             int64_t d, void* workspace, size_t workspace_bytes, void* stream, bool out_f32) {
   if (dtype != FMX_DTYPE_F16 && dtype != FMX_DTYPE_BF16) return fail(FMX_ERR_INVALID, "unknown dtype %d", dtype);
   int rc = check_common(Nq, B, Lq, Ld, d, q_stride_l, d_stride_b, d_stride_l, 2);
   if (rc) return rc;
@@ -667,6 +671,7 @@ int fmx_bwd_batched(int dtype, const void* Q, int64_t q_stride_n, int64_t q_stri
     a.ws = reinterpret_cast<float*>(w + dd_ws);
   }
   a.dd_slab = fmx::bwd_dd_slab((int)d);
+  a.out_f32 = out_f32 ? 1 : 0;
   a.sq_n = Nq > 1 ? q_stride_n : 0;
   a.sq_l = q_stride_l;
   a.sd_b = d_stride_b;
@@ -683,6 +688,55 @@ int fmx_bwd_batched(int dtype, const void* Q, int64_t q_stride_n, int64_t q_stri
   a.dd_chunks = (int)fmx::bwd_dd_chunks(Nq * Lq);
   const int kind = dtype == FMX_DTYPE_BF16 ? fmx::KIND_BF16 : fmx::KIND_F16;
   return hip_status(fmx::launch_bwd(kind, a, static_cast<hipStream_t>(stream)), "fmx_bwd launch");
+}
+
+}  // namespace
+
+extern "C" {
+
+int fmx_bwd_batched(int dtype, const void* Q, int64_t q_stride_n, int64_t q_stride_l, const void* D,
+                    int64_t d_stride_b, int64_t d_stride_l, const int32_t* lengths, const int32_t* argmax,
+                    const float* grad_scores, int64_t g_stride_n, int64_t g_stride_b, void* dQ, void* dD,
+                    int64_t Nq, int64_t B, int64_t Lq, int64_t Ld, int64_t d, void* workspace,
+                    size_t workspace_bytes, void* stream) {
+  return bwd_impl(dtype, Q, q_stride_n, q_stride_l, D, d_stride_b, d_stride_l, lengths, argmax, grad_scores, g_stride_n,
+                  g_stride_b, dQ, dD, Nq, B, Lq, Ld, d, workspace, workspace_bytes, stream, false);
+}
+
+int fmx_bwd_batched_f32(const void* Q, int64_t q_stride_n, int64_t q_stride_l, const void* D, int64_t d_stride_b,
+                        int64_t d_stride_l, const int32_t* lengths, const int32_t* argmax, const float* grad_scores,
+                        int64_t g_stride_n, int64_t g_stride_b, float* dQ, float* dD, int64_t Nq, int64_t B, int64_t Lq,
+                        int64_t Ld, int64_t d, void* workspace, size_t workspace_bytes, void* stream) {
+  return bwd_impl(FMX_DTYPE_F16, Q, q_stride_n, q_stride_l, D, d_stride_b, d_stride_l, lengths, argmax, grad_scores,
+                  g_stride_n, g_stride_b, dQ, dD, Nq, B, Lq, Ld, d, workspace, workspace_bytes, stream, true);
+}
+
+int fmx_convert_rows(int src_dtype, const void* src, int64_t s_stride_b, int64_t s_stride_l, int64_t B, int64_t Ld,
+                     int64_t d, int dst_dtype, void* dst, int64_t dp, void* stream) {
+  if (B < 0 || Ld < 0 || d < 1 || dp < d || (dp & 7) || s_stride_b < 0 || s_stride_l < 0)
+    return fail(FMX_ERR_INVALID, "invalid sizes B=%lld Ld=%lld d=%lld dp=%lld", (long long)B, (long long)Ld, (long long)d,
+                (long long)dp);
+  const bool same = src_dtype == dst_dtype && (src_dtype == FMX_DTYPE_F16 || src_dtype == FMX_DTYPE_BF16);
+  const bool cast = dst_dtype == FMX_DTYPE_F16 && (src_dtype == FMX_DTYPE_F32 || src_dtype == FMX_DTYPE_BF16);
+  if (!same && !cast) return fail(FMX_ERR_INVALID, "no conversion from dtype %d to %d", src_dtype, dst_dtype);
+  if (B == 0 || Ld == 0) return ok();
+  if (!src || !dst) return fail(FMX_ERR_INVALID, "src and dst must be non-null");
+  if (!aligned16(dst)) return fail(FMX_ERR_INVALID, "dst must be 16-byte aligned");
+  if (reinterpret_cast<uintptr_t>(src) & (src_dtype == FMX_DTYPE_F32 ? 3u : 1u))
+    return fail(FMX_ERR_INVALID, "src must be aligned to its element");
+  if (dp > INT32_MAX || Ld > INT32_MAX / (dp / 8)) return fail(FMX_ERR_UNSUPPORTED, "doc of %lld x %lld elements", (long long)Ld, (long long)dp);
+  fmx::ConvertArgs a = {};
+  a.src = src;
+  a.s_stride_b = s_stride_b;
+  a.s_stride_l = s_stride_l;
+  a.B = B;
+  a.Ld = Ld;
+  a.d = d;
+  a.dp = dp;
+  a.f32 = src_dtype == FMX_DTYPE_F32;
+  a.bf16 = src_dtype == FMX_DTYPE_BF16 && dst_dtype == FMX_DTYPE_F16;
+  a.dst = dst;
+  return hip_status(fmx::launch_convert(a, static_cast<hipStream_t>(stream)), "fmx_convert_rows launch");
 }
 
 int fmx_bwd(int dtype, const void* Q, int64_t q_stride_l, const void* D, int64_t d_stride_b,

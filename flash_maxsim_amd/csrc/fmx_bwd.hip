@@ -42,12 +42,25 @@ struct Elem<true> {
   }
 };
 
-// Loads elements k0 .. k0+7 of a 2-byte row as fp32, k0 < d: one 16-byte load
-// (rows start 16-byte aligned, a multiple of 8 elements apart). Elements at or
-// past d may be anything; they reach only sums that are not stored.
-template <bool BF>
-__device__ __forceinline__ void load8(const uint16_t* row, int k0, float (&x)[8]) {
-  const u32x4_t v = *reinterpret_cast<const u32x4_t*>(row + k0);
+// Gradient rows as they are stored: 2-byte elements with d % 8 == 0 (OUT_H8),
+// 2-byte elements of any d, or fp32. A lane has eight elements of a row: eight
+// in a row, or for fp32 two quads L quads apart, so that each store
+// instruction covers whole lines.
+enum Out : int { OUT_H8, OUT_H, OUT_F32 };
+
+// Loads elements p0 .. p0+3 and p1 .. p1+3 of a 2-byte row as fp32, p0 < d: one
+// 16-byte load where they are adjacent (rows start 16-byte aligned, a multiple
+// of 8 elements apart). Elements at or past d may be anything; they reach only
+// sums that are not stored.
+template <bool BF, int OUT>
+__device__ __forceinline__ void load8(const uint16_t* row, int p0, int p1, float (&x)[8]) {
+  u32x4_t v;
+  if constexpr (OUT == OUT_F32) {
+    const u32x2_t a = *reinterpret_cast<const u32x2_t*>(row + p0), b = *reinterpret_cast<const u32x2_t*>(row + p1);
+    v = u32x4_t{a[0], a[1], b[0], b[1]};
+  } else {
+    v = *reinterpret_cast<const u32x4_t*>(row + p0);
+  }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     x[2 * e] = Elem<BF>::to_f(v[e] & 0xffffu);
@@ -55,28 +68,47 @@ __device__ __forceinline__ void load8(const uint16_t* row, int k0, float (&x)[8]
   }
 }
 
-// Stores elements k0 .. k0+7 (those < d); 16-byte stores need d % 8 == 0 so
-// that every row of the contiguous output starts 16-byte aligned, 8-byte ones
-// d % 4 == 0 (D8: d % 8 == 0; backward of 18 queries of 32 tokens over 2000 docs of 1048 x 100: 512
-// -> 165 us with whole-row loads and these). dD is
-// written once and read only by the optimiser later: non-temporal stores
-// stream it out instead of leaving it dirty in the caches, where its
-// write-back would compete with the next forward's reads.
-template <bool BF, bool D8>
-__device__ __forceinline__ void store8(uint16_t* row, int k0, int d, const float (&x)[8]) {
+// Stores those elements (the ones below d) of a gradient row; 16-byte stores of
+// 2-byte elements need d % 8 == 0 so that every row of the contiguous output
+// starts 16-byte aligned, 8-byte ones (and 16-byte ones of fp32) d % 4 == 0
+// (backward of 18 queries of 32 tokens over 2000 docs of 1048 x 100: 512 -> 165
+// us with whole-row loads and these). dD is written once and read only by the
+// optimiser later: non-temporal stores stream it out instead of leaving it
+// dirty in the caches, where its write-back would compete with the next
+// forward's reads.
+template <bool BF, int OUT>
+__device__ __forceinline__ void store8(void* out_row, int p0, int p1, int d, const float (&x)[8]) {
+  if constexpr (OUT == OUT_F32) {
+    float* row = static_cast<float*>(out_row);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int p = h ? p1 : p0;
+      if ((d & 3) == 0) {
+        if (p < d)
+          __builtin_nontemporal_store(f32x4_t{x[4 * h], x[4 * h + 1], x[4 * h + 2], x[4 * h + 3]},
+                                      reinterpret_cast<f32x4_t*>(row + p));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (p + e < d) row[p + e] = x[4 * h + e];
+      }
+    }
+    return;
+  }
+  uint16_t* row = static_cast<uint16_t*>(out_row);
   u32x4_t v;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     v[i] = (uint32_t)Elem<BF>::from_f(x[2 * i]) | ((uint32_t)Elem<BF>::from_f(x[2 * i + 1]) << 16);
-  if constexpr (D8) {
-    __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(row + k0));
+  if constexpr (OUT == OUT_H8) {
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(row + p0));
   } else if ((d & 3) == 0) {
-    __builtin_nontemporal_store(u32x2_t{v[0], v[1]}, reinterpret_cast<u32x2_t*>(row + k0));
-    if (k0 + 4 < d) __builtin_nontemporal_store(u32x2_t{v[2], v[3]}, reinterpret_cast<u32x2_t*>(row + k0 + 4));
+    __builtin_nontemporal_store(u32x2_t{v[0], v[1]}, reinterpret_cast<u32x2_t*>(row + p0));
+    if (p1 < d) __builtin_nontemporal_store(u32x2_t{v[2], v[3]}, reinterpret_cast<u32x2_t*>(row + p1));
   } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-      if (k0 + e < d) row[k0 + e] = Elem<BF>::from_f(x[e]);
+      if (p0 + e < d) row[p0 + e] = Elem<BF>::from_f(x[e]);
   }
 }
 
@@ -135,7 +167,7 @@ __device__ __forceinline__ void dq_partial_block(const BwdArgs& a, int64_t bx, i
 #pragma unroll
     for (int u = 0; u < DB; ++u) {
       const uint16_t* row = D + (int64_t)bi[u] * a.sd_b + (int64_t)j[u] * a.sd_l;
-      load8<BF>(row, k0, x[u]);
+      load8<BF, OUT_H8>(row, k0, k0 + 4, x[u]);
     }
 #pragma unroll
     for (int u = 0; u < DB; ++u)
@@ -150,7 +182,7 @@ __device__ __forceinline__ void dq_partial_block(const BwdArgs& a, int64_t bx, i
 }
 
 // Stage 2 of dQ: dQ[r][k] = sum over chunks (in order) of ws[chunk][r][k].
-template <bool BF>
+template <bool BF, int OUT>
 __device__ __forceinline__ void dq_sum_block(const BwdArgs& a, int64_t block) {
   const int64_t n = (int64_t)a.Nq * a.Lq * a.d;
   const int64_t i = block * 256 + threadIdx.x;
@@ -158,7 +190,11 @@ __device__ __forceinline__ void dq_sum_block(const BwdArgs& a, int64_t block) {
   float s = 0.f;
 #pragma unroll 8
   for (int c = 0; c < a.nchunk; ++c) s += a.ws[(int64_t)c * n + i];  // chunk order: deterministic
-  static_cast<uint16_t*>(a.dQ)[i] = Elem<BF>::from_f(s);
+  if constexpr (OUT == OUT_F32) {
+    static_cast<float*>(a.dQ)[i] = s;
+  } else {
+    static_cast<uint16_t*>(a.dQ)[i] = Elem<BF>::from_f(s);
+  }
 }
 
 constexpr int kEntryBits = 13;  // entries of one chunk < 2^13 (kDdChunk)
@@ -334,7 +370,7 @@ __device__ __forceinline__ void dd_index_sort(const BwdArgs& a, int b, int chunk
 // with four: 1000 docs of 512 x 1024 under 256 tokens 357 -> 323 us, 4000 of
 // 300 x 128 under 200 144 -> 128; the smallest batches 35 -> 38).
 constexpr int kDdAhead = 4;
-template <bool BF, bool DENSE, bool D8>
+template <bool BF, bool DENSE, int OUT>
 __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
   const int nkc = (a.d + 7) >> 3;
   const int lane = threadIdx.x & 63;
@@ -349,6 +385,8 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
   const int64_t r0 = slab * a.dd_slab;
   const int64_t r1 = r0 + a.dd_slab < total ? r0 + a.dd_slab : total;
   const int step = 4 * rpw;
+  // the lane's elements p0 .. p0+3 and p1 .. p1+3 of the row's part from 8 * kb on
+  auto at = [&](int kb, int h) { return OUT == OUT_F32 ? 8 * kb + 4 * (h * L + kc0) : 8 * (kb + kc0) + 4 * h; };
   int64_t r = r0 + wave * rpw + sub;
   int b = (int)(r / a.Ld);
   int j = (int)(r - (int64_t)b * a.Ld);
@@ -366,14 +404,14 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
 #pragma unroll
   for (int p = 0; p < kDdMaxPasses; ++p, r += step) {
     if (r >= r1) break;
-    uint16_t* orow = static_cast<uint16_t*>(a.dD) + r * a.d;
+    void* orow = static_cast<char*>(a.dD) + r * a.d * (OUT == OUT_F32 ? 4 : 2);
     const uint32_t info0 = infos[p];
     if (a.dd_chunks == 1 && info0 == kNoRow) {
-      for (int kc = kc0; kc < nkc; kc += 64) store8<BF, D8>(orow, kc * 8, a.d, zero);
+      for (int kb = 0; at(kb, 0) < a.d; kb += 64) store8<BF, OUT>(orow, at(kb, 0), at(kb, 1), a.d, zero);
     } else if (!DENSE || (a.dd_chunks == 1 &&
                           __builtin_amdgcn_ballot_w64(info0 != kNoRow && (info0 >> 16) > 2u) == 0)) {
-      for (int kc = kc0; kc < nkc; kc += 64) {
-        const int k0 = kc * 8;
+      for (int kb = 0; at(kb, 0) < a.d; kb += 64) {
+        const int p0 = at(kb, 0), p1 = at(kb, 1);
         float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         // the row's entries chunk by chunk: entry order overall
         for (int ch = 0; ch < a.dd_chunks; ++ch) {
@@ -387,19 +425,20 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
             const int qi = e / a.Lq, q = e - qi * a.Lq;
             const float g = a.grad[(int64_t)qi * a.g_n + (int64_t)b * a.g_b];
             float x[8];
-            load8<BF>(Q + (int64_t)qi * a.sq_n + (int64_t)q * a.sq_l, k0, x);
+            load8<BF, OUT>(Q + (int64_t)qi * a.sq_n + (int64_t)q * a.sq_l, p0, p1 < a.d ? p1 : p0, x);
 #pragma unroll
             for (int k = 0; k < 8; ++k) acc[k] = fmaf(g, x[k], acc[k]);
           }
         }
-        store8<BF, D8>(orow, k0, a.d, acc);
+        store8<BF, OUT>(orow, p0, p1, a.d, acc);
       }
     } else if constexpr (DENSE) {
       // every lane of the row takes part in each step below, those past its
       // last k chunk too (they fetch entries; their loads repeat chunk 0)
       for (int kb = 0; kb < nkc; kb += 64) {
-        const bool live = kb + kc0 < nkc;
-        const int k0 = live ? (kb + kc0) * 8 : 0;
+        const int p0 = at(kb, 0), p1 = at(kb, 1);
+        const bool live = p0 < a.d;
+        const int l0 = live ? p0 : 0, l1 = p1 < a.d ? p1 : l0;  // places to load from
         float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         // the row's entries chunk by chunk: entry order overall
         for (int ch = 0; ch < a.dd_chunks; ++ch) {
@@ -428,7 +467,7 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
               const int src = (lane & ~(L - 1)) + u0 + u;
               const uint16_t* row = Q + (int64_t)lane_fetch(off, src) * 8;
               gu[u] = __builtin_bit_cast(float, lane_fetch(__builtin_bit_cast(uint32_t, g), src));
-              load8<BF>(row, k0, x[u]);
+              load8<BF, OUT>(row, l0, l1, x[u]);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u)
@@ -449,7 +488,7 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
             g = ng;
           }
         }
-        if (live) store8<BF, D8>(orow, k0, a.d, acc);
+        if (live) store8<BF, OUT>(orow, p0, p1, a.d, acc);
       }
     }
     j += step;
@@ -488,13 +527,13 @@ __global__ void __launch_bounds__(256) bwd_front_kernel(BwdArgs a, unsigned n_ga
   }
 }
 
-template <bool BF, bool DENSE, bool D8>
+template <bool BF, bool DENSE, int OUT>
 __global__ void __launch_bounds__(256) bwd_back_kernel(BwdArgs a, unsigned n_sum) {
   const unsigned x = blockIdx.x;
   if (x < n_sum) {
-    dq_sum_block<BF>(a, x);
+    dq_sum_block<BF, OUT>(a, x);
   } else {
-    dd_write_block<BF, DENSE, D8>(a, x - n_sum);
+    dd_write_block<BF, DENSE, OUT>(a, x - n_sum);
   }
 }
 
@@ -542,8 +581,11 @@ hipError_t launch_back(const BwdArgs& a, int64_t n_sum, int64_t n_write, hipStre
     return e != hipSuccess ? e : launch_back<BF>(a, 0, n_write, s);
   }
   const bool dense = dd_dense(a);
-  auto kern = (a.d & 7) == 0 ? (dense ? bwd_back_kernel<BF, true, true> : bwd_back_kernel<BF, false, true>)
-                             : (dense ? bwd_back_kernel<BF, true, false> : bwd_back_kernel<BF, false, false>);
+  auto kern = (a.d & 7) == 0 ? (dense ? bwd_back_kernel<BF, true, OUT_H8> : bwd_back_kernel<BF, false, OUT_H8>)
+                             : (dense ? bwd_back_kernel<BF, true, OUT_H> : bwd_back_kernel<BF, false, OUT_H>);
+  if constexpr (!BF) {
+    if (a.out_f32) kern = dense ? bwd_back_kernel<BF, true, OUT_F32> : bwd_back_kernel<BF, false, OUT_F32>;
+  }
   hipLaunchKernelGGL(kern, dim3((unsigned)(n_sum + n_write)), dim3(256),
                      kWriterLds, s, a, (unsigned)n_sum);
   return hipGetLastError();

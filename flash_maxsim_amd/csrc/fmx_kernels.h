@@ -57,6 +57,7 @@ struct BwdArgs {
   uint32_t* dd_rows;          // dD index [dd_chunks, B, Ld]: first sorted entry | count << 16, or ~0
   uint16_t* dd_ent;           // dD index [B, Nq*Lq]: each chunk's entries sorted by row (chunk-local)
   int dd_slab;                // rows per dD writer workgroup
+  int out_f32;                // dQ and dD are fp32 (fp16 operands only), else in the operands' type
 };
 
 // Shape class handled by the streaming kernel (query tile in VGPRs, docs read
@@ -128,6 +129,19 @@ hipError_t launch_quantize(int src_kind, const QuantArgs& a, hipStream_t s);  //
 // Its inverse over contiguous [rows, d] codes with one fp16 scale and min per row.
 hipError_t launch_dequantize(const uint8_t* codes, const uint16_t* scales, const uint16_t* mins, float* out,
                              int64_t rows, int64_t d, hipStream_t s);
+
+// Operand rows made ready for the kernels: [B, Ld] rows of d elements cast to fp16
+// (or moved as they are, 2-byte types) into contiguous rows of dp >= d elements,
+// zeros past d.
+struct ConvertArgs {
+  const void* src;            // strides s_stride_b, s_stride_l in elements
+  int64_t s_stride_b, s_stride_l;
+  int64_t B, Ld, d, dp;
+  int f32;                    // fp32 source, else 2-byte elements
+  int bf16;                   // 2-byte source: bf16 to be cast to fp16
+  void* dst;
+};
+hipError_t launch_convert(const ConvertArgs& a, hipStream_t s);
 
 // Packed docs: where each doc starts, and the copy of its rows.
 hipError_t launch_layout(const int32_t* lengths, int64_t B, int32_t Ld, int32_t* out, int64_t* tok_group,

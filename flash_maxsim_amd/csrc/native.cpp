@@ -1,10 +1,11 @@
 // The host path of the ordinary calls, in native code: flash_maxsim_amd._native.
 //
-// A call whose operands the kernels read as they are (GPU tensors of one
-// kernel dtype on the current device, strides and alignment as include/fmx.h
-// asks, int32 lengths) is checked, given its outputs and workspace and launched
-// here. Every other call (casts, copies, other devices, empty sizes, wrong
-// shapes) gets None and takes the Python path, which has the asserts and the
+// A call on floating-point GPU tensors of the current device with int32 lengths
+// is checked, given its outputs and workspace and launched here; operands that
+// the kernels do not read as they are (float32, mixed types, rows off the
+// alignment that include/fmx.h asks for) go through fmx_convert_rows first, one
+// pass each. Every other call (other types and devices, inner strides, empty
+// sizes, wrong shapes) gets None and takes the Python path, which has the asserts and the
 // error messages. In Python and ctypes an ordinary call's checks, allocations
 // and the conversion of twenty arguments took longer than the kernels of a
 // rerank: 100 docs of up to 300 x 128 under 32 tokens
@@ -50,11 +51,27 @@ bool rows_ready(const Tensor& t) {
   return (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) == 0;
 }
 
-// The kernels' code of Q and D's common dtype, or -1.
+// The library's code of a floating-point type, or -1.
+int code_of(const Tensor& t) {
+  switch (t.scalar_type()) {
+    case at::kHalf: return FMX_DTYPE_F16;
+    case at::kBFloat16: return FMX_DTYPE_BF16;
+    case at::kFloat: return FMX_DTYPE_F32;
+    default: return -1;
+  }
+}
+
+// The type the kernels run Q and D in: bf16 when both are, else fp16; -1 for types cast elsewhere.
 int kernel_dtype(const Tensor& Q, const Tensor& D) {
-  if (Q.scalar_type() != D.scalar_type()) return -1;
-  if (Q.scalar_type() == at::kHalf) return FMX_DTYPE_F16;
-  return Q.scalar_type() == at::kBFloat16 ? FMX_DTYPE_BF16 : -1;
+  const int q = code_of(Q), x = code_of(D);
+  if (q < 0 || x < 0) return -1;
+  return q == FMX_DTYPE_BF16 && x == FMX_DTYPE_BF16 ? FMX_DTYPE_BF16 : FMX_DTYPE_F16;
+}
+
+// Whether `ready` can make t an operand.
+bool convertible(const Tensor& t) {
+  const int64_t n = t.dim(), d = t.size(n - 1);
+  return (n == 2 || n == 3) && t.stride(n - 1) == 1 && d >= 1 && t.numel() > 0 && t.size(n - 2) <= INT32_MAX / (d / 8 + 1);
 }
 
 bool is_row_of(const Tensor* t, at::ScalarType type, int64_t n) {
@@ -76,6 +93,31 @@ bool take_lengths(PyObject* o, int64_t n, const Tensor& like, const int32_t** ou
 bool here(const Tensor& t) {
   return t.device().index() == c10::hip::current_device() && !c10::impl::TorchDispatchModeTLS::any_modes_set();
 }
+
+void* stream_of(const Tensor& t);
+
+// t as the kernels read it in type `dtype`: itself, or a converted copy with its
+// rows padded to a multiple of 8 elements. Undefined, with *rc set: the conversion failed.
+Tensor ready(const Tensor& t, int dtype, int* rc) {
+  if (code_of(t) == dtype && rows_ready(t)) return t;
+  const int64_t n = t.dim(), d = t.size(n - 1), dp = (d + 7) / 8 * 8, rows = t.size(n - 2);
+  auto sizes = t.sizes().vec();
+  sizes[n - 1] = dp;
+  Tensor out = at::empty(sizes, t.options().dtype(dtype == FMX_DTYPE_BF16 ? at::kBFloat16 : at::kHalf));
+  *rc = fmx_convert_rows(code_of(t), t.const_data_ptr(), n == 3 ? t.stride(0) : 0, t.stride(n - 2),
+                         n == 3 ? t.size(0) : 1, rows, d, dtype, out.data_ptr(), dp, stream_of(t));
+  return *rc ? Tensor() : out;
+}
+
+// Q and D as operands, in place of their originals.
+#define FMX_READY(Q, D)                                \
+  int prc = 0;                                         \
+  const Tensor Qk = ready(*Q, dtype, &prc);            \
+  if (prc) return failed(prc);                         \
+  const Tensor Dk = ready(*D, dtype, &prc);            \
+  if (prc) return failed(prc)
+
+PyObject* failed(int rc);
 
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
@@ -114,14 +156,15 @@ PyObject* score(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t Lq = Q->size(0), d = Q->size(1), B = D->size(0), Ld = D->size(1);
   const int dtype = kernel_dtype(*Q, *D);
   const int32_t* lengths;
-  FMX_ORDINARY(dtype >= 0 && B > 0 && Lq > 0 && rows_ready(*Q) && rows_ready(*D) && Q->device() == D->device() &&
+  FMX_ORDINARY(dtype >= 0 && B > 0 && Lq > 0 && convertible(*Q) && convertible(*D) && Q->device() == D->device() &&
                take_lengths(args[2], B, *D, &lengths) && here(*Q));
   Tensor out = at::empty({B}, D->options().dtype(at::kFloat));
   const size_t n = fmx_fwd_workspace_bytes(1, B, Lq, Ld, d);
   const Tensor ws = scratch(n, *D);
+  FMX_READY(Q, D);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
-    return fmx_fwd(dtype, Q->const_data_ptr(), 0, Q->stride(0), D->const_data_ptr(), D->stride(0), D->stride(1),
+    return fmx_fwd(dtype, Qk.const_data_ptr(), 0, Qk.stride(0), Dk.const_data_ptr(), Dk.stride(0), Dk.stride(1),
                    lengths, out.data_ptr<float>(), B, 1, nullptr, 1, B, Lq, Ld, d, 1, ptr(ws), n, s);
   });
   return rc ? failed(rc) : THPVariable_Wrap(std::move(out));
@@ -141,15 +184,16 @@ PyObject* batched(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int dtype = kernel_dtype(*Q, *D);
   const int32_t* lengths;
   FMX_ORDINARY(D->size(k + 2) == d && (shared || (D->size(0) == Nq && D->stride(0) == B * D->stride(1))));
-  FMX_ORDINARY(dtype >= 0 && Nq > 0 && B > 0 && Lq > 0 && rows_ready(*Q) && rows_ready(*D) &&
+  FMX_ORDINARY(dtype >= 0 && Nq > 0 && B > 0 && Lq > 0 && convertible(*Q) && (shared ? convertible(*D) : code_of(*D) == dtype && rows_ready(*D)) &&
                Q->device() == D->device() && take_lengths(args[2], shared ? B : Nq * B, *D, &lengths) && here(*Q));
   Tensor out = at::empty({Nq, B}, D->options().dtype(at::kFloat));
   const size_t n = fmx_fwd_workspace_bytes(Nq, B, Lq, Ld, d);
   const Tensor ws = scratch(n, *D);
+  FMX_READY(Q, D);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
-    return fmx_fwd(dtype, Q->const_data_ptr(), Q->stride(0), Q->stride(1), D->const_data_ptr(), D->stride(k),
-                   D->stride(k + 1), lengths, out.data_ptr<float>(), B, 1, nullptr, Nq, B, Lq, Ld, d, shared, ptr(ws),
+    return fmx_fwd(dtype, Qk.const_data_ptr(), Qk.stride(0), Qk.stride(1), Dk.const_data_ptr(), Dk.stride(k),
+                   Dk.stride(k + 1), lengths, out.data_ptr<float>(), B, 1, nullptr, Nq, B, Lq, Ld, d, shared, ptr(ws),
                    n, s);
   });
   return rc ? failed(rc) : THPVariable_Wrap(std::move(out));
@@ -166,14 +210,15 @@ PyObject* sparse(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int dtype = kernel_dtype(*Q, *D);
   const int32_t* lengths;
   FMX_ORDINARY(dtype >= 0 && B > 0 && Lq > 0 && K > 0 && idx->size(0) == B && is_row_of(idx, at::kInt, B * K));
-  FMX_ORDINARY(rows_ready(*Q) && rows_ready(*D) && Q->device() == D->device() && idx->device() == D->device() &&
+  FMX_ORDINARY(convertible(*Q) && convertible(*D) && Q->device() == D->device() && idx->device() == D->device() &&
                take_lengths(args[3], B, *D, &lengths) && here(*Q));
   Tensor out = at::empty({B}, D->options().dtype(at::kFloat));
   const size_t n = fmx_fwd_sparse_workspace_bytes(B, K, Ld, d);
   const Tensor ws = scratch(n, *D);
+  FMX_READY(Q, D);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
-    return fmx_fwd_sparse(dtype, Q->const_data_ptr(), Q->stride(0), Lq, D->const_data_ptr(), D->stride(0), D->stride(1),
+    return fmx_fwd_sparse(dtype, Qk.const_data_ptr(), Qk.stride(0), Lq, Dk.const_data_ptr(), Dk.stride(0), Dk.stride(1),
                           idx->const_data_ptr<int32_t>(), K, 1, K, lengths, out.data_ptr<float>(), B, Ld, d, ptr(ws), n,
                           s);
   });
@@ -196,16 +241,17 @@ PyObject* topk(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t Lq = Q->size(0), d = Q->size(1), B = D->size(0), Ld = D->size(1);
   const int dtype = kernel_dtype(*Q, *D);
   const int32_t* lengths;
-  FMX_ORDINARY(dtype >= 0 && Lq > 0 && k > 0 && k <= B && rows_ready(*Q) && rows_ready(*D) &&
+  FMX_ORDINARY(dtype >= 0 && Lq > 0 && k > 0 && k <= B && convertible(*Q) && convertible(*D) &&
                Q->device() == D->device() && take_lengths(args[3], B, *D, &lengths) && here(*Q));
   const auto f32 = D->options().dtype(at::kFloat);
   const Tensor scores = at::empty({B}, f32);
   Tensor values = at::empty({k}, f32), indices = at::empty({k}, D->options().dtype(at::kLong));
   const size_t n = fmx_fwd_topk_workspace_bytes(B, Lq, Ld, d, k);
   const Tensor ws = scratch(n, *D);
+  FMX_READY(Q, D);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
-    return fmx_fwd_topk(dtype, Q->const_data_ptr(), Q->stride(0), D->const_data_ptr(), D->stride(0), D->stride(1),
+    return fmx_fwd_topk(dtype, Qk.const_data_ptr(), Qk.stride(0), Dk.const_data_ptr(), Dk.stride(0), Dk.stride(1),
                         lengths, B, Lq, Ld, d, k, scores.data_ptr<float>(), values.data_ptr<float>(),
                         indices.data_ptr<int64_t>(), ptr(ws), n, s);
   });
@@ -267,16 +313,17 @@ PyObject* packed(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   int64_t B;
   const int64_t* group;
   const int32_t *lengths, *ids;
-  FMX_ORDINARY(dtype >= 0 && Q->device() == D->device() && rows_ready(*Q) && rows_ready(*D) &&
+  FMX_ORDINARY(dtype >= 0 && Q->device() == D->device() && convertible(*Q) && convertible(*D) &&
                take_slots(args[2], args[3], args[5], *D, &B, &group, &lengths, &ids) && B > 0 && Lq > 0 && T > 0 &&
                here(*Q));
   const int64_t Ld = max_len > 1 ? max_len : 1;
   Tensor out = at::empty({B}, D->options().dtype(at::kFloat));
   const size_t n = fmx_fwd_packed_workspace_bytes(B, Lq, Ld, d);
   const Tensor ws = scratch(n, *D);
+  FMX_READY(Q, D);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
-    return fmx_fwd_packed(dtype, Q->const_data_ptr(), Q->stride(0), Lq, D->const_data_ptr(), D->stride(0), T, group,
+    return fmx_fwd_packed(dtype, Qk.const_data_ptr(), Qk.stride(0), Lq, Dk.const_data_ptr(), Dk.stride(0), T, group,
                           lengths, ids, out.data_ptr<float>(), B, Ld, d, ptr(ws), n, s);
   });
   return rc ? failed(rc) : THPVariable_Wrap(std::move(out));
@@ -315,59 +362,68 @@ PyObject* int8_packed(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// forward(Q [Nq, Lq, >= d], D [B, Ld, >= d], lengths, d): (scores [Nq, B], argmax [Nq * B, Lq] int32), of training
+// forward(Q [Nq, Lq, d], D [B, Ld, d], lengths): (scores [Nq, B], argmax [Nq * B, Lq] int32, and Q and D as the
+// kernels read them), of training
 PyObject* forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  FMX_ARGS(4);
+  FMX_ARGS(3);
   const Tensor *Q = plain(args[0]), *D = plain(args[1]);
-  FMX_ORDINARY(Q && D && Q->dim() == 3 && D->dim() == 3 && PyLong_CheckExact(args[3]));
-  const int64_t d = PyLong_AsLongLong(args[3]);
-  if (PyErr_Occurred()) return nullptr;
-  const int64_t Nq = Q->size(0), Lq = Q->size(1), B = D->size(0), Ld = D->size(1);
+  FMX_ORDINARY(Q && D && Q->dim() == 3 && D->dim() == 3 && Q->size(2) == D->size(2));
+  const int64_t Nq = Q->size(0), Lq = Q->size(1), d = Q->size(2), B = D->size(0), Ld = D->size(1);
   const int dtype = kernel_dtype(*Q, *D);
   const int32_t* lengths;
-  FMX_ORDINARY(dtype >= 0 && Nq > 0 && B > 0 && Lq > 0 && d > 0 && d <= Q->size(2) && d <= D->size(2));
-  FMX_ORDINARY(rows_ready(*Q) && rows_ready(*D) && Q->device() == D->device() &&
-               take_lengths(args[2], B, *D, &lengths) && here(*Q));
+  FMX_ORDINARY(dtype >= 0 && Nq > 0 && B > 0 && Lq > 0 && convertible(*Q) && convertible(*D) &&
+               Q->device() == D->device() && take_lengths(args[2], B, *D, &lengths) && here(*Q));
   Tensor scores = at::empty({Nq, B}, D->options().dtype(at::kFloat));
   Tensor argmax = at::empty({Nq * B, Lq}, D->options().dtype(at::kInt));
   const size_t n = fmx_fwd_workspace_bytes(Nq, B, Lq, Ld, d);
   const Tensor ws = scratch(n, *D);
+  FMX_READY(Q, D);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
-    return fmx_fwd(dtype, Q->const_data_ptr(), Q->stride(0), Q->stride(1), D->const_data_ptr(), D->stride(0),
-                   D->stride(1), lengths, scores.data_ptr<float>(), B, 1, argmax.data_ptr<int32_t>(), Nq, B, Lq, Ld, d,
+    return fmx_fwd(dtype, Qk.const_data_ptr(), Qk.stride(0), Qk.stride(1), Dk.const_data_ptr(), Dk.stride(0),
+                   Dk.stride(1), lengths, scores.data_ptr<float>(), B, 1, argmax.data_ptr<int32_t>(), Nq, B, Lq, Ld, d,
                    1, ptr(ws), n, s);
   });
   if (rc) return failed(rc);
-  return Py_BuildValue("(NN)", THPVariable_Wrap(std::move(scores)), THPVariable_Wrap(std::move(argmax)));
+  return Py_BuildValue("(NNNN)", THPVariable_Wrap(std::move(scores)), THPVariable_Wrap(std::move(argmax)),
+                       THPVariable_Wrap(Qk), THPVariable_Wrap(Dk));
   END_HANDLE_TH_ERRORS
 }
 
-// backward(Q, D, lengths, argmax, grad [Nq, B] float32, d, need_q, need_d): (dQ [Nq, Lq, d] or None, dD [B, Ld, d] or None)
+// backward(Q, D, lengths, argmax, grad [Nq, B] float32, d, need_q, need_d, f32): (dQ [Nq, Lq, d] or None,
+// dD [B, Ld, d] or None), float32 when f32 and the operands are fp16, else in their type
 PyObject* backward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  FMX_ARGS(8);
+  FMX_ARGS(9);
   const Tensor *Q = plain(args[0]), *D = plain(args[1]), *am = plain(args[3]), *g = plain(args[4]);
   FMX_ORDINARY(Q && D && am && g && Q->dim() == 3 && D->dim() == 3 && g->dim() == 2 && PyLong_CheckExact(args[5]));
   const int64_t d = PyLong_AsLongLong(args[5]);
   const int need_q = PyObject_IsTrue(args[6]), need_d = PyObject_IsTrue(args[7]);
+  const int want_f32 = PyObject_IsTrue(args[8]);
   if (PyErr_Occurred()) return nullptr;
   const int64_t Nq = Q->size(0), Lq = Q->size(1), B = D->size(0), Ld = D->size(1);
   const int dtype = kernel_dtype(*Q, *D);
   const int32_t* lengths;
-  FMX_ORDINARY(dtype >= 0 && Nq > 0 && Lq > 0 && B > 0 && Ld > 0 && d > 0 && d <= Q->size(2) && d <= D->size(2) &&
+  FMX_ORDINARY(dtype >= 0 && code_of(*Q) == dtype && code_of(*D) == dtype && Nq > 0 && Lq > 0 && B > 0 && Ld > 0 && d > 0 && d <= Q->size(2) && d <= D->size(2) &&
                (need_q || need_d) && rows_ready(*Q) && rows_ready(*D) && is_row_of(am, at::kInt, Nq * B * Lq));
   FMX_ORDINARY(g->scalar_type() == at::kFloat && g->size(0) == Nq && g->size(1) == B && g->stride(0) >= 0 &&
                g->stride(1) >= 0 && Q->device() == D->device() && am->device() == D->device() &&
                g->device() == D->device() && take_lengths(args[2], B, *D, &lengths) && here(*Q));
   Tensor dQ, dD;
-  if (need_q) dQ = at::empty({Nq, Lq, d}, Q->options());
-  if (need_d) dD = at::empty({B, Ld, d}, D->options());
+  const bool f32 = want_f32 && dtype == FMX_DTYPE_F16;
+  const auto options = f32 ? Q->options().dtype(at::kFloat) : Q->options();
+  if (need_q) dQ = at::empty({Nq, Lq, d}, options);
+  if (need_d) dD = at::empty({B, Ld, d}, options);
   const size_t n = fmx_bwd_batched_workspace_bytes(Nq, B, Lq, Ld, d);
   const Tensor ws = scratch(n, *D);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
+    if (f32)
+      return fmx_bwd_batched_f32(Q->const_data_ptr(), Q->stride(0), Q->stride(1), D->const_data_ptr(), D->stride(0),
+                                 D->stride(1), lengths, am->const_data_ptr<int32_t>(), g->const_data_ptr<float>(),
+                                 g->stride(0), g->stride(1), static_cast<float*>(ptr(dQ)), static_cast<float*>(ptr(dD)),
+                                 Nq, B, Lq, Ld, d, ptr(ws), n, s);
     return fmx_bwd_batched(dtype, Q->const_data_ptr(), Q->stride(0), Q->stride(1), D->const_data_ptr(), D->stride(0),
                            D->stride(1), lengths, am->const_data_ptr<int32_t>(), g->const_data_ptr<float>(),
                            g->stride(0), g->stride(1), ptr(dQ), ptr(dD), Nq, B, Lq, Ld, d, ptr(ws), n, s);

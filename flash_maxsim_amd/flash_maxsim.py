@@ -181,10 +181,15 @@ class _FlashMaxSimFn(torch.autograd.Function):
         Q3 = Q if batched else Q.unsqueeze(0)
         Nq, Lq, d = Q3.shape
         B, Ld = D.shape[:2]
-        kdt = _kernel_dtype(Q, D)
-        Qk, Dk = _prep(Q3, kdt), _prep(D, kdt)
-        out = _lib.native().forward(Qk, Dk, lengths, d)
-        scores, argmax = out if out is not None else _launch_fwd(Qk, Dk, lengths, Nq, B, Lq, Ld, d, True, True)
+        out = _lib.native().forward(Q3, D, lengths)
+        if out is not None:
+            scores, argmax, Qk, Dk = out
+        else:
+            kdt = _kernel_dtype(Q, D)
+            Qk, Dk = _prep(Q3, kdt), _prep(D, kdt)
+            scores, argmax = _launch_fwd(Qk, Dk, lengths, Nq, B, Lq, Ld, d, True, True)
+        # float32 leaves take the gradients' fp32 sums as they are, others the kernel dtype
+        ctx.f32 = Q.dtype == D.dtype == torch.float32
         ctx.save_for_backward(Qk, Dk, argmax, lengths)
         ctx.d = d
         ctx.batched = batched
@@ -198,13 +203,15 @@ class _FlashMaxSimFn(torch.autograd.Function):
         B, Ld = Dk.shape[:2]
         need_q, need_d = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         grad = grad_scores if ctx.batched else grad_scores.unsqueeze(0)
-        out = _lib.native().backward(Qk, Dk, lengths, argmax, grad, d, need_q, need_d)
+        out = _lib.native().backward(Qk, Dk, lengths, argmax, grad, d, need_q, need_d, ctx.f32)
         if out is not None:
             grad_Q, grad_D = out
             return (grad_Q if ctx.batched or grad_Q is None else grad_Q[0]), grad_D, None
         dev = _check_devices(Qk, Dk, grad_scores)
-        grad_Q = torch.empty(Nq, Lq, d, device=dev, dtype=Qk.dtype) if need_q else None
-        grad_D = torch.empty(B, Ld, d, device=dev, dtype=Dk.dtype) if need_d else None
+        f32 = ctx.f32 and Qk.dtype == torch.float16
+        out_dtype = torch.float32 if f32 else Qk.dtype
+        grad_Q = torch.empty(Nq, Lq, d, device=dev, dtype=out_dtype) if need_q else None
+        grad_D = torch.empty(B, Ld, d, device=dev, dtype=out_dtype) if need_d else None
         if (grad_Q is None and grad_D is None) or Lq == 0 or Ld == 0 or B == 0:
             if grad_Q is not None:
                 grad_Q.zero_()
@@ -219,9 +226,10 @@ class _FlashMaxSimFn(torch.autograd.Function):
             lib = _lib.load()
             nbytes = lib.fmx_bwd_batched_workspace_bytes(Nq, B, Lq, Ld, d)
             ws = _lib.workspace(nbytes, dev)
+            bwd, kind = (lib.fmx_bwd_batched_f32, ()) if f32 else (lib.fmx_bwd_batched, (_lib.dtype_code(Qk),))
             with _device_guard(dev):
-                rc = lib.fmx_bwd_batched(
-                    _lib.dtype_code(Qk), Qk.data_ptr(), Qk.stride(0), Qk.stride(1), Dk.data_ptr(), Dk.stride(0),
+                rc = bwd(
+                    *kind, Qk.data_ptr(), Qk.stride(0), Qk.stride(1), Dk.data_ptr(), Dk.stride(0),
                     Dk.stride(1), _lib.ptr(lengths), argmax.data_ptr(), g.data_ptr(), g.stride(0), g.stride(1),
                     _lib.ptr(grad_Q), _lib.ptr(grad_D), Nq, B, Lq, Ld, d, _lib.ptr(ws), nbytes, _lib.stream_of(Qk),
                 )
@@ -234,8 +242,9 @@ class _FlashMaxSimFn(torch.autograd.Function):
 def flash_maxsim_train(Q: torch.Tensor, D: torch.Tensor, doc_lengths=None) -> torch.Tensor:
     """flash_maxsim differentiable in Q and D: float32 [B].
 
-    Gradients come back in the kernel dtype (fp16, or bf16 for bf16 inputs);
-    autograd casts them to the leaves' dtypes. Reference signature:
+    Gradients are fp32 sums, stored in the kernel dtype (fp16, or bf16 for bf16
+    inputs), or as they are when both inputs are float32; autograd casts them to
+    the leaves' dtypes. Reference signature:
     flash_maxsim.py:289 (Q, D); doc_lengths is an extension (the reference
     trains on full-length docs only, :260).
     """

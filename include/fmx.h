@@ -40,7 +40,7 @@ extern "C" {
 
 #define FMX_DTYPE_F16 0
 #define FMX_DTYPE_BF16 1
-#define FMX_DTYPE_F32 2 /* fmx_quantize_int8 sources only */
+#define FMX_DTYPE_F32 2 /* sources of fmx_quantize_int8 and fmx_convert_rows only */
 
 /* Widest d. Up to 4096 the forward kernels hold each query slice in
  * registers; wider rows (which the reference reaches by padding d to a power
@@ -341,6 +341,28 @@ int fmx_bwd_batched(int dtype, const void* Q, int64_t q_stride_n, int64_t q_stri
                     const float* grad_scores, int64_t g_stride_n, int64_t g_stride_b, void* dQ, void* dD,
                     int64_t Nq, int64_t B, int64_t Lq, int64_t Ld, int64_t d, void* workspace,
                     size_t workspace_bytes, void* stream);
+
+/*
+ * fmx_bwd_batched of fp16 operands with the gradients written as the fp32 sums
+ * they are (leaves that were float32 before they were cast to fp16: reference
+ * flash_maxsim/flash_maxsim.py:258-259 casts them, autograd casts the fp16
+ * gradients back). Workspace: fmx_bwd_batched_workspace_bytes.
+ */
+int fmx_bwd_batched_f32(const void* Q, int64_t q_stride_n, int64_t q_stride_l, const void* D, int64_t d_stride_b,
+                        int64_t d_stride_l, const int32_t* lengths, const int32_t* argmax, const float* grad_scores,
+                        int64_t g_stride_n, int64_t g_stride_b, float* dQ, float* dD, int64_t Nq, int64_t B, int64_t Lq,
+                        int64_t Ld, int64_t d, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * Operand rows made ready for the other entry points in one pass: rows of d
+ * elements, [B, Ld] of them at strides s_stride_b and s_stride_l, to contiguous
+ * rows of dp elements (a multiple of 8, dp >= d) in dst (16-byte aligned), zeros
+ * past d. FMX_DTYPE_F32 and FMX_DTYPE_BF16 to FMX_DTYPE_F16 round to nearest
+ * even; FMX_DTYPE_F16 and FMX_DTYPE_BF16 to themselves are moved. (The
+ * reference casts and copies with torch, flash_maxsim/flash_maxsim.py:226-227.)
+ */
+int fmx_convert_rows(int src_dtype, const void* src, int64_t s_stride_b, int64_t s_stride_l, int64_t B, int64_t Ld,
+                     int64_t d, int dst_dtype, void* dst, int64_t dp, void* stream);
 
 /* Workspace of fmx_bwd_batched: as fmx_bwd_workspace_bytes with Nq*Lq entries per doc. */
 size_t fmx_bwd_batched_workspace_bytes(int64_t Nq, int64_t B, int64_t Lq, int64_t Ld, int64_t d);

@@ -148,11 +148,78 @@ def test_native_takes_the_ordinary_calls():
     Q, D = sim((2, 20, 128), 11, torch.float16).to(DEV), sim((6, 36, 128), 12, torch.float16).to(DEV)
     n = _lib.native()
     assert n.score(Q[0], D, None) is not None and n.batched(Q, D, None, True) is not None
-    assert n.topk(Q[0], D, 3, None) is not None and n.forward(Q, D, None, 128) is not None
-    assert n.score(Q[0].cpu(), D, None) is None and n.score(Q[0].float(), D, None) is None
+    assert n.topk(Q[0], D, 3, None) is not None and n.forward(Q, D, None) is not None
+    assert n.score(Q[0].float(), D[..., :100], None) is None  # shapes are the Python path's to refuse
+    assert n.score(Q[0].float(), D, None) is not None and n.score(Q[0][:, 1:], D[..., 1:], None) is not None
+    assert n.score(Q[0].cpu(), D, None) is None and n.score(Q[0].double(), D, None) is None
     assert n.score(Q[0], [1], None) is None
     with pytest.raises(TypeError):
         n.score(Q[0], D)
+
+
+@pytest.mark.parametrize("d", [1, 4, 7, 8, 30, 100, 128, 130])
+@pytest.mark.parametrize("kinds", [("f32", "f16"), ("bf16", "f16"), ("f16", "f16"), ("bf16", "bf16")])
+def test_convert_rows_bitwise_torch(d, kinds):
+    """fmx_convert_rows against torch's cast and pad: halfway cases, overflow to
+    infinity, fp16 subnormals, NaN, strided rows, sources off alignment."""
+    types = {"f16": (torch.float16, 0), "bf16": (torch.bfloat16, 1), "f32": (torch.float32, 2)}
+    (src_t, src_c), (dst_t, dst_c) = types[kinds[0]], types[kinds[1]]
+    gen = torch.Generator().manual_seed(2800 + d)
+    x = torch.randn(3, 21, d + 3, generator=gen)
+    x[0] *= 2.0 ** torch.randint(-30, 20, (21, d + 3), generator=gen)
+    x[1, :4, 0] = torch.tensor([float("inf"), float("nan"), 65520.0, -65519.0])
+    x[2, :5] = torch.tensor([1 + 2.0**-11, 1 + 3 * 2.0**-11, 2.0**-25, 3 * 2.0**-25, 0.0])[:, None]
+    x = x.to(src_t).to(DEV)
+    dp = (d + 7) // 8 * 8
+    for lead in (0, 1, 3):
+        for v in (x[..., lead : lead + d], x[..., lead : lead + d].contiguous(), x[:1, :, lead : lead + d].expand(3, 21, d)):
+            out = torch.full((3, 21, dp), 7.0, dtype=dst_t, device=DEV)
+            _lib.check(_lib.load().fmx_convert_rows(src_c, v.data_ptr(), v.stride(0), v.stride(1), 3, 21, d, dst_c,
+                                                    out.data_ptr(), dp, torch.cuda.current_stream().cuda_stream))
+            want = torch.nn.functional.pad(v.to(dst_t), (0, dp - d))
+            nan = torch.isnan(want)
+            assert torch.equal(torch.isnan(out), nan)
+            assert torch.equal(out.masked_fill(nan, 0).view(torch.int16), want.masked_fill(nan, 0).view(torch.int16))
+
+
+@pytest.mark.parametrize("Nq, B, Lq, Ld, d", [(1, 40, 20, 33, 128), (3, 12, 50, 30, 100), (1, 6, 300, 9, 30), (9, 5, 40, 17, 520),
+                                              (2, 4, 30, 40, 1100), (1, 3, 5, 2, 7)])
+def test_float32_gradients_are_the_sums(Nq, B, Lq, Ld, d):
+    """float32 leaves: gradients against float64 sums over the same argmax, to the
+    rounding of an fp32 sum of that many terms, in both writers and past one
+    wave's width; the same by a 2-byte store of the same sums for fp16 leaves."""
+    gen = torch.Generator().manual_seed(2900 + d)
+    Q = (torch.randint(-8, 9, (Nq, Lq, d), generator=gen) / 8).to(DEV)
+    D = (torch.randint(-8, 9, (B, Ld, d), generator=gen) / 8).to(DEV)
+    g = torch.randn(Nq, B, generator=gen).to(DEV)
+    ln = torch.randint(1, Ld + 1, (B,), generator=gen, dtype=torch.int32).to(DEV)
+    grads = {}
+    for dtype in (torch.float32, torch.float16):
+        q, x = Q.to(dtype).requires_grad_(True), D.to(dtype).requires_grad_(True)
+        s = fm.flash_maxsim_train_batched(q, x, ln)
+        grads[dtype] = torch.autograd.grad(s, (q, x), g)
+    _, am = _argmax(Q, D, ln, Nq, B, Lq, Ld, d)
+    am = am.view(Nq, B, Lq).long()
+    dQ, dD = torch.zeros(Nq, Lq, d, dtype=torch.float64), torch.zeros(B, Ld, d, dtype=torch.float64)
+    aQ, aD = dQ.clone(), dD.clone()  # sums of absolute values
+    Qc, Dc, gc, amc = Q.double().cpu(), D.double().cpu(), g.double().cpu(), am.cpu()
+    for i in range(Nq):
+        for b in range(B):
+            rows = Dc[b][amc[i, b]]
+            dQ[i] += gc[i, b] * rows
+            aQ[i] += (gc[i, b] * rows).abs()
+            dD[b].index_add_(0, amc[i, b], gc[i, b] * Qc[i])
+            aD[b].index_add_(0, amc[i, b], (gc[i, b] * Qc[i]).abs())
+    for got, half, want, total, terms in zip(grads[torch.float32], grads[torch.float16], (dQ, dD), (aQ, aD), (B, Nq * Lq)):
+        assert got.dtype == torch.float32
+        assert ((got.double().cpu() - want).abs() <= terms * 2.0**-24 * total).all()
+        assert torch.equal(got.half(), half)
+
+
+def _argmax(Q, D, ln, Nq, B, Lq, Ld, d):
+    from flash_maxsim_amd.flash_maxsim import _launch_fwd, _prep
+
+    return _launch_fwd(_prep(Q, torch.float16), _prep(D, torch.float16), ln, Nq, B, Lq, Ld, d, True, True)
 
 
 def test_native_launches_on_the_current_stream():
