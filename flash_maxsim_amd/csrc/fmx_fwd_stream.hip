@@ -758,6 +758,172 @@ __global__ void __launch_bounds__(256) stream_u8_shared_kernel(FwdArgs a) {
   }
 }
 
+// Many short docs of one query (fp16/bf16, one pass of 17-32 tokens, d in (64,
+// 128], docs of up to 96 tokens): a wave scores whole docs alone. A workgroup
+// takes G consecutive docs, which its four waves draw from a counter in LDS; a
+// wave's ring of P tiles runs on from one doc to the next, and a doc ends with
+// the wave's own reduction. Dealing a doc's few tiles to four waves, as
+// stream_fwd_kernel does, leaves waves without a tile where docs have one to
+// five, and merges four waves' maxima per doc behind a barrier. 32 tokens,
+// docs all long / of U[0, Ld]: 20000 docs of 77 tokens 76.9 / 44.9 -> 68.6 /
+// 37.9 us, of 40 40.3 / 33.8 -> 35.0 / 24.2, at d = 96 57.1 / 38.3 -> 51.0 /
+// 30.6. Three tiles in flight (four: 74.0 / 41.1, a wave per SIMD less).
+// G: eight docs a workgroup, sixteen from 2^15 docs (60000 docs of U[0, 50]
+// tokens 77 -> 69 us; 20000 of 77 39.1 against 37.9, and 32 41.4). The line at
+// 2^13 docs: below it the groups are too few to fill the GPU (5000 docs of 77
+// tokens 17.9 / 13.4 -> 21.4 / 14.9). Queries of 16 tokens (63.2 / 34.0 ->
+// 68.0 / 35.5), longer docs (128 tokens 112.6 -> 114.3) and d <= 64 (equal)
+// stay with stream_fwd_kernel.
+constexpr int64_t kDocsMin = 1 << 13;
+bool stream_docs_takes(const FwdArgs& a) {
+  return a.Nq == 1 && !a.qidx && a.Ld <= 96 && a.B >= kDocsMin;
+}
+
+template <int KIND, int NQB, int KS, bool KMASK, int P>
+__global__ void __launch_bounds__(256) stream_docs_kernel(FwdArgs a, int G) {  // G <= 64: a lane per doc
+  constexpr int NW = kStreamWaves, NF = NQB * KS;
+  constexpr bool BF = KindInfo<KIND>::bf;
+  static_assert(KIND != KIND_U8, "2-byte docs");
+  __shared__ u32x4_t qs[NF][64];
+  __shared__ int taken;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int64_t b0 = (int64_t)blockIdx.x * G;
+  const int docs = a.B - b0 < G ? (int)(a.B - b0) : G;
+  if (threadIdx.x == 0) taken = NW;  // the waves start with docs 0 .. NW - 1
+
+  // lane i: length of the group's doc i
+  int lens = 0;
+  if (lane < docs) {
+    lens = a.lengths ? a.lengths[b0 + lane] : a.Ld;
+    lens = lens < 0 ? 0 : (lens > a.Ld ? a.Ld : lens);
+  }
+
+  // query fragments: each wave loads every NW-th, they meet in LDS
+  const int kp = a.d & ~7;
+  int tp, gp;
+  frag_slot<KIND>(kp, tp, gp);
+  const u32x4_t pmask = prefix_mask16(g == gp ? (a.d & 7) : 8);
+  const bool has_partial = KMASK && (a.d & 7) != 0;
+  const rsrc_t rq = make_rsrc(a.Q, (uint32_t)(a.Lq_rows * a.sq_l * 2));
+#pragma unroll
+  for (int j = 0; j < (NF + NW - 1) / NW; ++j) {
+    const int f = wave + NW * j;
+    if (f < NF) {
+      const int nb = f / KS, t = f - nb * KS, k0 = frag_k0<KIND>(t, g);
+      u32x4_t v = ld16(rq, !KMASK || k0 < a.d ? query_row_offset(a, 0, nb * 16 + c) + (uint32_t)(k0 * 2) : kOOB);
+      if (has_partial && t == tp) v &= pmask;
+      qs[f][lane] = v;
+    }
+  }
+  __syncthreads();
+  u32x4_t qf[NQB][KS];
+#pragma unroll
+  for (int nb = 0; nb < NQB; ++nb)
+#pragma unroll
+    for (int t = 0; t < KS; ++t) qf[nb][t] = qs[nb * KS + t][lane];
+  uint32_t koff[KS];
+#pragma unroll
+  for (int t = 0; t < KS; ++t) {
+    const int k0 = frag_k0<KIND>(t, g);
+    koff[t] = (KMASK && k0 >= a.d) ? kOOB : (uint32_t)(k0 * 2);
+  }
+
+  // Fetch cursor: tile ft of doc fi (of the group), of fn tiles; fi >= docs: none left.
+  int fi = wave, ft = 0, fn = 0, flen = 0;
+  DocRes fr = make_doc_res<KIND, true>(a, b0, 0);
+  auto open = [&]() __attribute__((always_inline)) {
+    if (fi < docs) {
+      flen = __builtin_amdgcn_readlane(lens, fi);
+      fn = flen > 0 ? (flen + 15) >> 4 : 1;  // an empty doc takes one tile, all masked
+      fr = make_doc_res<KIND, true>(a, b0 + fi, flen);
+    } else {
+      fr.d = make_rsrc(a.D, 0u);  // reads zeros, no memory access: a fixed load count
+    }
+    ft = 0;
+  };
+  // Ring slot: its tile, and which doc's it is.
+  struct Slot {
+    Tile<KIND, KS> t;
+    int doc, tile, len, last;  // uniform; doc >= docs: no tile
+  };
+  Slot ring[P];
+  auto fetch = [&](Slot& S) __attribute__((always_inline)) {
+    load_tile<KIND, KS, true>(S.t, fr, ft, c, g, koff);
+    S.doc = fi;
+    S.tile = ft;
+    S.len = flen;
+    S.last = ft + 1 >= fn;
+    if (fi < docs && ++ft >= fn) {
+      int n = 0;
+      if (lane == 0) n = atomicAdd(&taken, 1);
+      fi = __builtin_amdgcn_readfirstlane(n);
+      open();
+    }
+  };
+  open();
+#pragma unroll
+  for (int s = 0; s < P; ++s) fetch(ring[s]);
+
+  float m[NQB];
+#pragma unroll
+  for (int nb = 0; nb < NQB; ++nb) m[nb] = -INFINITY;
+  auto step = [&](Slot& S) __attribute__((always_inline)) -> bool {
+    const int doc = S.doc, tile = S.tile, len = S.len, last = S.last;
+    if (doc >= docs) return false;
+    u32x4_t af[KS];
+#pragma unroll
+    for (int t = 0; t < KS; ++t) {
+      af[t] = S.t.v[t];
+      if (has_partial && t == tp) af[t] &= pmask;
+    }
+    fetch(S);
+    // full and partial tiles are separate instances, each with its MFMAs and
+    // the first reads of their results in one basic block
+    auto score = [&](auto tail_tag) __attribute__((always_inline)) {
+      constexpr bool TAIL = decltype(tail_tag)::value;
+      const int row0 = tile * 16 + 4 * g;
+#pragma unroll
+      for (int nb = 0; nb < NQB; ++nb) {
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < KS; ++t) acc = mfma16x16x32<BF>(af[t], qf[nb][t], acc);
+        if constexpr (TAIL) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[r] = row0 + r < len ? acc[r] : -INFINITY;
+        }
+        m[nb] = fold_max4(m[nb], acc[0], acc[1], acc[2], acc[3]);
+      }
+    };
+    if (tile * 16 + 16 > len) {
+      score(std::true_type{});
+    } else {
+      score(std::false_type{});
+    }
+    if (last) {
+      // sum over the query tokens in wave_sum's order over lanes = tokens: each
+      // block's 16 columns first, then the blocks
+      float total = 0.f;
+#pragma unroll
+      for (int nb = 0; nb < NQB; ++nb) {
+        float v = max_over_groups(m[nb]);
+        v = group_sum(nb * 16 + c < a.Lq ? v : 0.f, 16);
+        total = nb == 0 ? v : total + v;
+        m[nb] = -INFINITY;
+      }
+      if (lane == 0) store_score(a, 0, b0 + doc, total);
+    }
+    return true;
+  };
+  for (;;) {
+    bool more = true;
+#pragma unroll
+    for (int s = 0; s < P; ++s) more = more && step(ring[s]);
+    if (!more) break;
+  }
+}
+
 template <int KIND, int NQB, int KS, bool KMASK, bool ARGMAX, bool VEC = true, bool C16 = VEC>
 hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
   constexpr int QROWS = NQB * 16;
@@ -844,6 +1010,14 @@ hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
     // Per-query docs pair two of one query's docs (100 queries x 1000 docs
     // of 77 tokens: 577 -> 376 us).
     constexpr bool BIG = NQB * KS >= 32;
+    if constexpr (NQB == 2 && KS == 4) {
+      if (npass == 1 && stream_docs_takes(a)) {
+        const int G = a.B >= (1 << 15) ? 16 : 8;
+        hipLaunchKernelGGL((stream_docs_kernel<KIND, NQB, KS, KMASK, 3>), dim3((unsigned)((a.B + G - 1) / G)), dim3(256),
+                           0, s, a, G);
+        return hipGetLastError();
+      }
+    }
     if (!BIG && (a.Nq == 1 || !a.shared_docs) && npass == 1 && !a.qidx && a.Ld <= 128) {
       // docs of up to 128 tokens: a two-tile ring, as for uint8 (Lq = 32 over
       // 20000 docs of 77 tokens 75.8 -> 62.2 us, 10000 of 64 -19 %, 5000 of 77
