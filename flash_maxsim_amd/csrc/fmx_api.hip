@@ -522,7 +522,7 @@ int fmx_pack_rows(const void* src, int64_t s_stride_b, int64_t s_stride_l, int64
 
 size_t fmx_topk_workspace_bytes(int64_t Nq, int64_t B, int64_t k) {
   if (Nq < 1 || B < 1 || k < 1 || k > FMX_MAX_TOPK) return 0;
-  return (size_t)fmx::topk_ws_keys(Nq, B, k, fmx::topk_chunk((int)k)) * sizeof(uint64_t);
+  return (size_t)fmx::topk_ws_keys(Nq, B, k, fmx::topk_chunk(Nq, B, k)) * sizeof(uint64_t);
 }
 
 int fmx_topk(const float* scores, int64_t s_stride_n, int64_t Nq, int64_t B, int64_t k, float* values,

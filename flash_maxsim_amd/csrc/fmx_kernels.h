@@ -167,9 +167,9 @@ struct TopkArgs {
   float* values;              // [Nq, k], row stride o_stride
   int64_t* indices;           // [Nq, k], row stride o_stride
   int64_t o_stride;
-  uint64_t* ws;               // topk_ws_keys(Nq, B, k, topk_chunk(k)) keys
+  uint64_t* ws;               // topk_ws_keys(Nq, B, k, topk_chunk(Nq, B, k)) keys
 };
-int topk_chunk(int k);                                            // keys sorted per workgroup
+int64_t topk_chunk(int64_t Nq, int64_t B, int64_t k);             // keys per workgroup of the first level
 int64_t topk_ws_keys(int64_t Nq, int64_t B, int64_t k, int64_t C);
 hipError_t launch_topk(const TopkArgs& a, hipStream_t s);
 

@@ -649,10 +649,11 @@ template <int MAXK>
 hipError_t run_levels(const TopkArgs& a, hipStream_t s) {
   int64_t n = a.B;
   const uint64_t* in = nullptr;
-  uint64_t* bufs[2] = {a.ws, a.ws + topk_ws_keys(a.Nq, a.B, a.k, kTopkC) / 2};
+  uint64_t* bufs[2] = {a.ws, a.ws + topk_ws_keys(a.Nq, a.B, a.k, topk_chunk(a.Nq, a.B, a.k)) / 2};
   int which = 0;
   while (true) {
-    const int64_t chunks = (n + kTopkC - 1) / kTopkC;
+    const int64_t C = in ? kTopkC : topk_chunk(a.Nq, a.B, a.k);  // keys per workgroup of this level
+    const int64_t chunks = (n + C - 1) / C;
     const bool last = chunks == 1;
     if (chunks > 0x7fffffff || a.Nq > 65535) return hipErrorInvalidValue;
     uint64_t* out = last ? nullptr : bufs[which];
@@ -670,7 +671,7 @@ hipError_t run_levels(const TopkArgs& a, hipStream_t s) {
       }
     } else {
       constexpr int T = kTopkThreads;
-      auto kern = n <= 4 * T ? topk_level_kernel<T, 4, MAXK>
+      auto kern = n <= 4 * T || C == 4 * T ? topk_level_kernel<T, 4, MAXK>
                 : n <= 8 * T ? topk_level_kernel<T, 8, MAXK> : topk_level_kernel<T, 16, MAXK>;
       hipLaunchKernelGGL(kern, dim3((unsigned)chunks, (unsigned)a.Nq), dim3(T), 0, s, a.scores, a.s_stride, in, n,
                          a.k, out, last ? a.values : nullptr, last ? a.indices : nullptr, a.o_stride);
@@ -685,9 +686,14 @@ hipError_t run_levels(const TopkArgs& a, hipStream_t s) {
 
 }  // namespace
 
-int topk_chunk(int k) {
-  (void)k;
-  return kTopkC;
+// Keys per workgroup of the first level: 16384, or for one row past that 4096
+// where it then still ends with one more level (up to 64 chunks of k <= 128
+// keys), each workgroup's chain of loads, bound and packing over a quarter of
+// the keys (the best 100 of 20000: first level 7.7 -> 6.2 us). Rows of up to
+// 16384 keys are one launch as they are (9000: 10.4 against 14.3 us), and many
+// rows fill the GPU with the larger chunks (128 of 40000: 20.0 against 28.9).
+int64_t topk_chunk(int64_t Nq, int64_t B, int64_t k) {
+  return Nq == 1 && k <= kTopkSmallK && B > kTopkC && B <= 64 * 4 * kTopkThreads ? 4 * kTopkThreads : kTopkC;
 }
 
 // Keys of both ping-pong buffers: level 1 holds ceil(B / C) * k keys per row,

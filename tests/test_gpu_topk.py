@@ -238,3 +238,15 @@ def test_one_call_topk_many_calls(oracle_mod):
         same = torch.equal(i, wi) and torch.equal(v.view(torch.int32), wv.view(torch.int32))
         bad += 0 if same else 1
     assert bad == 0, f"{bad} of 300 selections differ"
+
+
+@pytest.mark.parametrize("Nq, B, k", [(1, 16384, 100), (1, 16385, 100), (1, 20481, 128), (1, 20000, 129), (1, 262144, 128),
+                                      (1, 262145, 10), (1, 65537, 1), (2, 20000, 100)])
+def test_topk_first_level_chunks(oracle_mod, Nq, B, k):
+    """One row's first level over chunks of 4096 keys and its neighbours over
+    16384: chunk remainders, a row of equal scores, the best keys in one chunk."""
+    s = scores_with_ties(B + k, (Nq, B))
+    got = fm.topk_scores(torch.from_numpy(s).to(DEV), k)
+    assert_same_selection(got, oracle_mod.topk(s, k))
+    for s in (np.full((Nq, B), 0.5, np.float32), -np.arange(Nq * B, dtype=np.float32).reshape(Nq, B)):
+        assert_same_selection(fm.topk_scores(torch.from_numpy(s).to(DEV), k), oracle_mod.topk(s, k))
