@@ -86,20 +86,23 @@ size_t fwd_ws_bytes(int64_t Nq, int64_t B, int64_t Lq, int64_t Ld, int64_t d) {
   return n;
 }
 
-// Checks shared by the forward entry points. esz: bytes per D element.
+// Checks shared by the forward entry points. esz: bytes per D element; rows are
+// 16-byte aligned (uint8 rows 8), so strides are multiples of 8 elements, of
+// 4 for fp32.
 int check_common(int64_t Nq, int64_t B, int64_t Lq, int64_t Ld, int64_t d, int64_t q_stride_l,
                  int64_t d_stride_b, int64_t d_stride_l, int esz) {
+  const int m = esz == 4 ? 3 : 7;
   if (Nq < 1 || B < 0 || Lq < 1 || Ld < 0 || d < 1)
     return fail(FMX_ERR_INVALID, "invalid sizes Nq=%lld B=%lld Lq=%lld Ld=%lld d=%lld", (long long)Nq,
                 (long long)B, (long long)Lq, (long long)Ld, (long long)d);
   if (d > FMX_MAX_D) return fail(FMX_ERR_UNSUPPORTED, "d=%lld exceeds FMX_MAX_D=%d", (long long)d, FMX_MAX_D);
-  if (q_stride_l < d || (q_stride_l & 7))
-    return fail(FMX_ERR_INVALID, "Q row stride %lld must be >= d and a multiple of 8", (long long)q_stride_l);
-  if (d_stride_l < d || (d_stride_l & 7))
-    return fail(FMX_ERR_INVALID, "D row stride %lld must be >= d and a multiple of 8", (long long)d_stride_l);
-  if (d_stride_b & 7) return fail(FMX_ERR_INVALID, "D doc stride %lld must be a multiple of 8", (long long)d_stride_b);
+  if (q_stride_l < d || (q_stride_l & m))
+    return fail(FMX_ERR_INVALID, "Q row stride %lld must be >= d and a multiple of %d", (long long)q_stride_l, m + 1);
+  if (d_stride_l < d || (d_stride_l & m))
+    return fail(FMX_ERR_INVALID, "D row stride %lld must be >= d and a multiple of %d", (long long)d_stride_l, m + 1);
+  if (d_stride_b & m) return fail(FMX_ERR_INVALID, "D doc stride %lld must be a multiple of %d", (long long)d_stride_b, m + 1);
   if (Nq * B >= kOffLimit) return fail(FMX_ERR_UNSUPPORTED, "Nq*B=%lld too large", (long long)(Nq * B));
-  if ((Lq + 128) * q_stride_l * 2 >= kOffLimit)
+  if ((Lq + 128) * q_stride_l * (esz == 4 ? 4 : 2) >= kOffLimit)
     return fail(FMX_ERR_UNSUPPORTED, "query of %lld x %lld elements exceeds 2 GiB", (long long)Lq,
                 (long long)q_stride_l);
   if ((Ld + 16) * d_stride_l * esz >= kOffLimit)
@@ -158,6 +161,8 @@ size_t fmx_fwd_workspace_bytes(int64_t Nq, int64_t B, int64_t Lq, int64_t Ld, in
   return fwd_ws_bytes(Nq, B, Lq, Ld, d);
 }
 
+int fmx_fwd_reads_f32(int64_t Lq, int64_t d) { return Lq >= 1 && Lq <= 32 && d >= 1 && d <= 128; }
+
 size_t fmx_fwd_int8_workspace_bytes(int64_t B, int64_t Lq, int64_t Ld, int64_t d) {
   return fwd_ws_bytes(1, B, Lq, Ld, d);  // every kernel family takes uint8 docs
 }
@@ -172,14 +177,18 @@ int fwd_impl(int dtype, const void* Q, int64_t q_stride_n, int64_t q_stride_l, c
              int64_t s_stride_n, int64_t s_stride_b, int32_t* argmax, int64_t Nq, int64_t B, int64_t Lq, int64_t Ld,
              int64_t d, int shared_docs, void* workspace, size_t workspace_bytes, void* stream,
              bool noalloc = false, const int32_t* doc_ids = nullptr) {
-  if (dtype != FMX_DTYPE_F16 && dtype != FMX_DTYPE_BF16) return fail(FMX_ERR_INVALID, "unknown dtype %d", dtype);
-  int rc = check_common(Nq, B, Lq, Ld, d, q_stride_l, d_stride_b, d_stride_l, 2);
+  if (dtype != FMX_DTYPE_F16 && dtype != FMX_DTYPE_BF16 && dtype != FMX_DTYPE_F32)
+    return fail(FMX_ERR_INVALID, "unknown dtype %d", dtype);
+  const bool f32 = dtype == FMX_DTYPE_F32;
+  if (f32 && (Nq != 1 || argmax || !fmx_fwd_reads_f32(Lq, d)))
+    return fail(FMX_ERR_UNSUPPORTED, "fp32 operands: one query of up to 32 tokens, d <= 128, no argmax");
+  int rc = check_common(Nq, B, Lq, Ld, d, q_stride_l, d_stride_b, d_stride_l, f32 ? 4 : 2);
   if (rc) return rc;
   if (B == 0) return ok();
   if (!Q || !D || !scores) return fail(FMX_ERR_INVALID, "Q, D and scores must be non-null");
   if (!aligned16(Q) || !aligned16(D)) return fail(FMX_ERR_INVALID, "Q and D must be 16-byte aligned");
   if (Nq > 1 && (q_stride_n & 7)) return fail(FMX_ERR_INVALID, "Q query stride must be a multiple of 8");
-  const bool tiled = use_tiled(Nq, Lq, Ld, d, shared_docs);
+  const bool tiled = !f32 && use_tiled(Nq, Lq, Ld, d, shared_docs);
   fmx::TiledPlan tp = {};
   size_t need;
   if (tiled) {
@@ -230,7 +239,7 @@ int fwd_impl(int dtype, const void* Q, int64_t q_stride_n, int64_t q_stride_l, c
   a.Ld = (int)Ld;
   a.d = (int)d;
   a.shared_docs = shared_docs ? 1 : 0;
-  const int kind = dtype == FMX_DTYPE_BF16 ? fmx::KIND_BF16 : fmx::KIND_F16;
+  const int kind = f32 ? fmx::KIND_F32 : dtype == FMX_DTYPE_BF16 ? fmx::KIND_BF16 : fmx::KIND_F16;
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e;
   if (tiled) {
@@ -377,7 +386,7 @@ int fmx_fwd_topk(int dtype, const void* Q, int64_t q_stride_l, const void* D, in
   if (k < 0 || B < 0) return fail(FMX_ERR_INVALID, "invalid sizes B=%lld k=%lld", (long long)B, (long long)k);
   if (k > B) return fail(FMX_ERR_INVALID, "k=%lld exceeds the %lld scores", (long long)k, (long long)B);
   if (k > FMX_MAX_TOPK) return fail(FMX_ERR_UNSUPPORTED, "k=%lld exceeds FMX_MAX_TOPK=%d", (long long)k, FMX_MAX_TOPK);
-  int rc = check_common(1, B, Lq, Ld, d, q_stride_l, d_stride_b, d_stride_l, 2);
+  int rc = check_common(1, B, Lq, Ld, d, q_stride_l, d_stride_b, d_stride_l, dtype == FMX_DTYPE_F32 ? 4 : 2);
   if (rc) return rc;
   if (k > 0 && (!values || !indices)) return fail(FMX_ERR_INVALID, "values and indices must be non-null");
   const size_t need = fmx_fwd_topk_workspace_bytes(B, Lq, Ld, d, k);
@@ -562,9 +571,13 @@ int fmx_fwd_sparse(int dtype, const void* Q, int64_t q_stride_l, int64_t Lq, con
                    int64_t d_stride_b, int64_t d_stride_l, const int32_t* indices, int64_t idx_stride_b,
                    int64_t idx_stride_k, int64_t K, const int32_t* lengths, float* scores, int64_t B,
                    int64_t Ld, int64_t d, void* workspace, size_t workspace_bytes, void* stream) {
-  if (dtype != FMX_DTYPE_F16 && dtype != FMX_DTYPE_BF16) return fail(FMX_ERR_INVALID, "unknown dtype %d", dtype);
+  if (dtype != FMX_DTYPE_F16 && dtype != FMX_DTYPE_BF16 && dtype != FMX_DTYPE_F32)
+    return fail(FMX_ERR_INVALID, "unknown dtype %d", dtype);
+  const bool f32 = dtype == FMX_DTYPE_F32;
+  if (f32 && K >= 1 && !fmx_fwd_reads_f32(K, d))
+    return fail(FMX_ERR_UNSUPPORTED, "fp32 operands: up to 32 query tokens a doc, d <= 128");
   if (Lq < 1) return fail(FMX_ERR_INVALID, "Lq=%lld must be >= 1", (long long)Lq);
-  int rc = check_common(1, B, K > Lq ? K : Lq, Ld, d, q_stride_l, d_stride_b, d_stride_l, 2);
+  int rc = check_common(1, B, K > Lq ? K : Lq, Ld, d, q_stride_l, d_stride_b, d_stride_l, f32 ? 4 : 2);
   if (rc) return rc;
   if (K < 1) return fail(FMX_ERR_INVALID, "K=%lld must be >= 1", (long long)K);
   if (B == 0) return ok();
@@ -597,7 +610,7 @@ int fmx_fwd_sparse(int dtype, const void* Q, int64_t q_stride_l, int64_t Lq, con
   a.Ld = (int)Ld;
   a.d = (int)d;
   a.shared_docs = 1;
-  const int kind = dtype == FMX_DTYPE_BF16 ? fmx::KIND_BF16 : fmx::KIND_F16;
+  const int kind = f32 ? fmx::KIND_F32 : dtype == FMX_DTYPE_BF16 ? fmx::KIND_BF16 : fmx::KIND_F16;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const FwdPlan p = plan_fwd(K, d);
   const hipError_t e = p.wide     ? fmx::launch_wide_fwd(kind, a, false, static_cast<float*>(workspace), workspace_bytes, s)

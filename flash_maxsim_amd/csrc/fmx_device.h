@@ -31,11 +31,14 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x3_t __attribute__((ext_vector_type(3)));
 
 // Element kinds of the document operand.
-enum Kind : int { KIND_F16 = 0, KIND_BF16 = 1, KIND_U8 = 2 };
+// KIND_F32: fp32 docs and query, rounded to fp16 on their way to the MFMA (as a
+// cast beforehand would round them).
+enum Kind : int { KIND_F16 = 0, KIND_BF16 = 1, KIND_U8 = 2, KIND_F32 = 3 };
 
 template <int KIND> struct KindInfo;
 template <> struct KindInfo<KIND_F16> { static constexpr int esz = 2; static constexpr bool bf = false; };
 template <> struct KindInfo<KIND_BF16> { static constexpr int esz = 2; static constexpr bool bf = true; };
+template <> struct KindInfo<KIND_F32> { static constexpr int esz = 4; static constexpr bool bf = false; };
 // uint8 codes are widened to fp16 and multiplied against an fp16 query.
 template <> struct KindInfo<KIND_U8> { static constexpr int esz = 1; static constexpr bool bf = false; };
 
@@ -188,6 +191,18 @@ __device__ __forceinline__ float half_bits_to_float(uint32_t bits16) {
 }
 __device__ __forceinline__ float bf16_bits_to_float(uint32_t bits16) {
   return __builtin_bit_cast(float, bits16 << 16);
+}
+
+// Eight fp32 values rounded to fp16 (to nearest even, overflow to infinity).
+__device__ __forceinline__ u32x4_t f32_to_f16x8(u32x4_t lo, u32x4_t hi) {
+  u32x4_t o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t a = i < 2 ? lo[2 * i] : hi[2 * i - 4], b = i < 2 ? lo[2 * i + 1] : hi[2 * i - 3];
+    o[i] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)__builtin_bit_cast(float, a)) |
+           ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)__builtin_bit_cast(float, b)) << 16);
+  }
+  return o;
 }
 
 // Row sums of a 16-token fp16 query block held as B-fragments qf[0..KS-1]:

@@ -45,7 +45,7 @@ constexpr int kStreamWaves = 4;
 // against two tiles; three measured no better than two).
 template <int KIND, int NQB, int KS>
 constexpr int stream_depth() {
-  return (KIND != KIND_U8 && KS >= 8) ? 2 : 4;
+  return (KIND != KIND_U8 && KS >= 8) || (KIND == KIND_F32 && KS >= 4) ? 2 : 4;
 }
 
 // Doc tiles through a per-wave LDS ring (stream_fwd_kernel's DMA path) for
@@ -54,7 +54,7 @@ constexpr int stream_depth() {
 // wave (8 KB of LDS each), uint8 with the group scale loads' four (2 KB each).
 template <int KIND, int KS, bool KMASK, bool ARGMAX, int PD>
 constexpr bool stream_dma_fp() {
-  return KIND != KIND_U8 && KS == 4 && !KMASK && !ARGMAX && PD == 0;
+  return KIND != KIND_U8 && KIND != KIND_F32 && KS == 4 && !KMASK && !ARGMAX && PD == 0;
 }
 constexpr int kStreamDmaDepth = 2;
 // Docs of this many bytes or more (docs x Ld x d x element size) outgrow the
@@ -214,7 +214,8 @@ stream_fwd_kernel(FwdArgs a) {
 
   // ---- query tile of this pass (B operand) ----
   const int q0 = pass * QROWS;
-  const rsrc_t rq = make_rsrc((const char*)a.Q + (int64_t)qi * a.sq_n * 2, (uint32_t)(a.Lq_rows * a.sq_l * 2));
+  constexpr int QSZ = KIND == KIND_F32 ? 4 : 2;  // bytes per query element
+  const rsrc_t rq = make_rsrc((const char*)a.Q + (int64_t)qi * a.sq_n * QSZ, (uint32_t)(a.Lq_rows * a.sq_l * QSZ));
   // Each wave loads every NW-th fragment of the query tile; the fragments
   // meet in LDS once the first doc tiles are in flight (q_exchange), so the
   // workgroup issues the query loads once instead of once per wave.
@@ -243,7 +244,11 @@ stream_fwd_kernel(FwdArgs a) {
       const int nb = f / KS, t = f - (f / KS) * KS;
       const uint32_t rowoff = query_row_offset(a, b, q0 + nb * 16 + c);
       const int k0 = frag_k0<KIND>(t, g);
-      if constexpr (KMASK) {
+      if constexpr (KIND == KIND_F32) {
+        const uint32_t o = rowoff == kOOB || (KMASK && k0 >= a.d) ? kOOB : 2u * rowoff + (uint32_t)(k0 * 4);
+        qv[j] = f32_to_f16x8(ld16(rq, o), ld16(rq, o + 16u));
+        if (has_partial && t == tp) qv[j] &= pmask;
+      } else if constexpr (KMASK) {
         qv[j] = ld16(rq, k0 < a.d ? rowoff + (uint32_t)(k0 * 2) : kOOB);
         if (has_partial && t == tp) qv[j] &= pmask;
       } else {
@@ -1058,6 +1063,33 @@ hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// fp32 docs and query read as they are and rounded in registers: 4 bytes a value
+// where a cast before the scan moves 8, padding included (32 tokens over 5000
+// docs of 300 x 128 249 -> 133 us, 5.8 TB/s, of ragged lengths 231 -> 72; 3000 of
+// 300 x 100 236 -> 62; 100 of 300 x 128 22.7 -> 7.6). One query of up to 32 tokens,
+// d <= 128, no argmax (fmx_fwd_reads_f32); docs of up to 128 tokens in pairs with
+// a two-tile ring, as the 2-byte ones.
+template <int NQB, int KS, bool KMASK>
+hipError_t launch_f32(const FwdArgs& a, hipStream_t s) {
+  if (a.Ld <= 128 && !a.qidx) {
+    hipLaunchKernelGGL((stream_fwd_kernel<KIND_F32, NQB, KS, KMASK, false, true, 2, false, 2>),
+                       dim3((unsigned)((a.B + 1) / 2)), dim3(256), 0, s, a);
+  } else {
+    hipLaunchKernelGGL((stream_fwd_kernel<KIND_F32, NQB, KS, KMASK, false, true>), dim3((unsigned)a.B), dim3(256), 0, s, a);
+  }
+  return hipGetLastError();
+}
+
+template <int NQB>
+hipError_t dispatch_f32(const FwdArgs& a, hipStream_t s) {
+  switch (stream_fwd_ks(a.d)) {
+    case 1: return a.d == 32 ? launch_f32<NQB, 1, false>(a, s) : launch_f32<NQB, 1, true>(a, s);
+    case 2: return a.d == 64 ? launch_f32<NQB, 2, false>(a, s) : launch_f32<NQB, 2, true>(a, s);
+    case 4: return a.d == 128 ? launch_f32<NQB, 4, false>(a, s) : launch_f32<NQB, 4, true>(a, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 template <int KIND, int NQB, int KS>
 hipError_t dispatch_flags(const FwdArgs& a, bool am, hipStream_t s) {
   if constexpr (KIND == KIND_U8) {
@@ -1140,6 +1172,7 @@ hipError_t launch_stream_fwd(int kind, const FwdArgs& a, bool with_argmax, hipSt
     case KIND_F16: return dispatch_ks<KIND_F16>(a, with_argmax, s);
     case KIND_BF16: return dispatch_ks<KIND_BF16>(a, with_argmax, s);
     case KIND_U8: return dispatch_ks<KIND_U8>(a, false, s);
+    case KIND_F32: return a.Lq <= 16 ? dispatch_f32<1>(a, s) : dispatch_f32<2>(a, s);
     default: return hipErrorInvalidValue;
   }
 }

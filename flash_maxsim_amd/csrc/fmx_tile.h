@@ -7,7 +7,7 @@
 // k >= d, come back as zeros from the buffer range check.
 //
 // Fragment slot t of lane group g covers k = frag_k0(t, g) .. +7:
-//  * fp16/bf16: 32t + 8g, one 16-byte load per slot;
+//  * fp16/bf16: 32t + 8g, one 16-byte load per slot (fp32: two);
 //  * uint8: slots are paired, 64*(t/2) + 16g + 8*(t%2), so one 16-byte load of
 //    16 codes feeds slots t and t+1 and a wave's load instruction covers 64
 //    contiguous bytes of each of 16 rows (KS is even for uint8 docs).
@@ -46,7 +46,7 @@ template <int KIND, int KS>
 struct Tile {
   static constexpr bool kU8 = KIND == KIND_U8;
   static_assert(!kU8 || KS % 2 == 0, "uint8 tiles pair their k-steps");
-  u32x4_t v[kU8 ? KS / 2 : KS];
+  u32x4_t v[kU8 ? KS / 2 : KIND == KIND_F32 ? 2 * KS : KS];
   u32x2_t s, m;  // uint8 docs only: fp16 bits of 4 consecutive tokens
 };
 
@@ -157,6 +157,12 @@ __device__ __forceinline__ void load_tile(Tile<KIND, KS>& T, const DocRes& r, in
         T.v[h] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
       }
     }
+  } else if constexpr (KIND == KIND_F32) {
+#pragma unroll
+    for (int t = 0; t < KS; ++t) {
+      T.v[2 * t] = ld16(r.d, base + koff[t]);
+      T.v[2 * t + 1] = ld16(r.d, base + koff[t] + 16u);
+    }
   } else {
 #pragma unroll
     for (int t = 0; t < KS; ++t) T.v[t] = ld16(r.d, base + koff[t]);
@@ -198,6 +204,8 @@ __device__ __forceinline__ u32x4_t tile_operand(const Tile<KIND, KS>& T, int t) 
   if constexpr (KIND == KIND_U8) {
     const u32x4_t w = T.v[t >> 1];
     return codes_to_f16_biased((t & 1) ? u32x2_t{w[2], w[3]} : u32x2_t{w[0], w[1]});
+  } else if constexpr (KIND == KIND_F32) {
+    return f32_to_f16x8(T.v[2 * t], T.v[2 * t + 1]);
   } else {
     return T.v[t];
   }

@@ -42,12 +42,13 @@ const Tensor* plain(PyObject* o) {
 }
 
 // Operand rows that the kernels read in place: unit inner stride, rows at
-// least d apart, every other stride a multiple of 8, 16-byte aligned.
+// least d apart, every other stride a multiple of 8 (fp32: 4), 16-byte aligned.
 bool rows_ready(const Tensor& t) {
   const int64_t n = t.dim();
   if (n < 2 || t.stride(n - 1) != 1 || t.stride(n - 2) < t.size(n - 1)) return false;
+  const int64_t m = t.scalar_type() == at::kFloat ? 3 : 7;
   for (int64_t i = 0; i + 1 < n; ++i)
-    if (t.stride(i) & 7) return false;
+    if (t.stride(i) & m) return false;
   return (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) == 0;
 }
 
@@ -66,6 +67,13 @@ int kernel_dtype(const Tensor& Q, const Tensor& D) {
   const int q = code_of(Q), x = code_of(D);
   if (q < 0 || x < 0) return -1;
   return q == FMX_DTYPE_BF16 && x == FMX_DTYPE_BF16 ? FMX_DTYPE_BF16 : FMX_DTYPE_F16;
+}
+
+// The same for one query of Lq tokens (or Lq tokens a doc): float32 operands that the kernels read in place stay so.
+int scoring_dtype(const Tensor& Q, const Tensor& D, int64_t Lq, int64_t d) {
+  if (code_of(Q) == FMX_DTYPE_F32 && code_of(D) == FMX_DTYPE_F32 && fmx_fwd_reads_f32(Lq, d) && rows_ready(Q) && rows_ready(D))
+    return FMX_DTYPE_F32;
+  return kernel_dtype(Q, D);
 }
 
 // Whether `ready` can make t an operand.
@@ -154,7 +162,7 @@ PyObject* score(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Tensor *Q = plain(args[0]), *D = plain(args[1]);
   FMX_ORDINARY(Q && D && Q->dim() == 2 && D->dim() == 3 && Q->size(1) == D->size(2));
   const int64_t Lq = Q->size(0), d = Q->size(1), B = D->size(0), Ld = D->size(1);
-  const int dtype = kernel_dtype(*Q, *D);
+  const int dtype = scoring_dtype(*Q, *D, Lq, d);
   const int32_t* lengths;
   FMX_ORDINARY(dtype >= 0 && B > 0 && Lq > 0 && convertible(*Q) && convertible(*D) && Q->device() == D->device() &&
                take_lengths(args[2], B, *D, &lengths) && here(*Q));
@@ -207,7 +215,7 @@ PyObject* sparse(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Tensor *Q = plain(args[0]), *D = plain(args[1]), *idx = plain(args[2]);
   FMX_ORDINARY(Q && D && idx && Q->dim() == 2 && D->dim() == 3 && idx->dim() == 2 && Q->size(1) == D->size(2));
   const int64_t Lq = Q->size(0), d = Q->size(1), B = D->size(0), Ld = D->size(1), K = idx->size(1);
-  const int dtype = kernel_dtype(*Q, *D);
+  const int dtype = scoring_dtype(*Q, *D, K, d);
   const int32_t* lengths;
   FMX_ORDINARY(dtype >= 0 && B > 0 && Lq > 0 && K > 0 && idx->size(0) == B && is_row_of(idx, at::kInt, B * K));
   FMX_ORDINARY(convertible(*Q) && convertible(*D) && Q->device() == D->device() && idx->device() == D->device() &&
@@ -239,7 +247,7 @@ PyObject* topk(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   }
   const int64_t Lq = Q->size(0), d = Q->size(1), B = D->size(0), Ld = D->size(1);
-  const int dtype = kernel_dtype(*Q, *D);
+  const int dtype = scoring_dtype(*Q, *D, Lq, d);
   const int32_t* lengths;
   FMX_ORDINARY(dtype >= 0 && Lq > 0 && k > 0 && k <= B && convertible(*Q) && convertible(*D) &&
                Q->device() == D->device() && take_lengths(args[3], B, *D, &lengths) && here(*Q));
@@ -309,7 +317,7 @@ PyObject* packed(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t Lq = Q->size(0), d = Q->size(1), T = D->size(0);
   const long max_len = PyLong_AsLong(args[4]);
   if (max_len == -1 && PyErr_Occurred()) return nullptr;
-  const int dtype = kernel_dtype(*Q, *D);
+  const int dtype = scoring_dtype(*Q, *D, Lq, d);
   int64_t B;
   const int64_t* group;
   const int32_t *lengths, *ids;

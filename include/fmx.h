@@ -40,7 +40,7 @@ extern "C" {
 
 #define FMX_DTYPE_F16 0
 #define FMX_DTYPE_BF16 1
-#define FMX_DTYPE_F32 2 /* sources of fmx_quantize_int8 and fmx_convert_rows only */
+#define FMX_DTYPE_F32 2 /* fmx_quantize_int8 and fmx_convert_rows sources; forwards: fmx_fwd_reads_f32 */
 
 /* Widest d. Up to 4096 the forward kernels hold each query slice in
  * registers; wider rows (which the reference reaches by padding d to a power
@@ -80,6 +80,15 @@ int fmx_fwd(int dtype, const void* Q, int64_t q_stride_n, int64_t q_stride_l, co
             size_t workspace_bytes, void* stream);
 
 size_t fmx_fwd_workspace_bytes(int64_t Nq, int64_t B, int64_t Lq, int64_t Ld, int64_t d);
+
+/*
+ * Whether fmx_fwd (one query, no argmax), fmx_fwd_packed, fmx_fwd_topk and
+ * fmx_fwd_sparse (Lq: its K) also take FMX_DTYPE_F32 at these sizes: Q and D
+ * both fp32, strides multiples of 4 elements, each value rounded to fp16 as it
+ * is read (the scores of operands cast to fp16 beforehand). Elsewhere they
+ * return FMX_ERR_UNSUPPORTED for it.
+ */
+int fmx_fwd_reads_f32(int64_t Lq, int64_t d);
 
 /*
  * fmx_fwd for callers that cannot allocate: code under HIP graph capture,

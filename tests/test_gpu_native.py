@@ -236,3 +236,38 @@ def test_native_launches_on_the_current_stream():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, fm.flash_maxsim(Q, D))
+
+
+@pytest.mark.parametrize("Lq, B, Ld, d", [(1, 1, 1, 4), (16, 7, 128, 128), (17, 8, 129, 128), (32, 301, 300, 128), (32, 5, 77, 100),
+                                          (9, 30, 16, 32), (32, 11, 17, 36), (30, 6, 131, 64), (32, 4, 200, 68), (5, 9, 40, 124)])
+def test_float32_operands_read_in_place(Lq, B, Ld, d):
+    """fp32 docs and query rounded as they are read: the bits of the same call on
+    operands cast to fp16, for overflow, subnormals, NaN in and past d, views of
+    wider rows, ragged and empty docs, packed and sparse."""
+    gen = torch.Generator(device=DEV).manual_seed(3100 + d + Ld)
+    store = torch.full((B, Ld, d + 4), float("nan"), device=DEV)
+    store[..., :d] = torch.randn(B, Ld, d, generator=gen, device=DEV)
+    D = store[..., :d]
+    D[0, 0, : d // 2] *= 2.0**-16
+    D[B // 2, Ld // 2, 0] = 70000.0
+    D[B - 1, Ld - 1, d - 1] = float("nan")
+    Q = torch.randn(Lq, d, generator=gen, device=DEV)
+    ln = torch.randint(0, Ld + 1, (B,), generator=gen, device=DEV, dtype=torch.int32)
+    idx = torch.randint(-1, Lq + 1, (B, min(Lq, 13)), generator=gen, device=DEV, dtype=torch.int32)
+
+    def bits(t):
+        return t.nan_to_num(7e30).view(torch.int32)  # NaN's payload may differ
+
+    for x in (D, D.contiguous()):
+        assert _lib.load().fmx_fwd_reads_f32(Lq, d)
+        for le in (None, ln):
+            assert torch.equal(bits(fm.flash_maxsim(Q, x, le)), bits(fm.flash_maxsim(Q.half(), x.half(), le)))
+            assert torch.equal(bits(fm.flash_maxsim_sparse(Q, x, idx, le)), bits(fm.flash_maxsim_sparse(Q.half(), x.half(), idx, le)))
+        docs = fm.pack_docs(x, ln, True)
+        half = docs._replace(tokens=docs.tokens.half())
+        assert torch.equal(bits(fm.flash_maxsim_packed(Q, docs)), bits(fm.flash_maxsim_packed(Q.half(), half)))
+        v, i = fm.flash_maxsim_topk(Q, x, B, ln)
+        w, j = fm.flash_maxsim_topk(Q.half(), x.half(), B, ln)
+        assert torch.equal(bits(v), bits(w)) and torch.equal(i, j)
+    lib = _lib.load()
+    assert not lib.fmx_fwd_reads_f32(33, d) and not lib.fmx_fwd_reads_f32(Lq, 129)
