@@ -92,7 +92,7 @@ _SIGNATURES = {
         [_ptr, _i64, _i64, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _i64, _i64, _ptr, _ptr,
          _i64, _i64, _i64, _i64, _i64, _ptr, _size, _ptr],
     ),
-    "fmx_convert_rows": (_int, [_int, _ptr, _i64, _i64, _i64, _i64, _i64, _int, _ptr, _i64, _ptr]),
+    "fmx_convert_rows": (_int, [_int, _ptr, _i64, _i64, _i64, _i64, _i64, _ptr, _int, _ptr, _i64, _ptr]),
     "fmx_bwd_batched_workspace_bytes": (_size, [_i64, _i64, _i64, _i64, _i64]),
 }
 

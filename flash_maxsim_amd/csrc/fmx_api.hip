@@ -725,7 +725,7 @@ int fmx_bwd_batched_f32(const void* Q, int64_t q_stride_n, int64_t q_stride_l, c
 }
 
 int fmx_convert_rows(int src_dtype, const void* src, int64_t s_stride_b, int64_t s_stride_l, int64_t B, int64_t Ld,
-                     int64_t d, int dst_dtype, void* dst, int64_t dp, void* stream) {
+                     int64_t d, const int32_t* lengths, int dst_dtype, void* dst, int64_t dp, void* stream) {
   if (B < 0 || Ld < 0 || d < 1 || dp < d || (dp & 7) || s_stride_b < 0 || s_stride_l < 0)
     return fail(FMX_ERR_INVALID, "invalid sizes B=%lld Ld=%lld d=%lld dp=%lld", (long long)B, (long long)Ld, (long long)d,
                 (long long)dp);
@@ -737,7 +737,7 @@ int fmx_convert_rows(int src_dtype, const void* src, int64_t s_stride_b, int64_t
   if (!aligned16(dst)) return fail(FMX_ERR_INVALID, "dst must be 16-byte aligned");
   if (reinterpret_cast<uintptr_t>(src) & (src_dtype == FMX_DTYPE_F32 ? 3u : 1u))
     return fail(FMX_ERR_INVALID, "src must be aligned to its element");
-  if (dp > INT32_MAX || Ld > INT32_MAX / (dp / 8)) return fail(FMX_ERR_UNSUPPORTED, "doc of %lld x %lld elements", (long long)Ld, (long long)dp);
+  if (dp > INT32_MAX || Ld > (INT32_MAX - 4096) / (dp / 4)) return fail(FMX_ERR_UNSUPPORTED, "doc of %lld x %lld elements", (long long)Ld, (long long)dp);
   fmx::ConvertArgs a = {};
   a.src = src;
   a.s_stride_b = s_stride_b;
@@ -746,6 +746,7 @@ int fmx_convert_rows(int src_dtype, const void* src, int64_t s_stride_b, int64_t
   a.Ld = Ld;
   a.d = d;
   a.dp = dp;
+  a.lengths = lengths;
   a.f32 = src_dtype == FMX_DTYPE_F32;
   a.bf16 = src_dtype == FMX_DTYPE_BF16 && dst_dtype == FMX_DTYPE_F16;
   a.dst = dst;

@@ -139,6 +139,7 @@ struct ConvertArgs {
   int64_t B, Ld, d, dp;
   int f32;                    // fp32 source, else 2-byte elements
   int bf16;                   // 2-byte source: bf16 to be cast to fp16
+  const int32_t* lengths;     // [B] rows to convert of each doc, or null (= Ld); the others are left as they are
   void* dst;
 };
 hipError_t launch_convert(const ConvertArgs& a, hipStream_t s);

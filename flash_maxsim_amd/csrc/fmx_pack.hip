@@ -148,76 +148,104 @@ hipError_t launch_pack_units(const PackArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Eight elements of an operand row per thread: read 4, 8 or 2 bytes at a time as
-// the source's alignment allows, cast to fp16 (round to nearest even, as
-// torch's cast) or kept, and written as one 16-byte store. One pass where torch
-// casts, then pads (training step of 32 x 32 tokens over 256 fp32 docs of up to
-// 180 x 128 105 -> 86 us with the gradients written in fp32).
-// SRC: 0 fp16 or any 2-byte type kept, 1 bf16, 2 fp32. A: aligned elements a
-// load may take (1, 2, 4).
-template <int SRC, int A>
-__global__ void __launch_bounds__(256) convert_kernel(const void* src, int64_t sb, int64_t sl, uint32_t Ld, uint32_t d,
-                                                      uint32_t cpr, uint32_t rows_per_b, int64_t n, u32x4_t* dst) {
-  // a grid row per doc: chunk x of the doc's Ld * cpr
-  const uint32_t x = blockIdx.x * 256 + threadIdx.x;
-  if (x >= rows_per_b) return;
-  const uint32_t j = x / cpr, k0 = (x - j * cpr) * 8;
-  for (int64_t b = blockIdx.y; b < n; b += gridDim.y) {
-    const int64_t e0 = b * sb + (int64_t)j * sl + k0;
-    u32x4_t o;
-    if constexpr (SRC == 2) {
-      const float* p = static_cast<const float*>(src) + e0;
-      float v[8];
-#pragma unroll
-      for (int i = 0; i < 8; i += A) {
-        if constexpr (A == 4) {
-          const f32x4_t q = k0 + i < d ? *reinterpret_cast<const f32x4_t*>(p + i) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[i + e] = q[e];
-        } else {
-          v[i] = k0 + i < d ? p[i] : 0.f;
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        o[i] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v[2 * i]) |
-               ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v[2 * i + 1]) << 16);
-    } else {
-      const uint16_t* p = static_cast<const uint16_t*>(src) + e0;
-      uint32_t w[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if constexpr (A >= 2) {
-          w[i] = k0 + 2 * i < d ? *reinterpret_cast<const uint32_t*>(p + 2 * i) : 0u;
-        } else {
-          w[i] = k0 + 2 * i < d ? p[2 * i] : 0u;
-          w[i] |= k0 + 2 * i + 1 < d ? (uint32_t)p[2 * i + 1] << 16 : 0u;
-        }
-        if constexpr (SRC == 1) {
-          const uint16_t lo = __builtin_bit_cast(uint16_t, (_Float16)bf16_bits_to_float(w[i] & 0xffffu));
-          const uint16_t hi = __builtin_bit_cast(uint16_t, (_Float16)bf16_bits_to_float(w[i] >> 16));
-          w[i] = (uint32_t)lo | ((uint32_t)hi << 16);
-        }
-      }
-      o = u32x4_t{w[0], w[1], w[2], w[3]};
+// Operand rows cast to fp16 (round to nearest even, as torch's cast) or kept, and
+// padded with zeros to a multiple of 8 elements, in one pass where torch casts,
+// then pads (training step of 32 x 32 tokens over 256 fp32 docs of up to 180 x
+// 128 105 -> 86 us with the gradients written in fp32); rows past a doc's length
+// are left out, as nothing reads them. A thread takes kConvIter groups of four
+// elements, each load and store of a wave contiguous (eight elements a thread
+// left every fp32 load at a 32-byte stride: 8872 docs of 297 x 128 under 206
+// tokens 515 -> 499 us). NT: non-temporal loads, for sources the last-level cache
+// would not hold (there 507 -> 500; 500 docs of 100 x 128, 18.6 -> 21.9, keep the
+// default).
+// SRC: 0 fp16 or any 2-byte type kept, 1 bf16, 2 fp32. WIDE: groups are aligned
+// and do not straddle d, one load each.
+constexpr int kConvIter = 4;
+
+template <int SRC, bool WIDE, bool NT>
+__global__ void __launch_bounds__(256) convert_kernel(const void* src, int64_t sb, int64_t sl, int32_t Ld, uint32_t d,
+                                                      uint32_t gpr, int64_t B, const int32_t* lengths, u32x2_t* dst) {
+  const uint32_t x0 = blockIdx.x * (256 * kConvIter) + threadIdx.x;  // groups of a doc
+  for (int64_t b = blockIdx.y; b < B; b += gridDim.y) {
+    int32_t len = Ld;
+    if (lengths) {
+      len = ld_uniform(lengths + b);
+      len = len < 0 ? 0 : (len > Ld ? Ld : len);
     }
-    dst[b * rows_per_b + x] = o;
+    const uint32_t n = (uint32_t)len * gpr;
+    if (x0 - threadIdx.x >= n) continue;  // uniform
+    u32x4_t v[kConvIter];  // 2-byte sources: two words
+#pragma unroll
+    for (int k = 0; k < kConvIter; ++k) {
+      // Groups past the doc repeat its last one and groups past d the row's: the
+      // loads are unconditional, so all are in flight together.
+      const uint32_t x = x0 + k * 256 < n ? x0 + k * 256 : n - 1, j = x / gpr, k0 = (x - j * gpr) * 4;
+      const int64_t row = b * sb + (int64_t)j * sl;
+      if constexpr (WIDE) {
+        const bool pad = k0 >= d;
+        const int64_t e0 = row + (pad ? d - 4 : k0);
+        if constexpr (SRC == 2) {
+          const u32x4_t* p = reinterpret_cast<const u32x4_t*>(static_cast<const uint32_t*>(src) + e0);
+          v[k] = NT ? __builtin_nontemporal_load(p) : *p;
+        } else {
+          const u32x2_t* p = reinterpret_cast<const u32x2_t*>(static_cast<const uint16_t*>(src) + e0);
+          const u32x2_t w = NT ? __builtin_nontemporal_load(p) : *p;
+          v[k] = u32x4_t{w[0], w[1], 0u, 0u};
+        }
+        if (pad) v[k] = u32x4_t{0u, 0u, 0u, 0u};
+      } else {
+        v[k] = u32x4_t{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (SRC == 2) {
+            v[k][e] = k0 + e < d ? static_cast<const uint32_t*>(src)[row + k0 + e] : 0u;
+          } else {
+            v[k][e >> 1] |= k0 + e < d ? (uint32_t)static_cast<const uint16_t*>(src)[row + k0 + e] << (16 * (e & 1)) : 0u;
+          }
+        }
+      }
+    }
+    auto half = [](float f) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)f); };
+#pragma unroll
+    for (int k = 0; k < kConvIter; ++k) {
+      const uint32_t x = x0 + k * 256;
+      if (x >= n) continue;
+      u32x2_t o;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if constexpr (SRC == 2) {
+          // (copies: a vector subscript inside a bit cast takes the first element)
+          const uint32_t lo = v[k][2 * i], hi = v[k][2 * i + 1];
+          o[i] = half(__builtin_bit_cast(float, lo)) | (half(__builtin_bit_cast(float, hi)) << 16);
+        } else if constexpr (SRC == 1) {
+          o[i] = half(bf16_bits_to_float(v[k][i] & 0xffffu)) | (half(bf16_bits_to_float(v[k][i] >> 16)) << 16);
+        } else {
+          o[i] = v[k][i];
+        }
+      }
+      dst[b * ((int64_t)Ld * gpr) + x] = o;
+    }
   }
 }
 
 template <int SRC>
-hipError_t launch_convert_src(const ConvertArgs& a, hipStream_t s) {
-  const int esz = SRC == 2 ? 4 : 2;
-  const int64_t cpr = a.dp / 8, per_b = a.Ld * cpr;
-  if (per_b > INT32_MAX) return hipErrorInvalidValue;
-  // elements that every load's place is a multiple of, and that do not run past d
-  const uint64_t bits = reinterpret_cast<uintptr_t>(a.src) / esz | (uint64_t)a.s_stride_b | (uint64_t)a.s_stride_l | (uint64_t)a.d;
-  const int64_t gy = a.B < 65535 ? a.B : 65535;
-  auto kern = SRC == 2 ? ((bits & 3) == 0 ? convert_kernel<SRC, 4> : convert_kernel<SRC, 1>)
-                       : ((bits & 1) == 0 ? convert_kernel<SRC, 2> : convert_kernel<SRC, 1>);
-  hipLaunchKernelGGL(kern, dim3((unsigned)((per_b + 255) / 256), (unsigned)gy), dim3(256), 0, s, a.src, a.s_stride_b,
-                     a.s_stride_l, (uint32_t)a.Ld, (uint32_t)a.d, (uint32_t)cpr, (uint32_t)per_b, a.B,
-                     static_cast<u32x4_t*>(a.dst));
+hipError_t launch_convert_src(ConvertArgs a, hipStream_t s) {
+  constexpr int esz = SRC == 2 ? 4 : 2;
+  const int64_t gpr = a.dp / 4;
+  if (a.Ld * gpr > INT32_MAX - 4096) return hipErrorInvalidValue;
+  const bool nt = a.B * a.Ld * a.d * esz >= ((int64_t)1 << 28);
+  // docs back to back, all rows of them: one doc, without a part-filled workgroup each
+  if (!a.lengths && a.s_stride_b == a.Ld * a.s_stride_l && a.B * a.Ld <= (INT32_MAX - 4096) / gpr) {
+    a.Ld *= a.B;
+    a.B = 1;
+  }
+  const uint64_t bits = reinterpret_cast<uintptr_t>(a.src) / esz | (uint64_t)a.s_stride_b | (uint64_t)a.s_stride_l |
+                        (uint64_t)a.d;
+  const int64_t gy = a.B < 65535 ? a.B : 65535, gx = (a.Ld * gpr + 256 * kConvIter - 1) / (256 * kConvIter);
+  auto kern = (bits & 3) == 0 ? (nt ? convert_kernel<SRC, true, true> : convert_kernel<SRC, true, false>)
+                              : convert_kernel<SRC, false, false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, a.src, a.s_stride_b, a.s_stride_l,
+                     (int32_t)a.Ld, (uint32_t)a.d, (uint32_t)gpr, a.B, a.lengths, static_cast<u32x2_t*>(a.dst));
   return hipGetLastError();
 }
 

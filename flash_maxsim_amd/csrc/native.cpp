@@ -79,7 +79,7 @@ int scoring_dtype(const Tensor& Q, const Tensor& D, int64_t Lq, int64_t d) {
 // Whether `ready` can make t an operand.
 bool convertible(const Tensor& t) {
   const int64_t n = t.dim(), d = t.size(n - 1);
-  return (n == 2 || n == 3) && t.stride(n - 1) == 1 && d >= 1 && t.numel() > 0 && t.size(n - 2) <= INT32_MAX / (d / 8 + 1);
+  return (n == 2 || n == 3) && t.stride(n - 1) == 1 && d >= 1 && t.numel() > 0 && t.size(n - 2) <= (INT32_MAX - 4096) / (2 * (d / 8 + 1));
 }
 
 bool is_row_of(const Tensor* t, at::ScalarType type, int64_t n) {
@@ -105,24 +105,25 @@ bool here(const Tensor& t) {
 void* stream_of(const Tensor& t);
 
 // t as the kernels read it in type `dtype`: itself, or a converted copy with its
-// rows padded to a multiple of 8 elements. Undefined, with *rc set: the conversion failed.
-Tensor ready(const Tensor& t, int dtype, int* rc) {
+// rows padded to a multiple of 8 elements (of documents, the rows within `lengths`,
+// where given: nothing reads the others). Undefined, with *rc set: the conversion failed.
+Tensor ready(const Tensor& t, int dtype, const int32_t* lengths, int* rc) {
   if (code_of(t) == dtype && rows_ready(t)) return t;
   const int64_t n = t.dim(), d = t.size(n - 1), dp = (d + 7) / 8 * 8, rows = t.size(n - 2);
   auto sizes = t.sizes().vec();
   sizes[n - 1] = dp;
   Tensor out = at::empty(sizes, t.options().dtype(dtype == FMX_DTYPE_BF16 ? at::kBFloat16 : at::kHalf));
   *rc = fmx_convert_rows(code_of(t), t.const_data_ptr(), n == 3 ? t.stride(0) : 0, t.stride(n - 2),
-                         n == 3 ? t.size(0) : 1, rows, d, dtype, out.data_ptr(), dp, stream_of(t));
+                         n == 3 ? t.size(0) : 1, rows, d, lengths, dtype, out.data_ptr(), dp, stream_of(t));
   return *rc ? Tensor() : out;
 }
 
 // Q and D as operands, in place of their originals.
-#define FMX_READY(Q, D)                                \
+#define FMX_READY(Q, D, lengths)                       \
   int prc = 0;                                         \
-  const Tensor Qk = ready(*Q, dtype, &prc);            \
+  const Tensor Qk = ready(*Q, dtype, nullptr, &prc);   \
   if (prc) return failed(prc);                         \
-  const Tensor Dk = ready(*D, dtype, &prc);            \
+  const Tensor Dk = ready(*D, dtype, lengths, &prc);   \
   if (prc) return failed(prc)
 
 PyObject* failed(int rc);
@@ -169,7 +170,7 @@ PyObject* score(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Tensor out = at::empty({B}, D->options().dtype(at::kFloat));
   const size_t n = fmx_fwd_workspace_bytes(1, B, Lq, Ld, d);
   const Tensor ws = scratch(n, *D);
-  FMX_READY(Q, D);
+  FMX_READY(Q, D, lengths);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
     return fmx_fwd(dtype, Qk.const_data_ptr(), 0, Qk.stride(0), Dk.const_data_ptr(), Dk.stride(0), Dk.stride(1),
@@ -197,7 +198,7 @@ PyObject* batched(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Tensor out = at::empty({Nq, B}, D->options().dtype(at::kFloat));
   const size_t n = fmx_fwd_workspace_bytes(Nq, B, Lq, Ld, d);
   const Tensor ws = scratch(n, *D);
-  FMX_READY(Q, D);
+  FMX_READY(Q, D, lengths);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
     return fmx_fwd(dtype, Qk.const_data_ptr(), Qk.stride(0), Qk.stride(1), Dk.const_data_ptr(), Dk.stride(k),
@@ -223,7 +224,7 @@ PyObject* sparse(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Tensor out = at::empty({B}, D->options().dtype(at::kFloat));
   const size_t n = fmx_fwd_sparse_workspace_bytes(B, K, Ld, d);
   const Tensor ws = scratch(n, *D);
-  FMX_READY(Q, D);
+  FMX_READY(Q, D, lengths);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
     return fmx_fwd_sparse(dtype, Qk.const_data_ptr(), Qk.stride(0), Lq, Dk.const_data_ptr(), Dk.stride(0), Dk.stride(1),
@@ -256,7 +257,7 @@ PyObject* topk(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Tensor values = at::empty({k}, f32), indices = at::empty({k}, D->options().dtype(at::kLong));
   const size_t n = fmx_fwd_topk_workspace_bytes(B, Lq, Ld, d, k);
   const Tensor ws = scratch(n, *D);
-  FMX_READY(Q, D);
+  FMX_READY(Q, D, lengths);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
     return fmx_fwd_topk(dtype, Qk.const_data_ptr(), Qk.stride(0), Dk.const_data_ptr(), Dk.stride(0), Dk.stride(1),
@@ -328,7 +329,7 @@ PyObject* packed(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Tensor out = at::empty({B}, D->options().dtype(at::kFloat));
   const size_t n = fmx_fwd_packed_workspace_bytes(B, Lq, Ld, d);
   const Tensor ws = scratch(n, *D);
-  FMX_READY(Q, D);
+  FMX_READY(Q, D, nullptr);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
     return fmx_fwd_packed(dtype, Qk.const_data_ptr(), Qk.stride(0), Lq, Dk.const_data_ptr(), Dk.stride(0), T, group,
@@ -386,7 +387,7 @@ PyObject* forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Tensor argmax = at::empty({Nq * B, Lq}, D->options().dtype(at::kInt));
   const size_t n = fmx_fwd_workspace_bytes(Nq, B, Lq, Ld, d);
   const Tensor ws = scratch(n, *D);
-  FMX_READY(Q, D);
+  FMX_READY(Q, D, lengths);
   void* s = stream_of(*Q);
   const int rc = unlocked([&] {
     return fmx_fwd(dtype, Qk.const_data_ptr(), Qk.stride(0), Qk.stride(1), Dk.const_data_ptr(), Dk.stride(0),

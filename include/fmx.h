@@ -366,12 +366,13 @@ int fmx_bwd_batched_f32(const void* Q, int64_t q_stride_n, int64_t q_stride_l, c
  * Operand rows made ready for the other entry points in one pass: rows of d
  * elements, [B, Ld] of them at strides s_stride_b and s_stride_l, to contiguous
  * rows of dp elements (a multiple of 8, dp >= d) in dst (16-byte aligned), zeros
- * past d. FMX_DTYPE_F32 and FMX_DTYPE_BF16 to FMX_DTYPE_F16 round to nearest
+ * past d. Of doc b the first lengths[b] rows (int32, clamped to [0, Ld]; NULL:
+ * all), the others are not written. FMX_DTYPE_F32 and FMX_DTYPE_BF16 to FMX_DTYPE_F16 round to nearest
  * even; FMX_DTYPE_F16 and FMX_DTYPE_BF16 to themselves are moved. (The
  * reference casts and copies with torch, flash_maxsim/flash_maxsim.py:226-227.)
  */
 int fmx_convert_rows(int src_dtype, const void* src, int64_t s_stride_b, int64_t s_stride_l, int64_t B, int64_t Ld,
-                     int64_t d, int dst_dtype, void* dst, int64_t dp, void* stream);
+                     int64_t d, const int32_t* lengths, int dst_dtype, void* dst, int64_t dp, void* stream);
 
 /* Workspace of fmx_bwd_batched: as fmx_bwd_workspace_bytes with Nq*Lq entries per doc. */
 size_t fmx_bwd_batched_workspace_bytes(int64_t Nq, int64_t B, int64_t Lq, int64_t Ld, int64_t d);

@@ -174,12 +174,18 @@ def test_convert_rows_bitwise_torch(d, kinds):
     for lead in (0, 1, 3):
         for v in (x[..., lead : lead + d], x[..., lead : lead + d].contiguous(), x[:1, :, lead : lead + d].expand(3, 21, d)):
             out = torch.full((3, 21, dp), 7.0, dtype=dst_t, device=DEV)
-            _lib.check(_lib.load().fmx_convert_rows(src_c, v.data_ptr(), v.stride(0), v.stride(1), 3, 21, d, dst_c,
+            _lib.check(_lib.load().fmx_convert_rows(src_c, v.data_ptr(), v.stride(0), v.stride(1), 3, 21, d, None, dst_c,
                                                     out.data_ptr(), dp, torch.cuda.current_stream().cuda_stream))
             want = torch.nn.functional.pad(v.to(dst_t), (0, dp - d))
             nan = torch.isnan(want)
             assert torch.equal(torch.isnan(out), nan)
             assert torch.equal(out.masked_fill(nan, 0).view(torch.int16), want.masked_fill(nan, 0).view(torch.int16))
+            ln = torch.tensor([4, -1, 30], dtype=torch.int32, device=DEV)
+            part = torch.full_like(out, 7.0)
+            _lib.check(_lib.load().fmx_convert_rows(src_c, v.data_ptr(), v.stride(0), v.stride(1), 3, 21, d, ln.data_ptr(),
+                                                    dst_c, part.data_ptr(), dp, torch.cuda.current_stream().cuda_stream))
+            out[0, 4:], out[1] = 7.0, 7.0
+            assert torch.equal(part.view(torch.int16), out.view(torch.int16))
 
 
 @pytest.mark.parametrize("Nq, B, Lq, Ld, d", [(1, 40, 20, 33, 128), (3, 12, 50, 30, 100), (1, 6, 300, 9, 30), (9, 5, 40, 17, 520),
