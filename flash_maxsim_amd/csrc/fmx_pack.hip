@@ -157,12 +157,13 @@ hipError_t launch_pack_units(const PackArgs& a, hipStream_t s) {
 // left every fp32 load at a 32-byte stride: 8872 docs of 297 x 128 under 206
 // tokens 515 -> 499 us). NT: non-temporal loads, for sources the last-level cache
 // would not hold (there 507 -> 500; 500 docs of 100 x 128, 18.6 -> 21.9, keep the
-// default).
+// default). NTS: so the stores, for copies that it would not hold (502 -> 484;
+// 2000 docs of 300 x 1024 849 -> 814, of 300 x 128, 154 MB, 101 -> 111).
 // SRC: 0 fp16 or any 2-byte type kept, 1 bf16, 2 fp32. WIDE: groups are aligned
 // and do not straddle d, one load each.
 constexpr int kConvIter = 4;
 
-template <int SRC, bool WIDE, bool NT>
+template <int SRC, bool WIDE, bool NT, bool NTS>
 __global__ void __launch_bounds__(256) convert_kernel(const void* src, int64_t sb, int64_t sl, int32_t Ld, uint32_t d,
                                                       uint32_t gpr, int64_t B, const int32_t* lengths, u32x2_t* dst) {
   const uint32_t x0 = blockIdx.x * (256 * kConvIter) + threadIdx.x;  // groups of a doc
@@ -223,7 +224,12 @@ __global__ void __launch_bounds__(256) convert_kernel(const void* src, int64_t s
           o[i] = v[k][i];
         }
       }
-      dst[b * ((int64_t)Ld * gpr) + x] = o;
+      u32x2_t* p = dst + b * ((int64_t)Ld * gpr) + x;
+      if constexpr (NTS) {
+        __builtin_nontemporal_store(o, p);
+      } else {
+        *p = o;
+      }
     }
   }
 }
@@ -234,6 +240,7 @@ hipError_t launch_convert_src(ConvertArgs a, hipStream_t s) {
   const int64_t gpr = a.dp / 4;
   if (a.Ld * gpr > INT32_MAX - 4096) return hipErrorInvalidValue;
   const bool nt = a.B * a.Ld * a.d * esz >= ((int64_t)1 << 28);
+  const bool nts = nt && a.B * a.Ld * a.dp * 2 >= ((int64_t)1 << 28);
   // docs back to back, all rows of them: one doc, without a part-filled workgroup each
   if (!a.lengths && a.s_stride_b == a.Ld * a.s_stride_l && a.B * a.Ld <= (INT32_MAX - 4096) / gpr) {
     a.Ld *= a.B;
@@ -242,8 +249,11 @@ hipError_t launch_convert_src(ConvertArgs a, hipStream_t s) {
   const uint64_t bits = reinterpret_cast<uintptr_t>(a.src) / esz | (uint64_t)a.s_stride_b | (uint64_t)a.s_stride_l |
                         (uint64_t)a.d;
   const int64_t gy = a.B < 65535 ? a.B : 65535, gx = (a.Ld * gpr + 256 * kConvIter - 1) / (256 * kConvIter);
-  auto kern = (bits & 3) == 0 ? (nt ? convert_kernel<SRC, true, true> : convert_kernel<SRC, true, false>)
-                              : convert_kernel<SRC, false, false>;
+  auto kern = convert_kernel<SRC, false, false, false>;
+  if ((bits & 3) == 0)
+    kern = nts  ? convert_kernel<SRC, true, true, true>
+           : nt ? convert_kernel<SRC, true, true, false>
+                : convert_kernel<SRC, true, false, false>;
   hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, a.src, a.s_stride_b, a.s_stride_l,
                      (int32_t)a.Ld, (uint32_t)a.d, (uint32_t)gpr, a.B, a.lengths, static_cast<u32x2_t*>(a.dst));
   return hipGetLastError();
