@@ -14,9 +14,10 @@ Differences by design:
     doc for lengths > Ld) and must have one entry per doc row;
   * operands are read in place when their row strides are multiple of 8
     elements (d masked in the kernels), so D = store[..., :d] of a store padded
-    to a multiple of 8 costs no copy; other layouts, and contiguous rows with
-    d % 8 != 0, are copied once per call with d zero-padded to a multiple of 8
-    (the kernels read rows with 16-byte loads).
+    to a multiple of 8 costs no copy, and so are float32 docs under one
+    query of up to 32 tokens at d <= 128; other layouts and types, and contiguous
+    rows with d % 8 != 0, are copied once per call with d zero-padded to a multiple
+    of 8 (the kernels read rows with 16-byte loads).
 """
 
 from __future__ import annotations
