@@ -22,6 +22,8 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
+
 #include "../../include/fmx.h"
 
 namespace {
@@ -69,9 +71,19 @@ int kernel_dtype(const Tensor& Q, const Tensor& D) {
   return q == FMX_DTYPE_BF16 && x == FMX_DTYPE_BF16 ? FMX_DTYPE_BF16 : FMX_DTYPE_F16;
 }
 
-// The same for one query of Lq tokens (or Lq tokens a doc): float32 operands that the kernels read in place stay so.
-int scoring_dtype(const Tensor& Q, const Tensor& D, int64_t Lq, int64_t d) {
-  if (code_of(Q) == FMX_DTYPE_F32 && code_of(D) == FMX_DTYPE_F32 && fmx_fwd_reads_f32(Lq, d) && rows_ready(Q) && rows_ready(D))
+// Whether n fp32 rows of t and `slack` more span less than 2 GiB, as the library's
+// checks ask of a query (slack 128) and of a document (16).
+bool f32_in_range(const Tensor& t, int64_t n, int64_t slack) {
+  return t.stride(t.dim() - 2) <= (((int64_t)1 << 29) - 1) / (n + slack);
+}
+
+// The same for one query of Lq tokens (or Lq tokens a doc) over docs of up to Ld:
+// float32 operands that the kernels read in place stay so. Rows too far apart for
+// that (views of token-major storage), or too many of them, are cast like other
+// layouts: the fp16 copy is contiguous and half the size.
+int scoring_dtype(const Tensor& Q, const Tensor& D, int64_t Lq, int64_t Ld, int64_t d) {
+  if (code_of(Q) == FMX_DTYPE_F32 && code_of(D) == FMX_DTYPE_F32 && fmx_fwd_reads_f32(Lq, d) && rows_ready(Q) &&
+      rows_ready(D) && f32_in_range(Q, std::max(Lq, Q.size(0)), 128) && f32_in_range(D, Ld, 16))
     return FMX_DTYPE_F32;
   return kernel_dtype(Q, D);
 }
@@ -163,7 +175,7 @@ PyObject* score(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Tensor *Q = plain(args[0]), *D = plain(args[1]);
   FMX_ORDINARY(Q && D && Q->dim() == 2 && D->dim() == 3 && Q->size(1) == D->size(2));
   const int64_t Lq = Q->size(0), d = Q->size(1), B = D->size(0), Ld = D->size(1);
-  const int dtype = scoring_dtype(*Q, *D, Lq, d);
+  const int dtype = scoring_dtype(*Q, *D, Lq, Ld, d);
   const int32_t* lengths;
   FMX_ORDINARY(dtype >= 0 && B > 0 && Lq > 0 && convertible(*Q) && convertible(*D) && Q->device() == D->device() &&
                take_lengths(args[2], B, *D, &lengths) && here(*Q));
@@ -216,7 +228,7 @@ PyObject* sparse(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Tensor *Q = plain(args[0]), *D = plain(args[1]), *idx = plain(args[2]);
   FMX_ORDINARY(Q && D && idx && Q->dim() == 2 && D->dim() == 3 && idx->dim() == 2 && Q->size(1) == D->size(2));
   const int64_t Lq = Q->size(0), d = Q->size(1), B = D->size(0), Ld = D->size(1), K = idx->size(1);
-  const int dtype = scoring_dtype(*Q, *D, K, d);
+  const int dtype = scoring_dtype(*Q, *D, K, Ld, d);
   const int32_t* lengths;
   FMX_ORDINARY(dtype >= 0 && B > 0 && Lq > 0 && K > 0 && idx->size(0) == B && is_row_of(idx, at::kInt, B * K));
   FMX_ORDINARY(convertible(*Q) && convertible(*D) && Q->device() == D->device() && idx->device() == D->device() &&
@@ -248,7 +260,7 @@ PyObject* topk(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   }
   const int64_t Lq = Q->size(0), d = Q->size(1), B = D->size(0), Ld = D->size(1);
-  const int dtype = scoring_dtype(*Q, *D, Lq, d);
+  const int dtype = scoring_dtype(*Q, *D, Lq, Ld, d);
   const int32_t* lengths;
   FMX_ORDINARY(dtype >= 0 && Lq > 0 && k > 0 && k <= B && convertible(*Q) && convertible(*D) &&
                Q->device() == D->device() && take_lengths(args[3], B, *D, &lengths) && here(*Q));
@@ -318,14 +330,14 @@ PyObject* packed(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t Lq = Q->size(0), d = Q->size(1), T = D->size(0);
   const long max_len = PyLong_AsLong(args[4]);
   if (max_len == -1 && PyErr_Occurred()) return nullptr;
-  const int dtype = scoring_dtype(*Q, *D, Lq, d);
+  const int64_t Ld = max_len > 1 ? max_len : 1;
+  const int dtype = scoring_dtype(*Q, *D, Lq, Ld, d);
   int64_t B;
   const int64_t* group;
   const int32_t *lengths, *ids;
   FMX_ORDINARY(dtype >= 0 && Q->device() == D->device() && convertible(*Q) && convertible(*D) &&
                take_slots(args[2], args[3], args[5], *D, &B, &group, &lengths, &ids) && B > 0 && Lq > 0 && T > 0 &&
                here(*Q));
-  const int64_t Ld = max_len > 1 ? max_len : 1;
   Tensor out = at::empty({B}, D->options().dtype(at::kFloat));
   const size_t n = fmx_fwd_packed_workspace_bytes(B, Lq, Ld, d);
   const Tensor ws = scratch(n, *D);

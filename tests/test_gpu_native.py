@@ -277,3 +277,30 @@ def test_float32_operands_read_in_place(Lq, B, Ld, d):
         assert torch.equal(bits(v), bits(w)) and torch.equal(i, j)
     lib = _lib.load()
     assert not lib.fmx_fwd_reads_f32(33, d) and not lib.fmx_fwd_reads_f32(Lq, 129)
+
+
+def test_float32_rows_too_far_apart_are_cast():
+    """float32 operands whose rows span 2 GiB as they lie (documents and queries in
+    token-major storage): not for the kernels to read in place, so they are cast to
+    a contiguous copy, and score as the same values do from contiguous rows."""
+    B, d = 9, 64
+    gen = torch.Generator(device=DEV).manual_seed(3200)
+    Q, D = torch.randn(5, d, generator=gen, device=DEV), torch.randn(B, 2, d, generator=gen, device=DEV)
+    store = torch.empty(2, (1 << 29) // (18 * d) + 1, d, device=DEV)  # (2 + 16) rows of it are 2 GiB
+    far = store[:, :B].transpose(0, 1)
+    far.copy_(D)
+    assert 18 * far.stride(1) * 4 >= 1 << 31
+    apart = torch.empty(5, (1 << 29) // 133 // 4 * 4 + 4, device=DEV)[:, :d]  # 5 + 128 rows
+    apart.copy_(Q)
+    assert 133 * apart.stride(0) * 4 >= 1 << 31
+    ln = torch.tensor([2, 0, 1, 2, 2, 1, 2, 2, 2], dtype=torch.int32, device=DEV)
+    idx = torch.randint(-1, 6, (B, 3), generator=gen, device=DEV, dtype=torch.int32)
+    docs = fm.pack_docs(D[:2], ln[:2])
+    tokens = torch.empty(len(docs.tokens), (1 << 29) // 18 // 4 * 4 + 4, device=DEV)[:, :d]
+    tokens.copy_(docs.tokens)
+    for q, x in ((Q, far), (apart, D), (apart, far)):
+        for le in (None, ln):
+            assert torch.equal(fm.flash_maxsim(q, x, le), fm.flash_maxsim(Q, D, le))
+            assert same(fm.flash_maxsim_topk(q, x, 4, le), fm.flash_maxsim_topk(Q, D, 4, le))
+            assert torch.equal(fm.flash_maxsim_sparse(q, x, idx, le), fm.flash_maxsim_sparse(Q, D, idx, le))
+    assert torch.equal(fm.flash_maxsim_packed(Q, docs._replace(tokens=tokens)), fm.flash_maxsim_packed(Q, docs))
