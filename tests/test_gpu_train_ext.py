@@ -294,6 +294,41 @@ def test_bwd_index_and_writers_exact(Nq, B, Lq, Ld, d):
     test_bwd_exact_on_integer_grid(Nq, B, Lq, Ld, d)
 
 
+def test_bwd_queries_far_apart():
+    """dD of two queries 2^35 elements apart, past the places that the dense writer
+    keeps in 32 bits, equals dD of the same queries side by side."""
+    from flash_maxsim_amd import _lib
+
+    Nq, B, Lq, Ld, d = 2, 3, 40, 6, 64
+    apart = 1 << 35
+    if torch.cuda.mem_get_info()[0] < 2 * apart + (4 << 30):
+        pytest.skip("needs 68 GiB of free GPU memory")
+    gen = torch.Generator().manual_seed(2200)
+    Q = torch.randn(Nq, Lq, d, generator=gen).to(torch.float16).to(DEV)
+    store = torch.empty(apart + Lq * d, dtype=torch.float16, device=DEV)
+    far = store.as_strided((Nq, Lq, d), (apart, d, 1))
+    far.copy_(Q)
+    D = torch.randn(B, Ld, d, generator=gen).to(torch.float16).to(DEV)
+    am = torch.randint(0, Ld, (Nq * B, Lq), generator=gen, dtype=torch.int32).to(DEV)
+    g = torch.randn(Nq, B, generator=gen).to(DEV)
+    lib = _lib.load()
+    nbytes = lib.fmx_bwd_batched_workspace_bytes(Nq, B, Lq, Ld, d)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    out = []
+    for q in (Q, far):
+        dD = torch.empty(B, Ld, d, dtype=torch.float16, device=DEV)
+        rc = lib.fmx_bwd_batched(
+            _lib.FMX_DTYPE_F16, q.data_ptr(), q.stride(0), q.stride(1), D.data_ptr(), D.stride(0), D.stride(1), None,
+            am.data_ptr(), g.data_ptr(), g.stride(0), g.stride(1), None, dD.data_ptr(), Nq, B, Lq, Ld, d,
+            ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream,
+        )
+        _lib.check(rc)
+        out.append(dD)
+    del far, store
+    torch.cuda.empty_cache()
+    assert torch.count_nonzero(out[0]) > 0 and torch.equal(out[0], out[1])
+
+
 def test_bwd_graph_capture_replays():
     """fmx_bwd_batched captured into a HIP graph at a size that forks the dQ
     chain when run eagerly: under capture both chains stay on the capturing
