@@ -401,6 +401,31 @@ int splitd_unit_queries(const FwdArgs& a) {
   return qp;
 }
 
+// Doc groups of a walk whose units do not map onto XCDs, on n resident
+// workgroups: U * groups workgroups of ceil(B / groups) docs run in rounds of n.
+// floor(n / U) groups fit one round, but leave up to half of it out (130 units
+// of 256: 126 idle); more groups, queued behind the first, fill several rounds
+// better. The cost of a round is its docs and half a doc for the start; the
+// fewest groups among equals. 128-token queries over docs of 300 x 1024, one
+// round / these groups, and one workgroup per (unit, doc) for comparison (us):
+// 65 queries over 300 docs 1883 / 1589, 2107; 86 over 300 2804 / 2156, 2799; 130
+// over 200 3723 / 2276, 2840; 300 over 100 3816 / 2473, 3291; of U[Ld/32, Ld]
+// tokens 1144 / 945, 1492; 1636 / 1258, 2004; 2127 / 1309, 2104; 2167 / 1450, 2388.
+int splitd_walk_groups(int64_t U, int64_t B, int64_t n) {
+  const int64_t k0 = (U + n - 1) / n;
+  int64_t best = 1, cost = INT64_MAX;
+  for (int64_t k = k0; k < k0 + 8; ++k) {
+    int64_t G = k * n / U;
+    if (G > B) G = B;
+    const int64_t c = (U * G + n - 1) / n * (2 * ((B + G - 1) / G) + 1);
+    if (c < cost) {
+      cost = c;
+      best = G;
+    }
+  }
+  return (int)best;
+}
+
 template <int KIND, int NQB, int KSW, bool KMASK, bool ARGMAX, bool VEC = true, bool C16 = VEC>
 hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
   constexpr int QROWS = NQB * 16;
@@ -438,8 +463,7 @@ hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
         wk.groups = 8 * (per_xcd / wk.U);
         if (wk.groups > a.B) wk.groups = a.B / 8 * 8;
       } else {
-        wk.groups = wk.U < n ? n / wk.U : 1;
-        if (wk.groups > a.B) wk.groups = a.B;
+        wk.groups = splitd_walk_groups(wk.U, a.B, n);
       }
       auto kern = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, true>;
       if constexpr (NQB * KSW >= 32) {

@@ -27,6 +27,7 @@ DEV = "cuda"
         (4, 32, 5, 40, 1024),     # too few docs for units
         (3, 33, 100, 1, 640),     # one-token docs
         (300, 128, 3, 16, 320),   # more units than workgroups that fit
+        (130, 128, 7, 20, 264),   # units queued behind those that fit
         (1, 200, 270, 70, 1024),  # passes of one query
         (1, 64, 9, 90, 512),
         (1, 128, 600, 31, 1024),  # one unit of 128 VGPRs
@@ -64,3 +65,29 @@ def test_walk_exact_on_integer_grid(Nq, Lq, B, Ld, d, dtype):
             live = (lengths > 0).repeat(Nq).to(DEV)
             assert torch.equal(at[live].long(), want_at[live].long())
             assert (at[~live] == 0).all()
+
+
+def _us(call):
+    call()
+    best = float("inf")
+    for _ in range(6):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(20):
+            call()
+        end.record()
+        torch.cuda.synchronize()
+        best = min(best, start.elapsed_time(end) * 50)
+    return best
+
+
+def _batch(Nq, Lq, B, Ld, d):
+    gen = torch.Generator(device=DEV).manual_seed(Nq + B)
+    Q, D = (torch.randn(n, L, d, generator=gen, device=DEV).half() for n, L in ((Nq, Lq), (B, Ld)))
+    return lambda: _launch_fwd(Q, D, None, Nq, B, Lq, Ld, d, True, False)
+
+
+def test_walk_fills_the_gpu_for_any_number_of_units():
+    """130 units do not divide 256 workgroups as 128 do, and take about as long
+    (one group of workgroups a unit leaves half the GPU out: 1.8 times)."""
+    assert _us(_batch(130, 128, 100, 300, 1024)) < 1.4 * _us(_batch(128, 128, 100, 300, 1024))
