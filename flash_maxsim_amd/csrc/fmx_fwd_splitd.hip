@@ -88,6 +88,7 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a, SplitWalk wk
     slot = 8 * grp + k;
     if (slot >= nslots) return;  // uniform over the workgroup, before any barrier
   }
+  if (WALK && grp0 >= a.B) return;  // uniform over the workgroup, before any barrier
   const int pass = u % npass;
   int qi, b, nqh = 1;  // nqh: queries of this unit
   if constexpr (WALK) {
@@ -461,7 +462,9 @@ hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
       if (wk.U > 1 && wk.U <= per_xcd && per_xcd % wk.U * 10 <= per_xcd && a.B >= 8) {
         wk.xcd = 1;
         wk.groups = 8 * (per_xcd / wk.U);
-        if (wk.groups > a.B) wk.groups = a.B / 8 * 8;
+        // few docs: one a workgroup, the last groups without any (4 x 128 tokens
+        // over 15 docs of 300 x 1024 28 us; rounded down, two docs a workgroup, 46)
+        if (wk.groups > a.B) wk.groups = (a.B + 7) / 8 * 8;
       } else {
         wk.groups = splitd_walk_groups(wk.U, a.B, n);
       }

@@ -28,6 +28,8 @@ DEV = "cuda"
         (3, 33, 100, 1, 640),     # one-token docs
         (300, 128, 3, 16, 320),   # more units than workgroups that fit
         (130, 128, 7, 20, 264),   # units queued behind those that fit
+        (2, 128, 13, 33, 1024),   # fewer docs than groups: not a multiple of eight
+        (3, 100, 41, 20, 512),    # the same, three units
         (1, 200, 270, 70, 1024),  # passes of one query
         (1, 64, 9, 90, 512),
         (1, 128, 600, 31, 1024),  # one unit of 128 VGPRs
@@ -91,3 +93,9 @@ def test_walk_fills_the_gpu_for_any_number_of_units():
     """130 units do not divide 256 workgroups as 128 do, and take about as long
     (one group of workgroups a unit leaves half the GPU out: 1.8 times)."""
     assert _us(_batch(130, 128, 100, 300, 1024)) < 1.4 * _us(_batch(128, 128, 100, 300, 1024))
+
+
+def test_walk_of_few_docs_takes_one_doc_a_workgroup():
+    """Four units over 15 docs fit the GPU at once, as over 16 (groups rounded down
+    to a multiple of eight put two docs on a workgroup: 1.6 times)."""
+    assert _us(_batch(4, 128, 15, 600, 1024)) < 1.25 * _us(_batch(4, 128, 16, 600, 1024))
