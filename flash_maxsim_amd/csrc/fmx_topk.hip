@@ -117,8 +117,10 @@ __device__ __forceinline__ void wave_minmax_u32(uint32_t& mn, uint32_t& mx) {
 // the per-thread maxima m of those halves (0: a thread without keys). At
 // least `want` maxima sit in the bin (of a 256-bin histogram over the 8 bits
 // below the maxima's common prefix) that holds the want-th largest maximum or
-// above it, so at least `want` keys reach that bin's lower edge. 0 when fewer
-// than `want` threads hold keys. The largest maximum goes to *bmax.
+// above it, so at least `want` keys reach that bin's lower edge. Where that bin
+// holds far more maxima than wanted, the eight bits below it are taken too, in a
+// second histogram. 0 when fewer than `want` threads hold keys. The largest
+// maximum goes to *bmax.
 // PRECLEARED: hist was zeroed before the call (no clearing pass), every wave
 // scans the histogram itself (no broadcast of the bin), and the caller passes
 // a barrier before it rewrites hist, wlo or whi (none at the end).
@@ -168,25 +170,49 @@ __device__ __forceinline__ uint32_t maxima_bound(uint32_t m, int want, uint32_t*
     const int bin = __builtin_amdgcn_readlane(found, __builtin_ctzll(who));
     return hi | ((uint32_t)bin << sh);
   }
-  if (tid < 64) {
-    // lane l holds bins 4l .. 4l+3; maxima in higher bins = total - inclusive prefix
-    uint32_t h[4];
+  // The bin that holds the rest-th largest of the maxima in hist:
+  // (bin or -1, maxima in higher bins, maxima in it).
+  auto find = [&](int rest) {
+    if (tid < 64) {
+      // lane l holds bins 4l .. 4l+3; maxima in higher bins = total - inclusive prefix
+      uint32_t h[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) h[j] = hist[4 * tid + j];
-    const int incl = wave_incl_scan((int)(h[0] + h[1] + h[2] + h[3]));
-    uint32_t above = (uint32_t)(__builtin_amdgcn_readlane(incl, 63) - incl);
-    if (tid == 0) bc[0] = -1;
+      for (int j = 0; j < 4; ++j) h[j] = hist[4 * tid + j];
+      const int incl = wave_incl_scan((int)(h[0] + h[1] + h[2] + h[3]));
+      uint32_t above = (uint32_t)(__builtin_amdgcn_readlane(incl, 63) - incl);
+      if (tid == 0) bc[0] = -1;
 #pragma unroll
-    for (int j = 3; j >= 0; --j) {
-      if (above < (uint32_t)want && (uint32_t)want <= above + h[j]) bc[0] = 4 * tid + j;
-      above += h[j];
+      for (int j = 3; j >= 0; --j) {
+        if (above < (uint32_t)rest && (uint32_t)rest <= above + h[j]) {
+          bc[0] = 4 * tid + j;
+          bc[1] = (int)above;
+          bc[2] = (int)h[j];
+        }
+        above += h[j];
+      }
     }
-  }
-  __syncthreads();
-  const int bin = bc[0];
+    __syncthreads();
+  };
+  find(want);
+  const int bin = bc[0], over = bc[1], in = bc[2];
   __syncthreads();  // bc, hist, wlo and whi are rewritten later
   if (bin < 0) return 0u;
-  return hi | ((uint32_t)bin << sh);
+  const uint32_t edge = hi | ((uint32_t)bin << sh);
+  if (sh == 0 || over + in <= 2 * want + 64) return edge;  // uniform
+  // The maxima span so much (both signs, or an -inf among them) that the bin
+  // holds far more than `want` of them: the next bits within it. Without this a
+  // thousand candidates go to the ranking, or more to the radix passes (the best
+  // 100 of 40000 N(0, 1) scores 56.9 -> 11.5 us, of scores three in ten of which
+  // are -inf 15.9 -> 11.8).
+  const int sh2 = sh < 8 ? 0 : sh - 8;
+  if (tid < 256) hist[tid] = 0u;
+  __syncthreads();
+  if (m != 0u && (m >> sh) == (edge >> sh)) atomicAdd(&hist[(m >> sh2) & ((1u << (sh - sh2)) - 1u)], 1u);
+  __syncthreads();
+  find(want - over);
+  const int bin2 = bc[0];
+  __syncthreads();
+  return bin2 < 0 ? edge : edge | ((uint32_t)bin2 << sh2);
 }
 
 // Ranks the nsel distinct keys of sel[] (rank = keys greater) and writes the
@@ -388,10 +414,14 @@ __global__ void __launch_bounds__(NT) topk_level_kernel(const float* scores, int
   uint64_t key[kTopkE];
   int valid = 0;
   if (keys_in) {
+    // A chunk's keys arrive best first, k at a time. Where k divides NT, a stride
+    // of NT would give a thread keys of one rank only, and the best would crowd
+    // into few threads, whose maxima then bound them badly; 37 spreads them (the
+    // best 128 of 100000 24.7 -> 11.4 us).
     const rsrc_t r = make_rsrc(keys_in + row * n + c0, (uint32_t)left * 8u);
 #pragma unroll
     for (int e = 0; e < kTopkE; ++e) {
-      const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(r, (uint32_t)(tid + e * NT) * 8u, 0, 0);
+      const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(r, (uint32_t)(((tid + 37 * e) & (NT - 1)) + e * NT) * 8u, 0, 0);
       key[e] = ((uint64_t)v[1] << 32) | v[0];
     }
 #pragma unroll
@@ -689,7 +719,9 @@ hipError_t run_levels(const TopkArgs& a, hipStream_t s) {
 // Keys per workgroup of the first level: 16384, or for one row past that 4096
 // where it then still ends with one more level (up to 64 chunks of k <= 128
 // keys), each workgroup's chain of loads, bound and packing over a quarter of
-// the keys (the best 100 of 20000: first level 7.7 -> 6.2 us). Rows of up to
+// the keys (both levels, the best 100 of 20000 12.2 -> 10.3 us, of 100000 12.4 ->
+// 11.1, of 262144 12.6 -> 11.5; the best 128 13.1 -> 11.3, 13.7 -> 11.4, 18.4 ->
+// 12.1). Rows of up to
 // 16384 keys are one launch as they are (9000: 10.4 against 14.3 us), and many
 // rows fill the GPU with the larger chunks (128 of 40000: 20.0 against 28.9).
 int64_t topk_chunk(int64_t Nq, int64_t B, int64_t k) {

@@ -250,3 +250,54 @@ def test_topk_first_level_chunks(oracle_mod, Nq, B, k):
     assert_same_selection(got, oracle_mod.topk(s, k))
     for s in (np.full((Nq, B), 0.5, np.float32), -np.arange(Nq * B, dtype=np.float32).reshape(Nq, B)):
         assert_same_selection(fm.topk_scores(torch.from_numpy(s).to(DEV), k), oracle_mod.topk(s, k))
+
+
+def spread_scores(kind, seed, shape):
+    """Scores around zero (both signs), positive ones, and those with empty docs' -inf among them."""
+    g = np.random.default_rng(seed)
+    s = g.standard_normal(shape).astype(np.float32)
+    if kind != "both signs":
+        s += 10.0
+    if kind == "empty docs":
+        s[g.random(shape) < 0.3] = -np.inf
+    return s
+
+
+@pytest.mark.parametrize("kind", ["both signs", "positive", "empty docs"])
+@pytest.mark.parametrize("Nq, B, k", [(1, 9000, 128), (1, 16385, 100), (1, 40000, 100), (1, 40000, 128), (1, 100000, 128),
+                                      (1, 100000, 64), (3, 70000, 100), (2, 50000, 256), (1, 200000, 1024), (1, 50000, 2000)])
+def test_topk_spread_scores(oracle_mod, kind, Nq, B, k):
+    """Rows whose maxima span two signs or reach down to -inf, where the bound of
+    the k-th best takes a second histogram, and later levels of k keys a chunk."""
+    s = spread_scores(kind, B + k, (Nq, B))
+    assert_same_selection(fm.topk_scores(torch.from_numpy(s).to(DEV), k), oracle_mod.topk(s, k))
+
+
+def test_topk_time_depends_little_on_the_scores():
+    """The best 100 of 40000 take about as long for scores of both signs and with
+    empty docs as for positive ones, and the best 128 of 100000 as the best 100
+    (a bound that admits a thousand candidates takes up to five times as long)."""
+
+    def us(x, k):
+        fm.topk_scores(x, k)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                fm.topk_scores(x, k)
+        best = float("inf")
+        for _ in range(6):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(5):
+                graph.replay()
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, start.elapsed_time(end) * 10)
+        return best
+
+    rows = {n: torch.from_numpy(spread_scores(n, 5, (100000,))).to(DEV) for n in ("positive", "both signs", "empty docs")}
+    base = us(rows["positive"][:40000], 100)
+    for kind in ("both signs", "empty docs"):
+        assert us(rows[kind][:40000], 100) < 1.4 * base, kind
+    assert us(rows["positive"], 128) < 1.7 * us(rows["positive"], 100)
