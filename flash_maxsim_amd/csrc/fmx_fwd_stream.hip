@@ -769,19 +769,25 @@ __global__ void __launch_bounds__(256) stream_u8_shared_kernel(FwdArgs a) {
 // wave's ring of P tiles runs on from one doc to the next, and a doc ends with
 // the wave's own reduction. Dealing a doc's few tiles to four waves, as
 // stream_fwd_kernel does, leaves waves without a tile where docs have one to
-// five, and merges four waves' maxima per doc behind a barrier. 32 tokens,
-// docs all long / of U[0, Ld]: 20000 docs of 77 tokens 76.9 / 44.9 -> 68.6 /
-// 37.9 us, of 40 40.3 / 33.8 -> 35.0 / 24.2, at d = 96 57.1 / 38.3 -> 51.0 /
-// 30.6. Three tiles in flight (four: 74.0 / 41.1, a wave per SIMD less).
-// G: eight docs a workgroup, sixteen from 2^15 docs (60000 docs of U[0, 50]
-// tokens 77 -> 69 us; 20000 of 77 39.1 against 37.9, and 32 41.4). The line at
-// 2^13 docs: below it the groups are too few to fill the GPU (5000 docs of 77
-// tokens 17.9 / 13.4 -> 21.4 / 14.9). Queries of 16 tokens (63.2 / 34.0 ->
-// 68.0 / 35.5), longer docs (128 tokens 112.6 -> 114.3) and d <= 64 (equal)
-// stay with stream_fwd_kernel.
+// five, and merges four waves' maxima per doc behind a barrier. Three tiles in
+// flight (four: 20000 docs of 77 tokens, all long / of U[0, Ld], 74.0 / 41.1
+// against 68.6 / 37.9 us, a wave per SIMD less). G: eight docs a workgroup, sixteen
+// from 2^15 docs (60000 docs of U[0, 50] tokens 77 -> 69 us; 20000 of 77 39.1 against
+// 37.9, and 32 41.4).
+// It pays where docs differ in length or have up to three tiles. 32 tokens, d =
+// 128, stream_fwd_kernel -> this (us), all long / of U[Ld/32, Ld] tokens:
+//   20000 docs of 40 40.1 / 33.9 -> 34.8 / 24.7, 60 54.3 / 38.3 -> 49.3 / 31.3, 77 62.6
+//   / 42.7 -> 68.5 / 37.2, 96 77.2 / 48.2 -> 85.3 / 44.6, 112 90.2 / 53.4 -> 97.0 / 50.9,
+//   128 111.4 / 59.0 -> 114.5 / 59.6; 40000 of 128 217 / 115 -> 226 / 124;
+//   16384 of 60 40.1 / 31.8 -> 40.8 / 26.4, 96 63.6 / 38.9 -> 69.6 / 38.2;
+//   8192 of 40 18.7 / 15.9 -> 16.9 / 11.7, 60 22.3 / 17.8 -> 23.9 / 15.7, 77 25.8 / 19.5 ->
+//   28.1 / 19.7, 96 29.6 / 21.4 -> 35.0 / 22.9; 5000 of 77 17.9 / 13.4 -> 21.4 / 14.9.
+// So it takes docs without lengths (all long) of up to 48 tokens, docs with lengths
+// of up to 96, or 80 below 2^14 docs, and none below 2^13 docs. Queries of 16 tokens
+// (63.2 / 34.0 -> 68.0 / 35.5) and d <= 64 (equal) stay with stream_fwd_kernel.
 constexpr int64_t kDocsMin = 1 << 13;
 bool stream_docs_takes(const FwdArgs& a) {
-  return a.Nq == 1 && !a.qidx && a.Ld <= 96 && a.B >= kDocsMin;
+  return a.Nq == 1 && !a.qidx && a.B >= kDocsMin && a.Ld <= (!a.lengths ? 48 : a.B >= 2 * kDocsMin ? 96 : 80);
 }
 
 template <int KIND, int NQB, int KS, bool KMASK, int P>
