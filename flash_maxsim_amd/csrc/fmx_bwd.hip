@@ -509,7 +509,8 @@ __device__ __forceinline__ void dd_write_block(const BwdArgs& a, int64_t slab) {
 // two streams 4 % slower than this with 1000 docs of 512 x 1024, and its event
 // waits cost 20 us where dD is 77 MB, 41.8 -> 24.0 us).
 template <bool BF, bool COUNT>
-__global__ void __launch_bounds__(256) bwd_front_kernel(BwdArgs a, unsigned n_gather, unsigned gather_x) {
+__global__ void __launch_bounds__(256) bwd_front_kernel(BwdArgs a, unsigned n_gather, unsigned gather_x,
+                                                        unsigned index0) {
   extern __shared__ uint32_t smem[];
   const unsigned x = blockIdx.x;
   if (x < n_gather) {
@@ -517,7 +518,7 @@ __global__ void __launch_bounds__(256) bwd_front_kernel(BwdArgs a, unsigned n_ga
     const int by = __builtin_amdgcn_readfirstlane((int)(x / gather_x));
     dq_partial_block<BF>(a, x - (unsigned)by * gather_x, by);
   } else {
-    const unsigned y = x - n_gather;
+    const unsigned y = index0 + (x - n_gather);
     const int b = (int)(y % (unsigned)a.B), chunk = (int)(y / (unsigned)a.B);
     if constexpr (COUNT) {
       dd_index_count(a, b, chunk, smem);
@@ -563,17 +564,23 @@ constexpr int64_t kBwdMaxBlocks = ((int64_t)1 << 24) - 1;  // workgroups of 256 
 template <bool BF>
 hipError_t launch_front(const BwdArgs& a, int64_t n_index, int64_t n_gather, hipStream_t s) {
   if (n_index + n_gather == 0) return hipSuccess;
-  if (n_index + n_gather > kBwdMaxBlocks && n_index && n_gather) {
-    const hipError_t e = launch_front<BF>(a, n_index, 0, s);
-    return e != hipSuccess ? e : launch_front<BF>(a, 0, n_gather, s);
-  }
+  if (n_index > UINT32_MAX) return hipErrorInvalidValue;
   const size_t keys = n_index ? (size_t)a.sort_n * sizeof(uint32_t) : 0;
   const bool count = keys + dd_count_bytes(a.Ld) <= kDdIndexLds;
   const size_t lds = n_index ? keys + (count ? dd_count_bytes(a.Ld) : 0) : 0;
   auto kern = count ? bwd_front_kernel<BF, true> : bwd_front_kernel<BF, false>;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(n_index + n_gather)), dim3(256), lds, s, a, (unsigned)n_gather,
-                     (unsigned)(n_gather ? n_gather / a.nchunk : 1));
-  return hipGetLastError();
+  const int64_t gather_x = n_gather ? n_gather / a.nchunk : 1;
+  // one launch, and more for the index workgroups past a launch's limit
+  for (int64_t first = 0; n_gather || first < n_index; n_gather = 0) {
+    const int64_t room = kBwdMaxBlocks - n_gather, rest = n_index - first;
+    const int64_t n = rest < room ? rest : room > 0 ? room : 0;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(n_gather + n)), dim3(256), lds, s, a, (unsigned)n_gather,
+                       (unsigned)gather_x, (unsigned)first);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    first += n;
+  }
+  return hipSuccess;
 }
 
 template <bool BF>

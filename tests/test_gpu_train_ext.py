@@ -329,6 +329,31 @@ def test_bwd_queries_far_apart():
     assert torch.count_nonzero(out[0]) > 0 and torch.equal(out[0], out[1])
 
 
+def test_bwd_more_docs_than_a_launch_has_workgroups():
+    """2^24 + 3 documents of one row: the dD index takes one workgroup a document,
+    past what one launch holds. Integers, so both gradients are exact."""
+    from flash_maxsim_amd import _lib
+
+    B, d = (1 << 24) + 3, 8
+    gen = torch.Generator(device=DEV).manual_seed(2300)
+    Q = torch.tensor([[[1, -2, 3, -4, 5, -6, 7, -8]]], dtype=torch.float16, device=DEV)
+    D = torch.randint(-1, 2, (B, 1, d), generator=gen, device=DEV, dtype=torch.int8).half()
+    g = torch.randint(-2, 3, (1, B), generator=gen, device=DEV, dtype=torch.int8).float()
+    am = torch.zeros(B, 1, dtype=torch.int32, device=DEV)
+    dQ = torch.full((1, 1, d), float("nan"), device=DEV)
+    dD = torch.full((B, 1, d), float("nan"), device=DEV)
+    lib = _lib.load()
+    nbytes = lib.fmx_bwd_batched_workspace_bytes(1, B, 1, 1, d)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    _lib.check(lib.fmx_bwd_batched_f32(
+        Q.data_ptr(), Q.stride(0), Q.stride(1), D.data_ptr(), D.stride(0), D.stride(1), None, am.data_ptr(), g.data_ptr(),
+        g.stride(0), g.stride(1), dQ.data_ptr(), dD.data_ptr(), 1, B, 1, 1, d, ws.data_ptr(), nbytes,
+        torch.cuda.current_stream().cuda_stream,
+    ))
+    assert torch.equal(dD[:, 0], g[0, :, None] * Q[0].float())
+    assert torch.equal(dQ[0, 0].double(), (g[0, :, None].double() * D[:, 0].double()).sum(dim=0))
+
+
 def test_bwd_graph_capture_replays():
     """fmx_bwd_batched captured into a HIP graph at a size that forks the dQ
     chain when run eagerly: under capture both chains stay on the capturing
