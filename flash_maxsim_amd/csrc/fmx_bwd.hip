@@ -201,7 +201,7 @@ constexpr int kEntryBits = 13;  // entries of one chunk < 2^13 (kDdChunk)
 constexpr uint32_t kNoRow = 0xffffffffu;
 constexpr int kDdMaxPasses = 4;  // workgroup row passes per dD writer slab, at most
 // LDS of an index workgroup: its keys, and with the counting sort four
-// counters per doc row, which fit beside 8192 keys up to Ld = 2040.
+// counters per doc row, which fit beside 8192 keys up to Ld = 2044.
 constexpr size_t kDdIndexLds = 65536 - 64;
 constexpr size_t dd_count_bytes(int64_t Ld) { return (size_t)Ld * 4 * sizeof(uint32_t); }
 

@@ -304,3 +304,53 @@ def test_float32_rows_too_far_apart_are_cast():
             assert same(fm.flash_maxsim_topk(q, x, 4, le), fm.flash_maxsim_topk(Q, D, 4, le))
             assert torch.equal(fm.flash_maxsim_sparse(q, x, idx, le), fm.flash_maxsim_sparse(Q, D, idx, le))
     assert torch.equal(fm.flash_maxsim_packed(Q, docs._replace(tokens=tokens)), fm.flash_maxsim_packed(Q, docs))
+
+
+def test_calls_from_two_host_threads():
+    """Two host threads, each on its own stream, score and train at the same time,
+    several times over: operands that are read in place and operands that each call
+    converts. Every result, read on its own stream, equals the serial one."""
+    import threading
+
+    def work(i):
+        gen = torch.Generator().manual_seed(3300 + i)
+        Q = torch.randn(3, 40, 100, generator=gen).to(DEV)
+        D = torch.randn(150, 60, 100, generator=gen).to(DEV)
+        ln = torch.randint(1, 61, (150,), generator=gen, dtype=torch.int32).to(DEV)
+        g = torch.randn(3, 150, generator=gen).to(DEV)
+        half = torch.randn(150, 60, 128, generator=gen).to(torch.float16).to(DEV)
+
+        def call():
+            q, x = Q.detach().requires_grad_(True), D.detach().requires_grad_(True)
+            s = fm.flash_maxsim_train_batched(q, x, ln)
+            return (fm.flash_maxsim(half[0, :32], half, ln), fm.flash_maxsim(Q[0], D, ln), fm.flash_maxsim(Q[1, :20], D),
+                    *fm.flash_maxsim_topk(Q[2], D, 70, ln), s.detach(), *torch.autograd.grad(s, (q, x), g))
+
+        return call
+
+    calls = [work(i) for i in range(2)]
+    want = [c() for c in calls]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    got, errors = [[], []], []
+
+    def worker(i):
+        try:
+            with torch.cuda.stream(streams[i]):
+                for _ in range(8):
+                    got[i].append(calls[i]())
+                streams[i].synchronize()
+        except Exception as e:  # reported on the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=worker, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for i in range(2):
+        assert len(got[i]) == 8
+        for out in got[i]:
+            assert len(out) == len(want[i]) and all(torch.equal(a, b) for a, b in zip(out, want[i]))
