@@ -476,6 +476,7 @@ int fmx_quantize_int8(int src_dtype, const void* src, int64_t s_stride_b, int64_
            (reinterpret_cast<uintptr_t>(codes) & code_align) == 0 && (c_stride_l & code_align) == 0)
               ? 1
               : 0;
+  if (a.vec && (reinterpret_cast<uintptr_t>(codes) & 7u) == 0 && (c_stride_l & 7) == 0) a.vec |= 2;
   const int kind = src_dtype == FMX_DTYPE_F32 ? 2 : (src_dtype == FMX_DTYPE_BF16 ? 1 : 0);
   return hip_status(fmx::launch_quantize(kind, a, static_cast<hipStream_t>(stream)), "fmx_quantize_int8 launch");
 }

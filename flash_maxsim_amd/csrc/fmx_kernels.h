@@ -122,8 +122,8 @@ struct QuantArgs {
   void* scales;               // fp16 bits: padded [B, Ld] (doc stride sm_stride_b) or packed [T]
   void* mins;
   int64_t sm_stride_b;
-  int vec;                    // 16-byte source rows and 8-byte (fp32 sources: 4-byte) code rows:
-                              // vector loads/stores
+  int vec;                    // 1: 16-byte source rows and 8-byte (fp32 sources: 4-byte) code rows:
+                              // vector loads/stores; 2: beside 1, 8-byte code rows
 };
 hipError_t launch_quantize(int src_kind, const QuantArgs& a, hipStream_t s);  // 0 f16, 1 bf16, 2 f32
 // Its inverse over contiguous [rows, d] codes with one fp16 scale and min per row.

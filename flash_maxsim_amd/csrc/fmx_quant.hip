@@ -49,7 +49,15 @@ __device__ __forceinline__ float src_elem(const void* p, int64_t i) {
 template <int SRC, bool NT>
 __device__ __forceinline__ void load8(const void* row, int k0, int d, bool vec, float (&x)[8]) {
   if (vec && k0 + 8 <= d) {
-    {
+    if constexpr (SRC == 2) {
+      const f32x4_t* p = reinterpret_cast<const f32x4_t*>(static_cast<const float*>(row) + k0);
+      const f32x4_t a = p[0], b = p[1];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[i] = a[i];
+        x[4 + i] = b[i];
+      }
+    } else {
       const u32x4_t* p = reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(row) + k0);
       const u32x4_t v = NT ? __builtin_nontemporal_load(p) : *p;
 #pragma unroll
@@ -211,7 +219,7 @@ __device__ __forceinline__ float group_reduce(float v) {
 // Each LPR-lane group takes R consecutive token rows per step and issues all
 // their loads before reducing any of them, so R rows of source are in flight
 // per group instead of one.
-template <int SRC, int LPR, int CPL, int R>
+template <int SRC, int LPR, int CPL, int R, bool QUADS>
 __global__ void __launch_bounds__(256) quantize_kernel(QuantArgs a) {
   constexpr int GPB = 256 / LPR;  // lane groups per block
   const int lane_in_row = threadIdx.x % LPR;
@@ -231,9 +239,8 @@ __global__ void __launch_bounds__(256) quantize_kernel(QuantArgs a) {
     const int64_t jend = packed ? ((len + 3) & ~(int64_t)3) : a.Ld;
     const int64_t obase = packed ? 4 * a.tok_group[b] : b * a.Ld;
     constexpr bool PK = SRC == 0;  // packed fp16 halves (above)
-    // element i of a lane's chunk cc: k = (cc * LPR + lane) * 8 + i, or for fp32
-    // sources quads, (2 * cc * LPR + (i / 4) * LPR + lane) * 4 + i % 4
-    constexpr bool QUADS = SRC == 2;
+    // element i of a lane's chunk cc: k = (cc * LPR + lane) * 8 + i, or with quads
+    // (fp32 sources) (2 * cc * LPR + (i / 4) * LPR + lane) * 4 + i % 4
     auto quad_k0 = [&](int cc, int h) { return ((2 * cc + h) * LPR + lane_in_row) * 4; };
     float x[PK ? 1 : R][CPL][8];
     uint32_t xh[PK ? R : 1][CPL][4];
@@ -250,7 +257,7 @@ __global__ void __launch_bounds__(256) quantize_kernel(QuantArgs a) {
             load4_f32<(LPR >= 8)>(src, quad_k0(cc, 0), a.d, a.vec != 0, x[k][cc]);
             load4_f32<(LPR >= 8)>(src, quad_k0(cc, 1), a.d, a.vec != 0, x[k][cc] + 4);
           } else
-            load8<SRC, (LPR >= 8)>(src, (cc * LPR + lane_in_row) * 8, a.d, a.vec != 0, x[k][cc]);
+            load8<SRC, (SRC != 2 && LPR >= 8)>(src, (cc * LPR + lane_in_row) * 8, a.d, a.vec != 0, x[k][cc]);
         }
       }
     }
@@ -352,7 +359,7 @@ __global__ void __launch_bounds__(256) quantize_kernel(QuantArgs a) {
   }
 }
 
-template <int SRC, int LPR, int CPL>
+template <int SRC, int LPR, int CPL, bool QUADS = (SRC == 2)>
 hipError_t launch_q(const QuantArgs& a, hipStream_t s) {
   constexpr int R = CPL == 1 ? 4 : (CPL == 2 ? 2 : 1);  // rows in flight per lane group
   constexpr int RPB = 256 / LPR * R;
@@ -364,7 +371,7 @@ hipError_t launch_q(const QuantArgs& a, hipStream_t s) {
   // halved the resident waves (394 -> 490 us).
   const int64_t gy = (a.B + 1) / 2 < 65535 ? (a.B + 1) / 2 : 65535;
   if (gx > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((quantize_kernel<SRC, LPR, CPL, R>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((quantize_kernel<SRC, LPR, CPL, R, QUADS>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -434,9 +441,24 @@ __global__ void __launch_bounds__(256) quantize_wide_kernel(QuantArgs a) {
   }
 }
 
+// Short fp32 rows of whole 8-element chunks keep eight consecutive elements a
+// lane: a row's quads are too few to fill the lines that a wave's load covers
+// (padded docs, 160 MB of source, eights / quads, us: d = 8 78 / 139, 24 66 / 93,
+// 32 48 / 69, 48 62 / 80, 56 54 / 86; 800 MB: d = 8 463 / 958, 32 264 / 426, 56 334 /
+// 425; quads gain from d = 64, 245 / 237). Packed rows, whose codes lie closer, only
+// up to d = 16 (160 MB: d = 8 88 / 113, 24 85 / 84, 32 68 / 66; 800 MB: d = 16 372 / 420,
+// 48 410 / 299).
 template <int SRC>
 hipError_t dispatch_q(const QuantArgs& a, hipStream_t s) {
   const int chunks = (int)((a.d + 7) / 8);
+  if constexpr (SRC == 2) {
+    if ((a.vec & 2) && (a.d & 7) == 0 && a.d <= (a.tok_group ? 16 : 56)) {
+      if (chunks <= 1) return launch_q<SRC, 1, 1, false>(a, s);
+      if (chunks <= 2) return launch_q<SRC, 2, 1, false>(a, s);
+      if (chunks <= 4) return launch_q<SRC, 4, 1, false>(a, s);
+      return launch_q<SRC, 8, 1, false>(a, s);
+    }
+  }
   if (chunks <= 1) return launch_q<SRC, 1, 1>(a, s);
   if (chunks <= 2) return launch_q<SRC, 2, 1>(a, s);
   if (chunks <= 4) return launch_q<SRC, 4, 1>(a, s);
