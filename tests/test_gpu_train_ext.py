@@ -326,6 +326,40 @@ def test_bwd_queries_far_apart():
     assert torch.count_nonzero(out[0]) > 0 and torch.equal(out[0], out[1])
 
 
+def test_bwd_narrow_rows_take_one_entry_at_a_time():
+    """dD at d = 8, one lane a row, against d = 16, two lanes, over the same picks: the
+    writer that fetches a row's entries ahead, a lane's worth at a time, would take
+    1.9 times as long on one lane."""
+    from flash_maxsim_amd import _lib
+
+    Nq, B, Lq, Ld = 32, 200, 32, 60
+    gen = torch.Generator().manual_seed(2400)
+    am = torch.randint(0, Ld, (Nq * B, Lq), generator=gen, dtype=torch.int32).to(DEV)
+    g = torch.randn(Nq, B, generator=gen).to(DEV)
+    lib = _lib.load()
+
+    def us(d):
+        Q, D = torch.randn(Nq, Lq, d, device=DEV).half(), torch.randn(B, Ld, d, device=DEV).half()
+        nbytes = lib.fmx_bwd_batched_workspace_bytes(Nq, B, Lq, Ld, d)
+        ws, dD = torch.empty(nbytes, dtype=torch.uint8, device=DEV), torch.empty_like(D)
+        best = float("inf")
+        for _ in range(6):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(10):
+                _lib.check(lib.fmx_bwd_batched(
+                    _lib.FMX_DTYPE_F16, Q.data_ptr(), Q.stride(0), Q.stride(1), D.data_ptr(), D.stride(0), D.stride(1),
+                    None, am.data_ptr(), g.data_ptr(), g.stride(0), g.stride(1), None, dD.data_ptr(), Nq, B, Lq, Ld, d,
+                    ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream,
+                ))
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, start.elapsed_time(end) * 100)
+        return best
+
+    assert us(8) < 1.45 * us(16)
+
+
 def test_bwd_more_docs_than_a_launch_has_workgroups():
     """2^24 + 3 documents of one row: the dD index takes one workgroup a document,
     past what one launch holds. Integers, so both gradients are exact."""
