@@ -388,7 +388,12 @@ __global__ void __launch_bounds__(256) splitd_sum_passes_kernel(FwdArgs a, int n
 // them at once instead of once per query (2 x 128 tokens over 11901 docs of 72 x
 // 1024 1306 -> 694 us, 100 x 32 over 1000 of 150 x 384 1675 -> 876, 16 x 32 over
 // 1000 of 300 x 384 477 -> 255, 32 x 32 over 200 of 180 x 1024 293 -> 104).
-// Fewer where there are too few docs to fill the CUs with units otherwise.
+// Fewer where there are too few docs to fill the CUs with units otherwise. Up to d =
+// 384 two queries of more than 32 tokens stay apart: their 128-row tile takes a CU to
+// itself where two 64-row ones share it (two a unit / one, docs all long and ragged,
+// us: 2 x 64 over 300 of 300 x 384 35.9 / 27.3, 35.0 / 25.6; 8 x 64 over 500 of 300 x
+// 300 126 / 114, 97 / 86; 33 x 64 over 500 of 300 x 384 525 / 511, 328 / 314, of 512 526 /
+// 588, 324 / 348).
 int splitd_unit_queries(const FwdArgs& a) {
   const int ksw = splitd_fwd_ksw(a.d);
   if (a.Nq <= 1 || ksw > 4) return 1;
@@ -397,6 +402,7 @@ int splitd_unit_queries(const FwdArgs& a) {
   if (qp > a.Nq) qp = a.Nq;
   while (qp > 1 && (int64_t)((a.Nq + qp - 1) / qp) * a.B < 256) qp = qp / 2;
   if (qp < 1 || qp * a.Lq <= 32) return 1;
+  if (a.d <= 384 && a.Lq > 32 && qp < 3) return 1;
   // the unit's queries are read through one buffer range
   if (a.sq_n < 0 || ((qp - 1) * a.sq_n + (a.Lq + 16) * a.sq_l) * 2 >= ((int64_t)1 << 31)) return 1;
   return qp;

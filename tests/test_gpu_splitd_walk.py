@@ -30,6 +30,8 @@ DEV = "cuda"
         (130, 128, 7, 20, 264),   # units queued behind those that fit
         (2, 128, 13, 33, 1024),   # fewer docs than groups: not a multiple of eight
         (3, 100, 41, 20, 512),    # the same, three units
+        (20, 64, 30, 20, 384),    # two 64-row queries apart
+        (7, 41, 300, 20, 272),    # three 41-row queries a unit, the last with one
         (1, 200, 270, 70, 1024),  # passes of one query
         (1, 64, 9, 90, 512),
         (1, 128, 600, 31, 1024),  # one unit of 128 VGPRs
@@ -99,3 +101,9 @@ def test_walk_of_few_docs_takes_one_doc_a_workgroup():
     """Four units over 15 docs fit the GPU at once, as over 16 (groups rounded down
     to a multiple of eight put two docs on a workgroup: 1.6 times)."""
     assert _us(_batch(4, 128, 15, 600, 1024)) < 1.25 * _us(_batch(4, 128, 16, 600, 1024))
+
+
+def test_narrow_queries_of_64_tokens_share_a_cu():
+    """Two queries of 64 tokens at d = 384 take less than one of 128, whose tile has a
+    compute unit to itself (0.8; as one unit of two queries 1.0)."""
+    assert _us(_batch(2, 64, 300, 300, 384)) < 0.9 * _us(_batch(1, 128, 300, 300, 384))
