@@ -474,6 +474,12 @@ hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
       } else {
         wk.groups = splitd_walk_groups(wk.U, a.B, n);
       }
+      // Docs of different lengths, two a workgroup at most: one a workgroup, started
+      // as others end, so that two long ones do not fall to one (ragged docs, two a
+      // workgroup / one, us: 2 x 128 tokens over 150 of 300 x 512 35.0 / 29.9, 4 x 128
+      // over 70 of 300 x 384 31.7 / 23.9; of one length 9 % slower; three a workgroup
+      // equal).
+      if (a.lengths && a.B > wk.groups && a.B <= 2 * wk.groups) wk.groups = wk.xcd ? (a.B + 7) / 8 * 8 : a.B;
       auto kern = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, true>;
       if constexpr (NQB * KSW >= 32) {
         if (wk.U == 1) kern = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, false>;

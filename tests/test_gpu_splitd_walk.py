@@ -30,6 +30,7 @@ DEV = "cuda"
         (130, 128, 7, 20, 264),   # units queued behind those that fit
         (2, 128, 13, 33, 1024),   # fewer docs than groups: not a multiple of eight
         (3, 100, 41, 20, 512),    # the same, three units
+        (2, 128, 203, 33, 512),   # up to two docs a group: a workgroup for each
         (20, 64, 30, 20, 384),    # two 64-row queries apart
         (7, 41, 300, 20, 272),    # three 41-row queries a unit, the last with one
         (1, 200, 270, 70, 1024),  # passes of one query
@@ -101,6 +102,19 @@ def test_walk_of_few_docs_takes_one_doc_a_workgroup():
     """Four units over 15 docs fit the GPU at once, as over 16 (groups rounded down
     to a multiple of eight put two docs on a workgroup: 1.6 times)."""
     assert _us(_batch(4, 128, 15, 600, 1024)) < 1.25 * _us(_batch(4, 128, 16, 600, 1024))
+
+
+def test_two_long_docs_among_short_ones_do_not_wait_for_each_other():
+    """Two units over 200 docs, 128 groups: docs 3 and 131 would fall to one workgroup,
+    docs 3 and 4 do not; both pairs take about as long (one workgroup for two long
+    docs: 1.8 times)."""
+    Q, D = (torch.randn(n, L, 512, device=DEV).half() for n, L in ((2, 128), (200, 2000)))
+    times = []
+    for other in (131, 4):
+        ln = torch.full((200,), 16, dtype=torch.int32, device=DEV)
+        ln[[3, other]] = 2000
+        times.append(_us(lambda: _launch_fwd(Q, D, ln, 2, 200, 128, 2000, 512, True, False)))
+    assert times[0] < 1.3 * times[1], times
 
 
 def test_narrow_queries_of_64_tokens_share_a_cu():
