@@ -78,7 +78,13 @@ def _compile_native(verbose: bool) -> Path:
 
     obj = OBJ_DIR / "native.o"
     dirs = [*include_paths(device_type="cuda"), sysconfig.get_paths()["include"]]
-    _run(["g++", "-std=c++17", "-O2", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    # NDEBUG, as torch itself: without it pybind11's headers define a thread-local
+    # counter. Once a library with thread-local storage is loaded, glibc (2.35) takes
+    # its slow way for the thread-local variables of all libraries loaded before it,
+    # torch's among them, in every thread that has not used the new one's, and nothing
+    # here uses that counter: an add of two small GPU tensors took 5.3 us instead of
+    # 4.4, topk_scores of 10 x 500 12.0 instead of 10.5.
+    _run(["g++", "-std=c++17", "-O2", "-DNDEBUG", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
           *(f"-isystem{d}" for d in dirs), "-c", str(CSRC / "native.cpp"), "-o", str(obj)], "g++ on native.cpp", verbose)
     return obj
 

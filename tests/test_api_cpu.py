@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import re
+import struct
 from pathlib import Path
 
 import numpy as np
@@ -50,6 +51,17 @@ def test_header_and_binding_agree(lib):
 def test_library_exports_every_declared_symbol(lib):
     for name in _header_decls():
         assert hasattr(lib, name), f"libflashmaxsim.so does not export {name}"
+
+
+def test_native_host_path_has_no_thread_local_storage():
+    """A library that brings thread-local storage it does not use slows the
+    thread-local accesses of every library loaded before it, and with them all of
+    torch's calls: the host path's program headers (ELF64) hold no PT_TLS segment."""
+    data = Path(_lib.native().__file__).read_bytes()
+    assert data[:5] == b"\x7fELF\x02"
+    (offset,), (size, n) = struct.unpack_from("<Q", data, 32), struct.unpack_from("<HH", data, 54)
+    types = [struct.unpack_from("<I", data, offset + i * size)[0] for i in range(n)]
+    assert 1 in types and 7 not in types  # PT_LOAD, PT_TLS
 
 
 def test_version(lib):
