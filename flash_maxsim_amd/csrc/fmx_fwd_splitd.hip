@@ -41,7 +41,10 @@ struct SplitWalk {
 // short docs gain from (2 x 128 tokens over 11901 docs of 72 x 1024 694 -> 673
 // us, of ragged lengths 462 -> 439; 32 x 32 over 200 ragged docs of 180 x 1024
 // 77 -> 68). Not with one unit whose query slice takes 128 VGPRs, which it
-// pushes into spills (128 tokens over 1000 ragged docs of 512 x 1024 131 -> 141).
+// pushes into spills (128 tokens over 1000 ragged docs of 512 x 1024 131 -> 141), nor
+// with uint8 docs, whose waves load tiles with and without scales in two copies of
+// the loop: a load ahead of both makes the compiler wait for all of it (20000 docs of
+// 16 x 512 under 64 tokens 134 -> 140, under 128 169 -> 197).
 template <int KIND, int NQB, int KSW, bool KMASK, bool ARGMAX, bool VEC, bool WALK = false, bool C16 = VEC,
           bool AHEAD = false>
 __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a, SplitWalk wk) {
@@ -178,21 +181,14 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a, SplitWalk wk
   // so do uint8 rows without 16-byte alignment (one wave per SIMD fewer).
   constexpr bool FIXED = VEC && !(KMASK && (NQB * KSW >= 32 || KSW >= 16));
   static_assert(!WALK || FIXED, "the walk loads a doc's first tiles unconditionally");
+  static_assert(!AHEAD || !U8, "uint8 waves load tiles in two ways");
   auto first_tiles = [&](auto sm_tag) __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < P; ++s) load_tile<KIND, KSW, VEC, decltype(sm_tag)::value, C16>(buf[s], dr, s, c, g, koff);
   };
-  auto open_doc = [&]() __attribute__((always_inline)) {
-    if (!U8 || owner) {
-      first_tiles(std::true_type{});
-    } else {
-      first_tiles(std::false_type{});
-    }
-  };
-  if constexpr (AHEAD) open_doc();
+  if constexpr (AHEAD) first_tiles(std::true_type{});
 
   for (;;) {
-  if constexpr (FIXED && !AHEAD) open_doc();
   const int ntiles = (len + 15) >> 4;
   float m = -INFINITY;
   int mi = 0;
@@ -285,6 +281,7 @@ __global__ void __launch_bounds__(512) splitd_fwd_kernel(FwdArgs a, SplitWalk wk
     // load the tiles' scales and mins; the others run a copy of the loop
     // without those loads (same tiles and barriers).
     auto run = [&](auto sm_tag) __attribute__((always_inline)) {
+      if constexpr (!AHEAD) first_tiles(sm_tag);
       int i0 = 0;
       for (; i0 + P < ntiles; i0 += P) {
 #pragma unroll
@@ -444,6 +441,7 @@ hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
   // masked 128-row instances would spill.
   if constexpr (NQB >= 4 && VEC && !(KMASK && NQB * KSW >= 32)) {
     if ((a.Nq == 1 || a.shared_docs) && !a.qidx) {
+      constexpr bool AHEAD = KIND != KIND_U8;
       // resident workgroups: per CU x CUs (cached per device)
       static int cache[64] = {0};
       int dev = 0;
@@ -452,9 +450,9 @@ hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
       if (n == 0) {
         int cus = 0, per = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per, reinterpret_cast<const void*>(splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, true>), 512,
-                0) != hipSuccess || per <= 0)
+        auto first = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, AHEAD>;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(first), 512, 0) !=
+                hipSuccess || per <= 0)
           per = 1;
         n = cus * per;
         if (dev >= 0 && dev < 64) cache[dev] = n;
@@ -480,8 +478,8 @@ hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
       // over 70 of 300 x 384 31.7 / 23.9; of one length 9 % slower; three a workgroup
       // equal).
       if (a.lengths && a.B > wk.groups && a.B <= 2 * wk.groups) wk.groups = wk.xcd ? (a.B + 7) / 8 * 8 : a.B;
-      auto kern = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, true>;
-      if constexpr (NQB * KSW >= 32) {
+      auto kern = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, AHEAD>;
+      if constexpr (AHEAD && NQB * KSW >= 32) {
         if (wk.U == 1) kern = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, false>;
       }
       hipLaunchKernelGGL(kern, dim3((unsigned)wk.U * (unsigned)wk.groups), dim3(512), 0, s, a, wk);

@@ -7,7 +7,9 @@ from __future__ import annotations
 import pytest
 import torch
 
+import flash_maxsim_amd as fm
 from flash_maxsim_amd.flash_maxsim import _launch_fwd
+from launches import launches
 
 pytestmark = pytest.mark.gpu
 
@@ -121,3 +123,18 @@ def test_narrow_queries_of_64_tokens_share_a_cu():
     """Two queries of 64 tokens at d = 384 take less than one of 128, whose tile has a
     compute unit to itself (0.8; as one unit of two queries 1.0)."""
     assert _us(_batch(2, 64, 300, 300, 384)) < 0.9 * _us(_batch(1, 128, 300, 300, 384))
+
+
+def test_uint8_docs_are_not_loaded_ahead(tmp_path):
+    """The walk loads the next fp16 doc's tiles ahead of the current one's end. For
+    uint8 docs that took up to a sixth longer: their walk does not (the kernel's last
+    template argument)."""
+    Q = torch.randn(100, 512, device=DEV).half()
+    D = torch.randn(600, 16, 512, device=DEV).half()
+    codes = fm.quantize_int8(D)
+    (half, _), = launches(lambda: fm.flash_maxsim(Q[:64], D), tmp_path)
+    (byte, _), = launches(lambda: fm.flash_maxsim_int8(Q[:64], *codes), tmp_path)
+    (long, _), = launches(lambda: fm.flash_maxsim_int8(Q, *codes), tmp_path)
+    assert "splitd_fwd_kernel<0, 4, 2, false, false, true, true, true, true>" in half
+    assert "splitd_fwd_kernel<2, 4, 2, false, false, true, true, true, false>" in byte
+    assert "splitd_fwd_kernel<2, 8, 2, false, false, true, true, true, false>" in long
