@@ -386,43 +386,88 @@ __global__ void __launch_bounds__(256) splitd_sum_passes_kernel(FwdArgs a, int n
 // 1024 1306 -> 694 us, 100 x 32 over 1000 of 150 x 384 1675 -> 876, 16 x 32 over
 // 1000 of 300 x 384 477 -> 255, 32 x 32 over 200 of 180 x 1024 293 -> 104).
 // Fewer where there are too few docs to fill the CUs with units otherwise. Up to d =
-// 384 two queries of more than 32 tokens stay apart: their 128-row tile takes a CU to
-// itself where two 64-row ones share it (two a unit / one, docs all long and ragged,
-// us: 2 x 64 over 300 of 300 x 384 35.9 / 27.3, 35.0 / 25.6; 8 x 64 over 500 of 300 x
-// 300 126 / 114, 97 / 86; 33 x 64 over 500 of 300 x 384 525 / 511, 328 / 314, of 512 526 /
-// 588, 324 / 348).
+// 384 a unit keeps to 64 rows, as two such tiles share a CU where a 128-row one has
+// it to itself (128 rows / 64, docs all long and ragged, us: 2 x 64 tokens over 300 of
+// 300 x 384 35.9 / 27.3, 35.0 / 25.6; 16 x 32 over 140 of 300 x 264 49.4 / 35.2, 44.8 /
+// 24.3, of 300 x 384 51.7 / 42.3, 38.2 / 32.7), unless three queries fit the 128 rows
+// and one the 64 (60 x 40 over 102 of 300 x 320 144 / 182, 94 / 112). Up to d = 512 so
+// it does with lengths (2 x 64 over 358 of 1000 x 512 97.3 / 77.7) or fewer than 1024
+// (query, doc) pairs (104.9 / 97.1; past that 665 of them 161 / 180).
 int splitd_unit_queries(const FwdArgs& a) {
   const int ksw = splitd_fwd_ksw(a.d);
   if (a.Nq <= 1 || ksw > 4) return 1;
-  const int cap = a.d != 32 * ksw * kSplitWaves && ksw == 4 ? 64 : 128;
+  const bool narrow = a.d <= 384 || (a.d <= 512 && (a.lengths || (int64_t)a.Nq * a.B < 1024));
+  const int cap = (a.d != 32 * ksw * kSplitWaves && ksw == 4) || (narrow && (a.Lq <= 32 || 3 * a.Lq > 128)) ? 64 : 128;
   int qp = cap / a.Lq;
   if (qp > a.Nq) qp = a.Nq;
   while (qp > 1 && (int64_t)((a.Nq + qp - 1) / qp) * a.B < 256) qp = qp / 2;
   if (qp < 1 || qp * a.Lq <= 32) return 1;
-  if (a.d <= 384 && a.Lq > 32 && qp < 3) return 1;
   // the unit's queries are read through one buffer range
   if (a.sq_n < 0 || ((qp - 1) * a.sq_n + (a.Lq + 16) * a.sq_l) * 2 >= ((int64_t)1 << 31)) return 1;
   return qp;
 }
 
+// What starting a workgroup of the walk costs, its query slice above all, in tokens
+// of a doc.
+int64_t walk_start(int64_t d) { return 50 + d / 10; }
+
 // Doc groups of a walk whose units do not map onto XCDs, on n resident
 // workgroups: U * groups workgroups of ceil(B / groups) docs run in rounds of n.
 // floor(n / U) groups fit one round, but leave up to half of it out (130 units
 // of 256: 126 idle); more groups, queued behind the first, fill several rounds
-// better. The cost of a round is its docs and half a doc for the start; the
-// fewest groups among equals. 128-token queries over docs of 300 x 1024, one
-// round / these groups, and one workgroup per (unit, doc) for comparison (us):
-// 65 queries over 300 docs 1883 / 1589, 2107; 86 over 300 2804 / 2156, 2799; 130
+// better. The cost of a round is its docs (half as long, where lengths differ) and
+// the start; the fewest groups among equals. 128-token queries over docs of 300 x
+// 1024, one round / these groups, and one workgroup per (unit, doc) for comparison
+// (us): 65 queries over 300 docs 1883 / 1589, 2107; 86 over 300 2804 / 2156, 2799; 130
 // over 200 3723 / 2276, 2840; 300 over 100 3816 / 2473, 3291; of U[Ld/32, Ld]
-// tokens 1144 / 945, 1492; 1636 / 1258, 2004; 2127 / 1309, 2104; 2167 / 1450, 2388.
-int splitd_walk_groups(int64_t U, int64_t B, int64_t n) {
+// tokens 1144 / 945, 1492; 1636 / 1258, 2004; 2127 / 1309, 2104; 2167 / 1450, 2388;
+// 65 over 16 of 1000 x 384 302 / 265, 267, ragged 188 / 155, 251.
+int splitd_walk_groups(int64_t U, int64_t B, int64_t Ld, int64_t d, bool ragged, int64_t n) {
   const int64_t k0 = (U + n - 1) / n;
   int64_t best = 1, cost = INT64_MAX;
   for (int64_t k = k0; k < k0 + 8; ++k) {
     int64_t G = k * n / U;
     if (G > B) G = B;
-    const int64_t c = (U * G + n - 1) / n * (2 * ((B + G - 1) / G) + 1);
+    const int64_t docs = (B + G - 1) / G;
+    const int64_t c = (U * G + n - 1) / n * (walk_start(d) + docs * (ragged ? (Ld + 1) / 2 : Ld));
     if (c < cost) {
+      cost = c;
+      best = G;
+    }
+  }
+  // Two docs a workgroup at most: one, started as others end, so that two long ones do
+  // not fall to one.
+  if (U > 1 && ragged && B <= 2 * best) best = B;
+  return (int)best;
+}
+
+// The same where the units of a doc group share an XCD, so that they read its docs
+// through one L2: a multiple of eight, the last groups perhaps without a doc (few docs:
+// one a workgroup; 4 x 128 tokens over 15 of 300 x 1024 28 us, 46 rounded down).
+// Docs of one length: up to four docs a workgroup, or those of one round. Of several
+// lengths: one round, whose fixed lists share the starts out but may put long docs
+// together, or a workgroup for each doc, started as others end; with r docs a
+// workgroup of the round the former loses about 0.7 sqrt(r) docs at its end, the latter
+// r starts. One round / these (us): 3 x 100 tokens over 162 of 300 x 384 50.9 / 38.8;
+// ragged: 2 x 128 over 332 of 1000 x 384 137 / 117, over 537 of 1000 x 264 197 / 157,
+// over 150 of 300 x 512 35.0 / 29.9, 4 x 128 over 70 of 300 x 384 31.7 / 23.9. A workgroup
+// for each doc / these: 2 x 128 over 448 of 300 x 512 79.9 / 67.1, ragged 57.0 / 52.4, over
+// 192 of 72 x 512 19.7 / 15.5, ragged 18.4 / 14.7.
+int splitd_xcd_groups(int64_t U, int64_t B, int64_t Ld, int64_t d, bool ragged, int per_xcd, int cus) {
+  const int64_t fit = 8 * (per_xcd / U);  // groups in one round
+  const int64_t ones = (B + 7) / 8 * 8;   // a workgroup for each doc
+  const int64_t start = walk_start(d);
+  if (B <= fit) return (int)ones;
+  if (ragged) return (int)(B * 4 * start * start < fit * Ld * Ld ? ones : fit);
+  int64_t best = fit, cost = INT64_MAX;
+  for (int64_t m = 0; m <= 4; ++m) {
+    const int64_t G = m ? ((B + m - 1) / m + 7) / 8 * 8 : fit;
+    const int64_t W = U * (G / 8);  // workgroups of an XCD
+    // tenths of a round; a CU with one of its two workgroups is done with it a little sooner
+    const int64_t rest = W % per_xcd;
+    const int64_t turns = W / per_xcd * 10 + (rest == 0 ? 0 : per_xcd > cus && rest <= cus ? 8 : 10);
+    const int64_t c = turns * (start + (B + G - 1) / G * Ld);
+    if (c + c / 50 < cost) {
       cost = c;
       best = G;
     }
@@ -444,18 +489,25 @@ hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
       constexpr bool AHEAD = KIND != KIND_U8;
       // resident workgroups: per CU x CUs (cached per device)
       static int cache[64] = {0};
+      static int cu_cache[64] = {0};
       int dev = 0;
-      int n = 0;
-      if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) n = cache[dev];
-      if (n == 0) {
-        int cus = 0, per = 0;
+      int n = 0, cus = 0;
+      if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) {
+        n = cache[dev];
+        cus = cu_cache[dev];
+      }
+      if (n == 0 || cus == 0) {
+        int per = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
         auto first = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, AHEAD>;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(first), 512, 0) !=
                 hipSuccess || per <= 0)
           per = 1;
         n = cus * per;
-        if (dev >= 0 && dev < 64) cache[dev] = n;
+        if (dev >= 0 && dev < 64) {
+          cu_cache[dev] = cus;
+          cache[dev] = n;
+        }
       }
       SplitWalk wk = {};
       wk.qp = npass == 1 ? splitd_unit_queries(a) : 1;
@@ -465,19 +517,10 @@ hipError_t launch_one(const FwdArgs& a, hipStream_t s) {
       const int per_xcd = n / 8;
       if (wk.U > 1 && wk.U <= per_xcd && per_xcd % wk.U * 10 <= per_xcd && a.B >= 8) {
         wk.xcd = 1;
-        wk.groups = 8 * (per_xcd / wk.U);
-        // few docs: one a workgroup, the last groups without any (4 x 128 tokens
-        // over 15 docs of 300 x 1024 28 us; rounded down, two docs a workgroup, 46)
-        if (wk.groups > a.B) wk.groups = (a.B + 7) / 8 * 8;
+        wk.groups = splitd_xcd_groups(wk.U, a.B, a.Ld, a.d, a.lengths != nullptr, per_xcd, cus / 8);
       } else {
-        wk.groups = splitd_walk_groups(wk.U, a.B, n);
+        wk.groups = splitd_walk_groups(wk.U, a.B, a.Ld, a.d, a.lengths != nullptr, n);
       }
-      // Docs of different lengths, two a workgroup at most: one a workgroup, started
-      // as others end, so that two long ones do not fall to one (ragged docs, two a
-      // workgroup / one, us: 2 x 128 tokens over 150 of 300 x 512 35.0 / 29.9, 4 x 128
-      // over 70 of 300 x 384 31.7 / 23.9; of one length 9 % slower; three a workgroup
-      // equal).
-      if (a.lengths && a.B > wk.groups && a.B <= 2 * wk.groups) wk.groups = wk.xcd ? (a.B + 7) / 8 * 8 : a.B;
       auto kern = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, AHEAD>;
       if constexpr (AHEAD && NQB * KSW >= 32) {
         if (wk.U == 1) kern = splitd_fwd_kernel<KIND, NQB, KSW, KMASK, ARGMAX, VEC, true, VEC, false>;

@@ -35,6 +35,11 @@ DEV = "cuda"
         (2, 128, 203, 33, 512),   # up to two docs a group: a workgroup for each
         (20, 64, 30, 20, 384),    # two 64-row queries apart
         (7, 41, 300, 20, 272),    # three 41-row queries a unit, the last with one
+        (5, 20, 301, 24, 264),    # three 20-row queries a 64-row unit, the last with two
+        (3, 100, 163, 300, 264),  # a workgroup a doc, queued: docs of one length and of several
+        (2, 128, 290, 200, 264),  # one round of 128 groups, or a workgroup a doc
+        (8, 64, 150, 260, 300),   # 64-row units, two workgroups a CU
+        (33, 100, 19, 200, 264),  # no XCD mapping, queued
         (1, 200, 270, 70, 1024),  # passes of one query
         (1, 64, 9, 90, 512),
         (1, 128, 600, 31, 1024),  # one unit of 128 VGPRs
@@ -119,10 +124,33 @@ def test_two_long_docs_among_short_ones_do_not_wait_for_each_other():
     assert times[0] < 1.3 * times[1], times
 
 
-def test_narrow_queries_of_64_tokens_share_a_cu():
-    """Two queries of 64 tokens at d = 384 take less than one of 128, whose tile has a
-    compute unit to itself (0.8; as one unit of two queries 1.0)."""
-    assert _us(_batch(2, 64, 300, 300, 384)) < 0.9 * _us(_batch(1, 128, 300, 300, 384))
+@pytest.mark.parametrize(
+    "Nq, Lq, B, Ld, d, ragged, blocks, groups",
+    [
+        (2, 64, 300, 300, 384, False, 4, None),   # 64-row tiles, two a CU
+        (16, 32, 140, 300, 264, False, 4, None),
+        (60, 40, 102, 300, 320, False, 8, None),  # but three queries in 128 rows
+        (2, 64, 358, 100, 512, True, 4, None),    # d = 512: with lengths,
+        (2, 64, 358, 100, 512, False, 4, None),   # or few docs
+        (2, 64, 665, 100, 512, False, 8, None),
+        (2, 128, 15, 300, 1024, False, 8, 16),    # few docs: one a workgroup
+        (3, 100, 162, 300, 384, False, 8, 168),   # one length: the fewest rounds of docs,
+        (2, 128, 448, 300, 512, False, 8, 128),   # here one
+        (2, 128, 332, 1000, 384, True, 8, 336),   # long docs of several lengths: one a workgroup
+        (2, 128, 448, 300, 512, True, 8, 128),    # shorter ones: one round
+        (2, 128, 192, 72, 512, True, 8, 128),
+    ],
+)
+def test_walk_units_and_groups(Nq, Lq, B, Ld, d, ragged, blocks, groups, tmp_path):
+    """How queries are gathered into units and docs into groups on 256 CUs: 16-row
+    blocks of the query tile, and doc groups of the launch (None: not looked at)."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("256 CUs")
+    Q, D = (torch.randn(n, L, d, device=DEV).half() for n, L in ((Nq, Lq), (B, Ld)))
+    lengths = torch.randint(1, Ld + 1, (B,), dtype=torch.int32, device=DEV) if ragged else None
+    (name, grid), = launches(lambda: fm.flash_maxsim_batched(Q, D, lengths), tmp_path)
+    assert f"splitd_fwd_kernel<0, {blocks}," in name
+    assert groups is None or grid == groups * Nq, grid
 
 
 def test_uint8_docs_are_not_loaded_ahead(tmp_path):
