@@ -16,6 +16,7 @@ import pytest
 import torch
 
 import flash_maxsim_amd as fm
+from launches import launches
 from conftest import ROOT, sim, to_np32
 
 pytestmark = pytest.mark.gpu
@@ -430,10 +431,10 @@ def test_dequantize_gpu_bitwise_torch(shape):
 
 
 @pytest.mark.parametrize("B, Ld, d", [(1, 1, 1), (5, 7, 3), (9, 33, 100), (300, 20, 64), (3, 300, 128), (4, 9, 2050),
-                                      (4095, 3, 2), (4097, 5, 8), (65537, 2, 1)])
+                                      (4095, 3, 2), (4097, 5, 8), (49152, 2, 1), (65537, 2, 1)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.uint8, torch.float64])
 def test_pack_docs_gpu_equals_cpu(B, Ld, d, dtype):
-    """pack_docs on GPU tensors (layout and copy kernels, up to 65536 docs) against
+    """pack_docs on GPU tensors (layout and copy kernels, the layout up to 49152 docs) against
     the torch ops it runs on the CPU: lengths below 0 and past Ld, rows of any
     width and alignment, strided and expanded docs, the sorted layout, no lengths."""
     gen = torch.Generator().manual_seed(2600 + B + d)
@@ -454,6 +455,15 @@ def test_pack_docs_gpu_equals_cpu(B, Ld, d, dtype):
                 assert a.dtype == b.dtype and a.is_contiguous() and torch.equal(a.cpu(), b)
             if want.doc_ids is not None:
                 assert torch.equal(got.doc_ids.cpu(), want.doc_ids)
+
+
+def test_layout_of_many_docs_stays_with_torch(tmp_path):
+    """The one-workgroup layout kernel up to 49152 docs, past which it takes longer than
+    torch's ops."""
+    for B, kernel in ((49152, True), (49153, False)):
+        D, lengths = torch.zeros(B, 2, 8, device=DEV), torch.ones(B, dtype=torch.int32, device=DEV)
+        names = [name for name, _ in launches(lambda: fm.pack_docs(D, lengths), tmp_path)]
+        assert any("layout_kernel" in n for n in names) == kernel
 
 
 def test_pack_docs_keeps_gradients():
