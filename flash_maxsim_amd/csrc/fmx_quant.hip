@@ -447,7 +447,11 @@ __global__ void __launch_bounds__(256) quantize_wide_kernel(QuantArgs a) {
 // 32 48 / 69, 48 62 / 80, 56 54 / 86; 800 MB: d = 8 463 / 958, 32 264 / 426, 56 334 /
 // 425; quads gain from d = 64, 245 / 237). Packed rows, whose codes lie closer, only
 // up to d = 16 (160 MB: d = 8 88 / 113, 24 85 / 84, 32 68 / 66; 800 MB: d = 16 372 / 420,
-// 48 410 / 299).
+// 48 410 / 299). Wide rows keep it where the source fits the caches, which the quads'
+// non-temporal loads pass by (30 MB: d = 768 11.6 / 14.0, 1024 11.5 / 14.0, 4096 17.5 /
+// 22.4; 60 MB: d = 768 23 / 18, 1024 22 / 19), and from d = 1032 to 2048 at every size
+// measured (160 MB and 1 GB: d = 1536 34 / 49 and 223 / 264, 2048 35 / 47 and 213 / 252;
+// but d = 3072 1 GB 535 / 440).
 template <int SRC>
 hipError_t dispatch_q(const QuantArgs& a, hipStream_t s) {
   const int chunks = (int)((a.d + 7) / 8);
@@ -457,6 +461,12 @@ hipError_t dispatch_q(const QuantArgs& a, hipStream_t s) {
       if (chunks <= 2) return launch_q<SRC, 2, 1, false>(a, s);
       if (chunks <= 4) return launch_q<SRC, 4, 1, false>(a, s);
       return launch_q<SRC, 8, 1, false>(a, s);
+    }
+    if ((a.vec & 2) && (a.d & 7) == 0 && a.d > 640 &&
+        ((a.d > 1024 && a.d <= 2048) || a.B * a.Ld * a.d < ((int64_t)12 << 20))) {
+      if (chunks <= 128) return launch_q<SRC, 64, 2, false>(a, s);
+      if (chunks <= 256) return launch_q<SRC, 64, 4, false>(a, s);
+      if (chunks <= 512) return launch_q<SRC, 64, 8, false>(a, s);
     }
   }
   if (chunks <= 1) return launch_q<SRC, 1, 1>(a, s);

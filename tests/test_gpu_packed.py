@@ -476,8 +476,8 @@ def test_pack_docs_keeps_gradients():
     assert torch.equal(D.grad.cpu(), want)
 
 
-@pytest.mark.parametrize("d", [8, 16, 24, 32, 40, 48, 56, 64])
-def test_quantize_short_fp32_rows_bitwise(d):
+@pytest.mark.parametrize("d", [8, 16, 24, 32, 40, 48, 56, 64, 640, 648, 1024, 1032, 2048, 2056, 4096])
+def test_quantize_fp32_rows_bitwise(d):
     """Both ways an fp32 row of whole 8-element chunks is dealt to lanes: padded,
     packed, and codes off 8-byte alignment, against torch's formula on the CPU."""
     from flash_maxsim_amd import _lib
@@ -505,21 +505,18 @@ def test_quantize_short_fp32_rows_bitwise(d):
     assert torch.equal(out.cpu().view(codes.shape), codes)
 
 
-@pytest.mark.parametrize("d", [8, 32])
-def test_quantize_short_fp32_rows_take_no_longer_than_fp16_ones(d):
-    """Encoding short fp32 rows against the same rows in fp16 (1.2 times as long; dealt to
-    the lanes in quads 2.1 and 1.7 times)."""
-    D = torch.randn(40_000_000 // (200 * d), 200, d, device=DEV)
-    half = D.half()
-    best = {"fp32": float("inf"), "fp16": float("inf")}
-    for _ in range(6):
-        for name, x in (("fp32", D), ("fp16", half)):
-            fm.quantize_int8(x)
-            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            start.record()
-            for _ in range(10):
-                fm.quantize_int8(x)
-            end.record()
-            torch.cuda.synchronize()
-            best[name] = min(best[name], start.elapsed_time(end))
-    assert best["fp32"] < 1.45 * best["fp16"], best
+@pytest.mark.parametrize(
+    "d, rows, packed, quads",
+    [(8, 1000, False, False), (56, 1000, False, False), (64, 1000, False, True), (16, 1000, True, False),
+     (24, 1000, True, True), (640, 1000, False, True), (1000, 12000, False, False), (1000, 13000, False, True),
+     (1024, 1000, True, False), (1032, 13000, False, False), (2048, 7000, False, False), (2056, 7000, False, True),
+     (4096, 3000, False, False)],
+)
+def test_quantize_fp32_rows_as_measured_fastest(d, rows, packed, quads, tmp_path):
+    """Which way is taken: quads of a row across the lanes, or eight elements a lane for
+    narrow rows, sources that fit the caches, and rows of 1032 to 2048 elements (the
+    kernel's last template argument). Dealt in quads those took up to twice as long."""
+    D = torch.randn(rows // 100, 100, d, device=DEV)
+    call = (lambda: fm.quantize_int8_packed(D)) if packed else (lambda: fm.quantize_int8(D))
+    (name, _), = [e for e in launches(call, tmp_path) if "quantize_kernel" in e[0]]
+    assert f", {str(quads).lower()}>(" in name, name
