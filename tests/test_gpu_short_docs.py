@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import flash_maxsim_amd as fm
+from launches import launches
 
 pytestmark = pytest.mark.gpu
 
@@ -50,26 +51,16 @@ def test_short_docs_equal_general_kernel(Lq, B, Ld, d, dtype):
     assert torch.equal(values.view(torch.int32), want[idx].view(torch.int32))
 
 
-@pytest.mark.parametrize("B, Ld", [(40000, 96), (40000, 77)])
-def test_long_docs_take_less_than_their_parts(B, Ld):
-    """Docs without lengths in one call against the same docs in calls of 8000, too
-    few for the kernel of short docs, which takes 1.1 times as long on docs of five
-    or six full tiles: one call is the faster (0.91 and 0.86 of the parts' time, by
-    that kernel 1.00 and 0.96)."""
-    gen = torch.Generator(device=DEV).manual_seed(3400 + Ld)
-    Q = torch.randn(32, 128, generator=gen, device=DEV).half()
-    D = torch.randn(B, Ld, 128, generator=gen, device=DEV).half()
-    calls = {"whole": lambda: fm.flash_maxsim(Q, D),
-             "parts": lambda: [fm.flash_maxsim(Q, D[i : i + 8000]) for i in range(0, B, 8000)]}
-    best = dict.fromkeys(calls, float("inf"))
-    for _ in range(8):
-        for name, call in calls.items():
-            call()
-            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            start.record()
-            for _ in range(10):
-                call()
-            end.record()
-            torch.cuda.synchronize()
-            best[name] = min(best[name], start.elapsed_time(end))
-    assert best["whole"] < 0.945 * best["parts"], best
+@pytest.mark.parametrize(
+    "B, Ld, ragged, whole",
+    [(8192, 48, False, True), (8192, 49, False, False), (40000, 96, False, False), (8191, 40, True, False),
+     (8192, 80, True, True), (8192, 81, True, False), (16383, 96, True, False), (16384, 96, True, True),
+     (16384, 97, True, False)],
+)
+def test_short_docs_kernel_takes_what_it_is_faster_for(B, Ld, ragged, whole, tmp_path):
+    """The kernel whose waves score whole docs takes a tenth longer for docs of four
+    tiles or more that are all long: without lengths it takes up to 48 tokens."""
+    Q, D = (torch.randn(*n, 128, device=DEV).half() for n in ((32,), (B, Ld)))
+    lengths = torch.randint(1, Ld + 1, (B,), dtype=torch.int32, device=DEV) if ragged else None
+    (name, _), = launches(lambda: fm.flash_maxsim(Q, D, lengths), tmp_path)
+    assert ("stream_docs_kernel" in name) == whole, name

@@ -17,6 +17,7 @@ import pytest
 import torch
 
 import flash_maxsim_amd as fm
+from launches import launches
 from conftest import sim, to_np32
 from flash_maxsim_amd.flash_maxsim import _launch_fwd, _prep
 from test_gpu_parity import assert_argmax
@@ -326,38 +327,30 @@ def test_bwd_queries_far_apart():
     assert torch.count_nonzero(out[0]) > 0 and torch.equal(out[0], out[1])
 
 
-def test_bwd_narrow_rows_take_one_entry_at_a_time():
-    """dD at d = 8, one lane a row, against d = 16, two lanes, over the same picks: the
-    writer that fetches a row's entries ahead, a lane's worth at a time, would take
-    1.9 times as long on one lane."""
+@pytest.mark.parametrize(
+    "Nq, Lq, Ld, d, lengths, dense",
+    [(32, 32, 60, 8, False, False), (32, 32, 60, 9, False, True),  # one lane a row; two
+     (5, 20, 100, 16, False, False), (5, 21, 100, 16, False, True),  # an entry a row
+     (2, 20, 100, 16, True, False), (2, 21, 100, 16, True, True)],  # two entries to five rows
+)
+def test_bwd_writer_of_crowded_rows(Nq, Lq, Ld, d, lengths, dense, tmp_path):
+    """Which dD writer takes the call: the one that fetches a row's entries ahead, a
+    lane's worth at a time, not for rows of one lane, where it took 1.7 times as long."""
     from flash_maxsim_amd import _lib
 
-    Nq, B, Lq, Ld = 32, 200, 32, 60
-    gen = torch.Generator().manual_seed(2400)
-    am = torch.randint(0, Ld, (Nq * B, Lq), generator=gen, dtype=torch.int32).to(DEV)
-    g = torch.randn(Nq, B, generator=gen).to(DEV)
-    lib = _lib.load()
-
-    def us(d):
-        Q, D = torch.randn(Nq, Lq, d, device=DEV).half(), torch.randn(B, Ld, d, device=DEV).half()
-        nbytes = lib.fmx_bwd_batched_workspace_bytes(Nq, B, Lq, Ld, d)
-        ws, dD = torch.empty(nbytes, dtype=torch.uint8, device=DEV), torch.empty_like(D)
-        best = float("inf")
-        for _ in range(6):
-            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            start.record()
-            for _ in range(10):
-                _lib.check(lib.fmx_bwd_batched(
-                    _lib.FMX_DTYPE_F16, Q.data_ptr(), Q.stride(0), Q.stride(1), D.data_ptr(), D.stride(0), D.stride(1),
-                    None, am.data_ptr(), g.data_ptr(), g.stride(0), g.stride(1), None, dD.data_ptr(), Nq, B, Lq, Ld, d,
-                    ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream,
-                ))
-            end.record()
-            torch.cuda.synchronize()
-            best = min(best, start.elapsed_time(end) * 100)
-        return best
-
-    assert us(8) < 1.45 * us(16)
+    B, lib = 3, _lib.load()
+    Q, D = (torch.zeros(n, L, (d + 7) // 8 * 8, device=DEV).half() for n, L in ((Nq, Lq), (B, Ld)))
+    am = torch.zeros(Nq * B, Lq, dtype=torch.int32, device=DEV)
+    ln = torch.ones(B, dtype=torch.int32, device=DEV) if lengths else None
+    g, dD = torch.zeros(Nq, B, device=DEV), torch.empty(B, Ld, d, dtype=torch.float16, device=DEV)
+    nbytes = lib.fmx_bwd_batched_workspace_bytes(Nq, B, Lq, Ld, d)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    names = [name for name, _ in launches(lambda: _lib.check(lib.fmx_bwd_batched(
+        _lib.FMX_DTYPE_F16, Q.data_ptr(), Q.stride(0), Q.stride(1), D.data_ptr(), D.stride(0), D.stride(1),
+        _lib.ptr(ln), am.data_ptr(), g.data_ptr(), g.stride(0), g.stride(1), None, dD.data_ptr(), Nq, B, Lq, Ld, d,
+        ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream,
+    )), tmp_path)]
+    assert f"bwd_back_kernel<false, {str(dense).lower()}, " in names[-1], names
 
 
 def test_bwd_more_docs_than_a_launch_has_workgroups():
