@@ -100,7 +100,8 @@ int check_common(int64_t Nq, int64_t B, int64_t Lq, int64_t Ld, int64_t d, int64
     return fail(FMX_ERR_INVALID, "Q row stride %lld must be >= d and a multiple of %d", (long long)q_stride_l, m + 1);
   if (d_stride_l < d || (d_stride_l & m))
     return fail(FMX_ERR_INVALID, "D row stride %lld must be >= d and a multiple of %d", (long long)d_stride_l, m + 1);
-  if (d_stride_b & m) return fail(FMX_ERR_INVALID, "D doc stride %lld must be a multiple of %d", (long long)d_stride_b, m + 1);
+  if (d_stride_b & m)
+    return fail(FMX_ERR_INVALID, "D doc stride %lld must be a multiple of %d", (long long)d_stride_b, m + 1);
   if (Nq * B >= kOffLimit) return fail(FMX_ERR_UNSUPPORTED, "Nq*B=%lld too large", (long long)(Nq * B));
   if ((Lq + 128) * q_stride_l * (esz == 4 ? 4 : 2) >= kOffLimit)
     return fail(FMX_ERR_UNSUPPORTED, "query of %lld x %lld elements exceeds 2 GiB", (long long)Lq,
@@ -499,7 +500,8 @@ int fmx_dequantize_int8(const uint8_t* codes, const void* scales, const void* mi
 
 int fmx_packed_layout(const int32_t* lengths, int64_t B, int64_t Ld, int32_t* lengths_out, int64_t* tok_group,
                       int64_t* totals, void* stream) {
-  if (B < 0 || Ld < 0 || Ld > INT32_MAX) return fail(FMX_ERR_INVALID, "invalid sizes B=%lld Ld=%lld", (long long)B, (long long)Ld);
+  if (B < 0 || Ld < 0 || Ld > INT32_MAX)
+    return fail(FMX_ERR_INVALID, "invalid sizes B=%lld Ld=%lld", (long long)B, (long long)Ld);
   if (!totals || (B > 0 && (!lengths || !lengths_out || !tok_group)))
     return fail(FMX_ERR_INVALID, "lengths, lengths_out, tok_group and totals must be non-null");
   return hip_status(fmx::launch_layout(lengths, B, (int32_t)Ld, lengths_out, tok_group, totals,
@@ -728,8 +730,8 @@ int fmx_bwd_batched_f32(const void* Q, int64_t q_stride_n, int64_t q_stride_l, c
 int fmx_convert_rows(int src_dtype, const void* src, int64_t s_stride_b, int64_t s_stride_l, int64_t B, int64_t Ld,
                      int64_t d, const int32_t* lengths, int dst_dtype, void* dst, int64_t dp, void* stream) {
   if (B < 0 || Ld < 0 || d < 1 || dp < d || (dp & 7) || s_stride_b < 0 || s_stride_l < 0)
-    return fail(FMX_ERR_INVALID, "invalid sizes B=%lld Ld=%lld d=%lld dp=%lld", (long long)B, (long long)Ld, (long long)d,
-                (long long)dp);
+    return fail(FMX_ERR_INVALID, "invalid sizes B=%lld Ld=%lld d=%lld dp=%lld", (long long)B, (long long)Ld,
+                (long long)d, (long long)dp);
   const bool same = src_dtype == dst_dtype && (src_dtype == FMX_DTYPE_F16 || src_dtype == FMX_DTYPE_BF16);
   const bool cast = dst_dtype == FMX_DTYPE_F16 && (src_dtype == FMX_DTYPE_F32 || src_dtype == FMX_DTYPE_BF16);
   if (!same && !cast) return fail(FMX_ERR_INVALID, "no conversion from dtype %d to %d", src_dtype, dst_dtype);
@@ -738,7 +740,8 @@ int fmx_convert_rows(int src_dtype, const void* src, int64_t s_stride_b, int64_t
   if (!aligned16(dst)) return fail(FMX_ERR_INVALID, "dst must be 16-byte aligned");
   if (reinterpret_cast<uintptr_t>(src) & (src_dtype == FMX_DTYPE_F32 ? 3u : 1u))
     return fail(FMX_ERR_INVALID, "src must be aligned to its element");
-  if (dp > INT32_MAX || Ld > (INT32_MAX - 4096) / (dp / 4)) return fail(FMX_ERR_UNSUPPORTED, "doc of %lld x %lld elements", (long long)Ld, (long long)dp);
+  if (dp > INT32_MAX || Ld > (INT32_MAX - 4096) / (dp / 4))
+    return fail(FMX_ERR_UNSUPPORTED, "doc of %lld x %lld elements", (long long)Ld, (long long)dp);
   fmx::ConvertArgs a = {};
   a.src = src;
   a.s_stride_b = s_stride_b;

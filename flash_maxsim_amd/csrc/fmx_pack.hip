@@ -201,7 +201,8 @@ __global__ void __launch_bounds__(256) convert_kernel(const void* src, int64_t s
           if constexpr (SRC == 2) {
             v[k][e] = k0 + e < d ? static_cast<const uint32_t*>(src)[row + k0 + e] : 0u;
           } else {
-            v[k][e >> 1] |= k0 + e < d ? (uint32_t)static_cast<const uint16_t*>(src)[row + k0 + e] << (16 * (e & 1)) : 0u;
+            const uint32_t h = k0 + e < d ? static_cast<const uint16_t*>(src)[row + k0 + e] : 0u;
+            v[k][e >> 1] |= h << (16 * (e & 1));
           }
         }
       }

@@ -496,8 +496,9 @@ namespace {
 // value, where the formula's three tensor passes and the codes' conversion move
 // 21. A workgroup takes kDqBlock consecutive values of the [rows, d] matrix; a
 // thread takes 4 at a time (one 4-byte load, one 16-byte store, each contiguous
-// over the wave), all its loads issued first. Bound by the stores: 2000 docs of
-// 512 x 128 (655 MB) 660 -> 92.5 us, 7.1 TB/s.
+// over the wave), all its loads issued first. Bound by memory: 2000 docs of 512 x 128
+// (131 MB read, 524 MB written) 667 -> 127 us, 5.2 TB/s, the rate of a device copy
+// (92.5 us over one buffer, whose codes stay in the last-level cache).
 // VEC: d % 4 == 0, so four values share a row. NT: non-temporal stores, for
 // results the last-level cache would not hold.
 constexpr int kDqIter = 4, kDqBlock = 256 * 4 * kDqIter;
@@ -569,7 +570,8 @@ hipError_t launch_dequantize(const uint8_t* codes, const uint16_t* scales, const
   const bool vec = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(codes) & 3u) == 0 &&
                    (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
   const bool nt = rows * d * 4 >= ((int64_t)1 << 28);
-  auto kern = vec ? (nt ? dequantize_kernel<true, true> : dequantize_kernel<true, false>) : dequantize_kernel<false, false>;
+  auto kern = dequantize_kernel<false, false>;
+  if (vec) kern = nt ? dequantize_kernel<true, true> : dequantize_kernel<true, false>;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, s, codes, scales, mins, out, rows, (uint32_t)d, magic);
   return hipGetLastError();
 }

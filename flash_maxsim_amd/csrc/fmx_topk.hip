@@ -421,7 +421,8 @@ __global__ void __launch_bounds__(NT) topk_level_kernel(const float* scores, int
     const rsrc_t r = make_rsrc(keys_in + row * n + c0, (uint32_t)left * 8u);
 #pragma unroll
     for (int e = 0; e < kTopkE; ++e) {
-      const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(r, (uint32_t)(((tid + 37 * e) & (NT - 1)) + e * NT) * 8u, 0, 0);
+      const uint32_t at = (uint32_t)(((tid + 37 * e) & (NT - 1)) + e * NT);
+      const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(r, at * 8u, 0, 0);
       key[e] = ((uint64_t)v[1] << 32) | v[0];
     }
 #pragma unroll

@@ -9,8 +9,9 @@
 // error messages. In Python and ctypes an ordinary call's checks, allocations
 // and the conversion of twenty arguments took longer than the kernels of a
 // rerank: 100 docs of up to 300 x 128 under 32 tokens
-// 14.3 -> 4.8 us a call, 1000 docs with 16 tokens each 12.8 -> 9.1, a training
-// step of 32 x 32 tokens over 256 docs of up to 180 152 -> 105.
+// 14.3 -> 4.8 us a call, 1000 docs with 16 tokens each 12.8 -> 9.1. (A training
+// step's host time depends more on where autograd's thread runs: 85 or 150 us
+// before, 105 after, for 32 x 32 tokens over 256 docs of up to 180.)
 //
 // The library is reached through its C ABI alone.
 #include <Python.h>
@@ -91,7 +92,8 @@ int scoring_dtype(const Tensor& Q, const Tensor& D, int64_t Lq, int64_t Ld, int6
 // Whether `ready` can make t an operand.
 bool convertible(const Tensor& t) {
   const int64_t n = t.dim(), d = t.size(n - 1);
-  return (n == 2 || n == 3) && t.stride(n - 1) == 1 && d >= 1 && t.numel() > 0 && t.size(n - 2) <= (INT32_MAX - 4096) / (2 * (d / 8 + 1));
+  return (n == 2 || n == 3) && t.stride(n - 1) == 1 && d >= 1 && t.numel() > 0 &&
+         t.size(n - 2) <= (INT32_MAX - 4096) / (2 * (d / 8 + 1));
 }
 
 bool is_row_of(const Tensor* t, at::ScalarType type, int64_t n) {
@@ -205,7 +207,8 @@ PyObject* batched(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int dtype = kernel_dtype(*Q, *D);
   const int32_t* lengths;
   FMX_ORDINARY(D->size(k + 2) == d && (shared || (D->size(0) == Nq && D->stride(0) == B * D->stride(1))));
-  FMX_ORDINARY(dtype >= 0 && Nq > 0 && B > 0 && Lq > 0 && convertible(*Q) && (shared ? convertible(*D) : code_of(*D) == dtype && rows_ready(*D)) &&
+  FMX_ORDINARY(dtype >= 0 && Nq > 0 && B > 0 && Lq > 0 && convertible(*Q) &&
+               (shared ? convertible(*D) : code_of(*D) == dtype && rows_ready(*D)) &&
                Q->device() == D->device() && take_lengths(args[2], shared ? B : Nq * B, *D, &lengths) && here(*Q));
   Tensor out = at::empty({Nq, B}, D->options().dtype(at::kFloat));
   const size_t n = fmx_fwd_workspace_bytes(Nq, B, Lq, Ld, d);
@@ -426,7 +429,8 @@ PyObject* backward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t Nq = Q->size(0), Lq = Q->size(1), B = D->size(0), Ld = D->size(1);
   const int dtype = kernel_dtype(*Q, *D);
   const int32_t* lengths;
-  FMX_ORDINARY(dtype >= 0 && code_of(*Q) == dtype && code_of(*D) == dtype && Nq > 0 && Lq > 0 && B > 0 && Ld > 0 && d > 0 && d <= Q->size(2) && d <= D->size(2) &&
+  FMX_ORDINARY(dtype >= 0 && code_of(*Q) == dtype && code_of(*D) == dtype && Nq > 0 && Lq > 0 && B > 0 && Ld > 0 &&
+               d > 0 && d <= Q->size(2) && d <= D->size(2) &&
                (need_q || need_d) && rows_ready(*Q) && rows_ready(*D) && is_row_of(am, at::kInt, Nq * B * Lq));
   FMX_ORDINARY(g->scalar_type() == at::kFloat && g->size(0) == Nq && g->size(1) == B && g->stride(0) >= 0 &&
                g->stride(1) >= 0 && Q->device() == D->device() && am->device() == D->device() &&

@@ -13,7 +13,8 @@
  *    needed).
  *  - Strides are in elements of the tensor's type. The innermost (d) stride is
  *    1. Row strides of Q and D must be multiples of 8 elements, doc strides of
- *    D multiples of 8, and Q, D 16-byte aligned; d itself may be anything
+ *    D multiples of 8 (both of 4 where Q and D are fp32: fmx_fwd_reads_f32),
+ *    and Q, D 16-byte aligned; d itself may be anything
  *    from 1 to FMX_MAX_D (elements past d in a row are never used).
  *  - `stream` is a hipStream_t (NULL = the default stream). Work is enqueued
  *    asynchronously; nothing synchronises the host.
