@@ -124,6 +124,10 @@ void* stream_of(const Tensor& t);
 Tensor ready(const Tensor& t, int dtype, const int32_t* lengths, int* rc) {
   if (code_of(t) == dtype && rows_ready(t)) return t;
   const int64_t n = t.dim(), d = t.size(n - 1), dp = (d + 7) / 8 * 8, rows = t.size(n - 2);
+  // Docs of fewer than 1024 elements are converted whole: by lengths each takes a
+  // workgroup of its own, without them they are cut like one long doc (16666 docs of 5
+  // x 48 15.9 -> 4.6 us, 78125 of 8 x 64 60 -> 35; 146484 of 8 x 128 by lengths 121, whole 142).
+  if (rows * dp < 1024) lengths = nullptr;
   auto sizes = t.sizes().vec();
   sizes[n - 1] = dp;
   Tensor out = at::empty(sizes, t.options().dtype(dtype == FMX_DTYPE_BF16 ? at::kBFloat16 : at::kHalf));

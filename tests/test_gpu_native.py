@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import flash_maxsim_amd as fm
+from launches import launches
 from conftest import sim
 from flash_maxsim_amd import _lib
 
@@ -354,3 +355,17 @@ def test_calls_from_two_host_threads():
         assert len(got[i]) == 8
         for out in got[i]:
             assert len(out) == len(want[i]) and all(torch.equal(a, b) for a, b in zip(out, want[i]))
+
+
+@pytest.mark.parametrize("Ld, d, whole", [(13, 24, True), (1, 1, True), (7, 140, True), (8, 128, False), (40, 100, False)])
+def test_small_float32_docs_are_converted_whole(Ld, d, whole, tmp_path):
+    """Documents of fewer than 1024 elements are not converted by their lengths, a
+    workgroup each, but all rows as one; rows past a length (NaN here) reach no score."""
+    gen = torch.Generator(device=DEV).manual_seed(3600 + Ld)
+    Q, D = (torch.randn(*n, d, generator=gen, device=DEV) for n in ((40,), (3000, Ld)))
+    ln = torch.randint(0, Ld + 1, (3000,), generator=gen, device=DEV, dtype=torch.int32)
+    D[torch.arange(Ld, device=DEV) >= ln[:, None]] = float("nan")
+    assert torch.equal(fm.flash_maxsim(Q, D, ln), fm.flash_maxsim(Q.half(), D.half(), ln))
+    grids = [grid for name, grid in launches(lambda: fm.flash_maxsim(Q, D, ln), tmp_path) if "convert_kernel" in name]
+    groups = Ld * ((d + 7) // 8 * 2)
+    assert len(grids) == 2 and grids[1] == -(-(3000 * groups if whole else groups) // 1024), grids
